@@ -159,6 +159,33 @@ __device__ __forceinline__ double2 tw_of(const double2* tw, int j) {
   return tw[(j % NS) * ((1 << LOGN) / (NS * 8))];
 }
 
+// Orders a wave's LDS writes before its later reads (LDS executes one wave's
+// operations in order; this keeps the compiler from moving them).
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// t[r] *= W^(r k) (conjugated for S > 0), r < R, from w1 = W^k.
+template <int R, int S>
+__device__ __forceinline__ void apply_tw(double2* t, double2 w1) {
+  double2 w[R];
+  w[1] = w1;
+  if constexpr (R >= 4) {
+    w[2] = cmul(w[1], w[1]);
+    w[3] = cmul(w[1], w[2]);
+  }
+  if constexpr (R == 8) {
+    w[4] = cmul(w[2], w[2]);
+    w[5] = cmul(w[1], w[4]);
+    w[6] = cmul(w[2], w[4]);
+    w[7] = cmul(w[3], w[4]);
+  }
+#pragma unroll
+  for (int r = 1; r < R; ++r) t[r] = S < 0 ? cmul(t[r], w[r]) : cmulc(t[r], w[r]);
+}
+
 // One Stockham pass: radix R, stride Ns.  Butterfly jj (< N/R) reads
 // x[jj + (N/R) r'] and writes y[(jj/Ns) Ns R + jj%Ns + Ns r'].  With PRE the
 // pass takes its W^k from wc (loaded by the previous pass); with NSN > 0 it
@@ -183,23 +210,9 @@ __device__ __forceinline__ void reg_pass(double2* a, double2* buf, int j,
 #pragma unroll
     for (int r = 0; r < R; ++r) t[r] = a[b + NB * r];
     if constexpr (NS > 1) {
-      // W^(r k), r < R, from the table entries for r = 1, 2, 4
       constexpr int ST = N / (NS * R);
-      double2 w[R];
-      if constexpr (PRE) w[1] = wc;
-      else w[1] = tw[k * ST];
-      if constexpr (R >= 4) {
-        w[2] = cmul(w[1], w[1]);
-        w[3] = cmul(w[1], w[2]);
-      }
-      if constexpr (R == 8) {
-        w[4] = cmul(w[2], w[2]);
-        w[5] = cmul(w[1], w[4]);
-        w[6] = cmul(w[2], w[4]);
-        w[7] = cmul(w[3], w[4]);
-      }
-#pragma unroll
-      for (int r = 1; r < R; ++r) t[r] = S < 0 ? cmul(t[r], w[r]) : cmulc(t[r], w[r]);
+      if constexpr (PRE) apply_tw<R, S>(t, wc);
+      else apply_tw<R, S>(t, tw[k * ST]);
     }
     dft<R, S>(t);
     if constexpr (NSN > 0) {
@@ -264,6 +277,94 @@ __device__ __forceinline__ void fft_reg(double2* a, double2* buf, int j,
 }
 
 // ---------------------------------------------------------------------------
+// The same Stockham transform with the thread's twiddles in registers: one
+// W^k per radix-8 pass after the first and one per butterfly of a trailing
+// radix-2/4 pass, the same for every transform the thread runs, so a kernel
+// loads them once, beside its data, and stages no table.  Same operations
+// and roundings as fft_reg with SCHED 0.  A line of N <= 512 (at most 64
+// threads, N/8 dividing the wave) lies inside one wave: its transposes then
+// need no workgroup barrier, and its threads may call alone.  Longer lines:
+// every thread of the workgroup calls; waves with act = false only meet the
+// barriers.
+// ---------------------------------------------------------------------------
+template <int LOGN>
+struct HeldTw {
+  using L = Line<LOGN>;
+  static constexpr int NB = L::RLAST > 1 ? kE / L::RLAST : 0;  // last-pass butterflies
+  static constexpr int K = L::NPASS8 - 1 + NB;
+  double2 w[K > 0 ? K : 1];
+};
+template <int LOGN>
+__device__ __forceinline__ HeldTw<LOGN> held_tw(const double2* __restrict__ tw, int j) {
+  using L = Line<LOGN>;
+  HeldTw<LOGN> h;
+#pragma unroll
+  for (int i = 1; i < L::NPASS8; ++i) {
+    const int ns = 1 << (3 * i);
+    h.w[i - 1] = tw[(j % ns) * (L::N / (ns * 8))];
+  }
+#pragma unroll
+  for (int b = 0; b < HeldTw<LOGN>::NB; ++b)
+    h.w[L::NPASS8 - 1 + b] = tw[(j + L::TPL * b) % (1 << (3 * L::NPASS8))];
+  return h;
+}
+template <int LOGN>
+constexpr bool line_in_wave() { return Line<LOGN>::TPL <= 64; }
+template <int LOGN>
+__device__ __forceinline__ void line_sync() {
+  if constexpr (line_in_wave<LOGN>()) wave_sync();
+  else __syncthreads();
+}
+template <int LOGN, int S, int R, int NS, bool LAST>
+__device__ __forceinline__ void held_pass(double2* a, double2* buf, int j, const double2* w,
+                                          bool act) {
+  constexpr int N = 1 << LOGN;
+  constexpr int TPL = N / kE;
+  constexpr int NB = kE / R;
+  if (act) {
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      const int jj = j + TPL * b;
+      double2 t[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) t[r] = a[b + NB * r];
+      if constexpr (NS > 1) apply_tw<R, S>(t, w[b]);
+      dft<R, S>(t);
+      if constexpr (LAST) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) a[b + NB * r] = t[r];
+      } else {
+        double2* p = buf + lpad((jj / NS) * NS * R + jj % NS);
+#pragma unroll
+        for (int r = 0; r < R; ++r) p[lpad_off(r * NS)] = t[r];
+      }
+    }
+  }
+  if constexpr (!LAST) {
+    line_sync<LOGN>();
+    if (act) {
+      const double2* p = buf + lpad(j);
+#pragma unroll
+      for (int r = 0; r < kE; ++r) a[r] = p[lpad_off(TPL * r)];
+    }
+    line_sync<LOGN>();
+  }
+}
+template <int LOGN, int S>
+__device__ __forceinline__ void fft_held(double2* a, double2* buf, int j,
+                                         const HeldTw<LOGN>& h, bool act = true) {
+  using L = Line<LOGN>;
+  constexpr int P8 = L::NPASS8;
+  constexpr bool T = L::RLAST > 1;
+  held_pass<LOGN, S, 8, 1, P8 == 1 && !T>(a, buf, j, h.w, act);
+  if constexpr (P8 >= 2) held_pass<LOGN, S, 8, 8, P8 == 2 && !T>(a, buf, j, h.w, act);
+  if constexpr (P8 >= 3) held_pass<LOGN, S, 8, 64, P8 == 3 && !T>(a, buf, j, h.w + 1, act);
+  if constexpr (P8 >= 4) held_pass<LOGN, S, 8, 512, P8 == 4 && !T>(a, buf, j, h.w + 2, act);
+  if constexpr (T)
+    held_pass<LOGN, S, L::RLAST, (1 << (3 * P8)), true>(a, buf, j, h.w + P8 - 1, act);
+}
+
+// ---------------------------------------------------------------------------
 // In-place radix-8 transforms of a 4096-point line over 512 threads (eight
 // whole waves, thread j = lane + 64 wave).  The first pass combines the
 // elements j + 512 r that thread j holds; its outputs go to LDS, and each
@@ -285,14 +386,6 @@ __device__ __forceinline__ void fft_reg(double2* a, double2* buf, int j,
 constexpr int kIpLine = 4096 + 4096 / 8;  // double2 per line in LDS
 
 __device__ __forceinline__ int ip_pad(int e) { return e + (e >> 3); }
-
-// Orders a wave's LDS writes before its later reads (LDS executes one wave's
-// operations in order; this keeps the compiler from moving them).
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // t[r] *= W^(k r) (conjugated for S > 0), from w1 = W^k; each power is
 // applied as soon as it is formed (at most four live at a time).

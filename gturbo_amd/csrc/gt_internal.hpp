@@ -55,7 +55,8 @@ struct PassArgs {
   double2* znew;      // RK4 accumulator (compact)
   const double* emk;  // integrating factor (compact, real)
   double2* out;       // nonlinear term (compact), NLT mode
-  const double* ka;   // k2**(alpv/2) (compact), batched passes with akind 0
+  const double* ka;   // k2**(alpv/2) (compact); read by the batched passes and at
+                      // N <= 1024 when alpv != 2
   double2* sst;       // if set: the stage input formed by this y pass is
                       // also stored here (compact), for the adjoint's recompute
   // batched ensemble passes only: x-pass packing (0 = one row per line,
@@ -126,6 +127,9 @@ enum CMode : int {
 // are column pairs (wider tiles left 256^2 with six y workgroups).
 __host__ __device__ constexpr int bt_of(int logn) { return logn <= 12 ? 2 : 1; }
 __host__ __device__ constexpr int rows_of(int logn) { return logn <= 12 ? 2 : 1; }
+// Largest log2 N of the single-run passes that run a column's or row's
+// fields side by side (f_pass, fx_pass in gturbo_kernels.hip).
+constexpr int kFpMaxLogn = 10;
 __host__ __device__ constexpr int rp_of(int logn) {
   return logn <= 6 ? (1 << (logn - 1)) : logn == 7 ? 32 : logn == 8 ? 16
        : logn == 9 ? 8 : logn == 10 ? 4 : logn == 11 ? 2 : 1;

@@ -56,6 +56,7 @@ struct RectTables {
   Rect rc{-1, -1, -1};
   int kyp = 0;
   double* emk = nullptr;
+  double* ka = nullptr;  // k2**(alpv/2), alpv != 2 (rect_ka)
   ForcedMode* modes = nullptr;
   // the forced modes by kx column (fused step boundary): column c's updates
   // are fce[fcs[c] .. fcs[c+1]-1]
@@ -143,6 +144,7 @@ int ilog2(int n);
 int kyp_of(const Rect& r);
 int rect_kind(const gt_ctx* c, const Rect& r);
 int rect_tables(gt_ctx* c, const Rect& r, RectTables** out);
+int rect_ka(gt_ctx* c, const Rect& r, const double** out);
 int ensure_ybuf(gt_ctx* c, const Rect& r);
 int lookup(gt_ctx* c, const void* host, Mirror** m);
 int alloc_cmp(gt_ctx* c, Mirror& m, const Rect& r);
@@ -150,7 +152,7 @@ int ensure_ref(gt_ctx* c, Mirror& m);
 int ensure_cmp(gt_ctx* c, Mirror& m);
 void set_cmp_only(Mirror& m);
 void set_ref_only(Mirror& m);
-gt::PassArgs pass_args(gt_ctx* c, Mirror& z, RectTables* t);
+int pass_args(gt_ctx* c, Mirror& z, RectTables* t, gt::PassArgs* out);
 int c_pass(gt_ctx* c, int mode, const gt::PassArgs& a);
 int r_pass(gt_ctx* c, const gt::PassArgs& a);
 void forcing_phases(int nf, int32_t* seed, double2* out);

@@ -140,6 +140,7 @@ int fwd_step(gt_ctx* c, RectTables* t, int slot) {
   a.z = s->z;
   a.znew = s->znew;
   a.emk = t->emk;
+  CHK(rect_ka(c, s->rc, &a.ka));
   auto st = [&](int k) { return slot >= 0 ? stage_ptr(s, slot, k) : nullptr; };
   if (c->rko == 4) {
     a.sst = st(0);

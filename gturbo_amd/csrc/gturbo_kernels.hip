@@ -190,6 +190,93 @@ __device__ __forceinline__ void force_column(const PassArgs& a, int c, bool colo
   }
 }
 
+// Nonlinear term of one mode from the forward transforms A = (q u)^,
+// B = (q v)^ of its column: fft_dir normalisation /NY/NX (src/fft_dir.f90:19,
+// exact for N = 2^k), -ik. (src/nlt.f90:57-58), 2/3 mask.
+__device__ __forceinline__ double2 nl_term(const Phys& ph, double2 A, double2 B, double fkx,
+                                           double fkxs, double fky) {
+  const double2 Av = make_double2(A.x * ph.inv_n2, A.y * ph.inv_n2);
+  const double2 Bv = make_double2(B.x * ph.inv_n2, B.y * ph.inv_n2);
+  double2 k = make_double2(fkx * Av.y + fky * Bv.y, -fkx * Av.x - fky * Bv.x);
+  if (ph.truncate == 1 && cut_mode(ph, fkxs, fky * fky)) k = make_double2(0.0, 0.0);
+  return k;
+}
+
+// What the RK stage of a y pass reads of one mode (compact index q).
+struct StageIn {
+  double E;
+  double2 z, zn;
+};
+template <int MODE, bool NT>
+__device__ __forceinline__ StageIn stage_load(const PassArgs& a, unsigned q) {
+  constexpr bool RK4S = MODE == C_RK4_2 || MODE == C_RK4_3;
+  constexpr bool LAST4 = MODE == C_RK4_4 || MODE == C_RK4_4S;
+  StageIn in{};
+  if constexpr (MODE != C_NLT && MODE != C_START && !LAST4) {
+    in.E = ld_state<NT>(&a.emk[q]);
+    in.z = ld_state<NT>(&a.z[q]);
+  }
+  if constexpr (RK4S || LAST4) in.zn = ld_state<NT>(&a.znew[q]);
+  return in;
+}
+// The RK stage of one mode with nonlinear term k: stores what the stage
+// stores and returns the next stage input (for the fused step boundary the
+// updated state, which is forced and stored by the caller).
+template <int MODE, bool NT>
+__device__ __forceinline__ double2 stage_update(const PassArgs& a, unsigned q, bool mean,
+                                                double2 k, const StageIn& in) {
+  const Phys& ph = a.ph;
+  const double E = in.E;
+  const double2 zz = in.z, zn = in.zn;
+  double2 s = make_double2(0.0, 0.0);
+  if constexpr (MODE == C_NLT) {
+    if (mean) k = make_double2(0.0, 0.0);  // trunc.f90:24
+    a.out[q] = k;
+  } else if constexpr (MODE == C_RK4_1) {
+    // rkstep.f90:96,101
+    const double EE = E * E;
+    st_state<NT>(&a.znew[q], make_double2(EE * (zz.x + ph.dt6 * k.x), EE * (zz.y + ph.dt6 * k.y)));
+    s = make_double2(E * (zz.x + ph.dt2 * k.x), E * (zz.y + ph.dt2 * k.y));
+  } else if constexpr (MODE == C_RK4_2) {
+    // rkstep.f90:105,110
+    const double d3E = ph.dt3 * E;
+    st_state<NT>(&a.znew[q], make_double2(zn.x + d3E * k.x, zn.y + d3E * k.y));
+    s = make_double2(E * zz.x + ph.dt2 * k.x, E * zz.y + ph.dt2 * k.y);
+  } else if constexpr (MODE == C_RK4_3) {
+    // rkstep.f90:114,119
+    const double d3E = ph.dt3 * E;
+    st_state<NT>(&a.znew[q], make_double2(zn.x + d3E * k.x, zn.y + d3E * k.y));
+    s = make_double2(E * (E * zz.x + ph.dt * k.x), E * (E * zz.y + ph.dt * k.y));
+  } else if constexpr (MODE == C_RK4_4 || MODE == C_RK4_4S) {
+    // rkstep.f90:123,127
+    s = make_double2(zn.x + ph.dt6 * k.x, zn.y + ph.dt6 * k.y);
+    if (mean) s = make_double2(0.0, 0.0);
+    if constexpr (MODE == C_RK4_4) st_state<NT>(&a.z[q], s);
+  } else if constexpr (MODE == C_RK2_1) {
+    // rkstep.f90:24/34 and :42
+    s = make_double2(E * (zz.x + ph.dt2 * k.x), E * (zz.y + ph.dt2 * k.y));
+    if (mean) s = make_double2(0.0, 0.0);
+  } else if constexpr (MODE == C_RK2_2 || MODE == C_RK2_2S) {
+    // rkstep.f90:54/64 and :72
+    s = make_double2(E * (E * zz.x + ph.dt * k.x), E * (E * zz.y + ph.dt * k.y));
+    if (mean) s = make_double2(0.0, 0.0);
+    if constexpr (MODE == C_RK2_2) st_state<NT>(&a.z[q], s);
+  }
+  return s;
+}
+// Value of one mode in inverse transform f of a y pass: the stage input q
+// (f = 0), u = i ky q/ka (f = 1), v = -i kx q/ka (f = 2); src/nlt.f90:31-34.
+__device__ __forceinline__ double2 field_of(int f, double2 s, double fkx, double fky,
+                                            double ka) {
+  if (f == 0) return s;
+  if (f == 1) {
+    const double kyn = fky / ka;
+    return make_double2(-kyn * s.y, kyn * s.x);
+  }
+  const double kxn = fkx / ka;
+  return make_double2(kxn * s.y, -kxn * s.x);
+}
+
 // One tile of BT kx-columns; lds holds BT padded lines.  SCHED is the radix
 // order of the transforms (fft_reg).
 // IP (4096-point lines only): the y buffers hold the rows of a column in
@@ -264,74 +351,9 @@ __device__ __forceinline__ void c_body(const PassArgs& a, int tile, int tid,
       s[r] = make_double2(0.0, 0.0);
       if (live_r<TR>(r) && colok && row >= 0) {
         const double fky = (double)kyi_of(p, N) * ph.dky;
-        const double fkys = fky * fky;
-        // fft_dir normalisation /NY/NX (src/fft_dir.f90:19), exact for N = 2^k
-        const double2 Av = make_double2(A[r].x * ph.inv_n2, A[r].y * ph.inv_n2);
-        const double2 Bv = make_double2(z[r].x * ph.inv_n2, z[r].y * ph.inv_n2);
-        // src/nlt.f90:57-58
-        double2 k = make_double2(fkx * Av.y + fky * Bv.y, -fkx * Av.x - fky * Bv.x);
-        if (ph.truncate == 1 && cut_mode(ph, fkxs, fkys)) k = make_double2(0.0, 0.0);
+        const double2 k = nl_term(ph, A[r], z[r], fkx, fkxs, fky);
         const unsigned q = cbase + (unsigned)row;
-        const bool mean = (c == 0 && p == 0);
-        if constexpr (MODE == C_NLT) {
-          if (mean) k = make_double2(0.0, 0.0);  // trunc.f90:24
-          a.out[q] = k;
-        } else if constexpr (MODE == C_RK4_1) {
-          // rkstep.f90:96,101
-          const double E = ld_state<NT>(&a.emk[q]);
-          const double2 zz = ld_state<NT>(&a.z[q]);
-          const double EE = E * E;
-          st_state<NT>(&a.znew[q], make_double2(EE * (zz.x + ph.dt6 * k.x), EE * (zz.y + ph.dt6 * k.y)));
-          s[r] = make_double2(E * (zz.x + ph.dt2 * k.x), E * (zz.y + ph.dt2 * k.y));
-        } else if constexpr (MODE == C_RK4_2) {
-          // rkstep.f90:105,110
-          const double E = ld_state<NT>(&a.emk[q]);
-          const double2 zz = ld_state<NT>(&a.z[q]);
-          const double2 zn = ld_state<NT>(&a.znew[q]);
-          const double d3E = ph.dt3 * E;
-          st_state<NT>(&a.znew[q], make_double2(zn.x + d3E * k.x, zn.y + d3E * k.y));
-          s[r] = make_double2(E * zz.x + ph.dt2 * k.x, E * zz.y + ph.dt2 * k.y);
-        } else if constexpr (MODE == C_RK4_3) {
-          // rkstep.f90:114,119
-          const double E = ld_state<NT>(&a.emk[q]);
-          const double2 zz = ld_state<NT>(&a.z[q]);
-          const double2 zn = ld_state<NT>(&a.znew[q]);
-          const double d3E = ph.dt3 * E;
-          st_state<NT>(&a.znew[q], make_double2(zn.x + d3E * k.x, zn.y + d3E * k.y));
-          s[r] = make_double2(E * (E * zz.x + ph.dt * k.x), E * (E * zz.y + ph.dt * k.y));
-        } else if constexpr (MODE == C_RK4_4) {
-          // rkstep.f90:123,127
-          const double2 zn = ld_state<NT>(&a.znew[q]);
-          double2 zz = make_double2(zn.x + ph.dt6 * k.x, zn.y + ph.dt6 * k.y);
-          if (mean) zz = make_double2(0.0, 0.0);
-          st_state<NT>(&a.z[q], zz);
-        } else if constexpr (MODE == C_RK4_4S) {
-          // rkstep.f90:123,127; forced and stored below
-          const double2 zn = ld_state<NT>(&a.znew[q]);
-          double2 zz = make_double2(zn.x + ph.dt6 * k.x, zn.y + ph.dt6 * k.y);
-          if (mean) zz = make_double2(0.0, 0.0);
-          s[r] = zz;
-        } else if constexpr (MODE == C_RK2_2S) {
-          // rkstep.f90:54/64 and :72; forced and stored below
-          const double E = ld_state<NT>(&a.emk[q]);
-          const double2 zz = ld_state<NT>(&a.z[q]);
-          double2 zo = make_double2(E * (E * zz.x + ph.dt * k.x), E * (E * zz.y + ph.dt * k.y));
-          if (mean) zo = make_double2(0.0, 0.0);
-          s[r] = zo;
-        } else if constexpr (MODE == C_RK2_1) {
-          // rkstep.f90:24/34 and :42
-          const double E = ld_state<NT>(&a.emk[q]);
-          const double2 zz = ld_state<NT>(&a.z[q]);
-          s[r] = make_double2(E * (zz.x + ph.dt2 * k.x), E * (zz.y + ph.dt2 * k.y));
-          if (mean) s[r] = make_double2(0.0, 0.0);
-        } else if constexpr (MODE == C_RK2_2) {
-          // rkstep.f90:54/64 and :72
-          const double E = ld_state<NT>(&a.emk[q]);
-          const double2 zz = ld_state<NT>(&a.z[q]);
-          double2 zo = make_double2(E * (E * zz.x + ph.dt * k.x), E * (E * zz.y + ph.dt * k.y));
-          if (mean) zo = make_double2(0.0, 0.0);
-          st_state<NT>(&a.z[q], zo);
-        }
+        s[r] = stage_update<MODE, NT>(a, q, c == 0 && p == 0, k, stage_load<MODE, NT>(a, q));
       }
     }
     if constexpr (MODE == C_RK4_4S || MODE == C_RK2_2S) {
@@ -390,13 +412,7 @@ __device__ __forceinline__ void c_body(const PassArgs& a, int tile, int tid,
             const double kar =
                 AK == 0 ? ka[AK == 0 ? r : 0]
                         : kalpha_t<AK>(a, fkxs + fky * fky, cbase + (unsigned)row_of(p, rc, N));
-            if (f == 1) {
-              const double kyn = fky / kar;
-              v = make_double2(-kyn * s[r].y, kyn * s[r].x);  // nlt.f90:31-32
-            } else {
-              const double kxn = fkx / kar;
-              v = make_double2(kxn * s[r].y, -kxn * s[r].x);  // nlt.f90:33-34
-            }
+            v = field_of(f, s[r], fkx, fky, kar);
           }
         }
         z[r] = v;
@@ -441,6 +457,212 @@ __global__ void __launch_bounds__(bt_of(LOGN) * (1 << LOGN) / kE, AK == 1 ? 4 : 
   // column's, so neighbouring columns run on one XCD (y stages -5.6%).
   const int tile = LOGN == 13 ? xcd_remap(blockIdx.x, gridDim.x) : (int)blockIdx.x;
   c_body<LOGN, MODE, AK, TR, BT, 0, IP>(a, tile, threadIdx.x, lds, tw);
+}
+
+// ---------------------------------------------------------------------------
+// Small grids: the fields of a column (y pass) or row (x pass) side by side.
+// On these grids a pass has fewer workgroups than the chip has room for
+// (43 column pairs at 256^2 on 256 CUs) and its time is the chain of loads,
+// transforms and barriers inside one workgroup, not a rate.  Each of a
+// column's fields therefore has its own N/8 threads (whole waves per field):
+// the two forward transforms run together, then the three inverse ones (five
+// one after the other otherwise), and every load of the pass -- products,
+// state, twiddles, ka, forcing -- is issued before the first transform.
+// Against the five-in-turn passes (kernel durations, RK4, same operations,
+// bit-identical): y stage 64^2 11.1 -> 4.4 us, 256^2 12.0 -> 5.5, 512^2
+// (alpha 1) 14.6 -> 7.2, 1024^2 (alpha 1) 24.0 -> 18.0; step boundary 256^2
+// 15.4 -> 7.5, 1024^2 29.4 -> 20.7; x pass 5.0 -> 4.1, 5.8 -> 4.8, 7.8 ->
+// 6.5, 16.6 -> 15.6.  Up to 512^2 the rest is a kernel's own start and end
+// (about 2 us), two memory round trips and two transforms; at 1024^2 the
+// 41 MB a stage moves take half of it (12.7 us with the transforms skipped).
+// ---------------------------------------------------------------------------
+
+// Columns per workgroup of the y pass: a wave per field where a line is
+// shorter than a wave; 512: one (7.3 us; two 8.2); 1024: two (18.5 us; one,
+// whose workgroups each touch half of every line, 20.8).
+__host__ __device__ constexpr int fp_cols(int logn) { return logn < 9 ? 512 >> logn : logn == 9 ? 1 : 2; }
+constexpr int kFpForce = 32;  // forced modes of a column staged in LDS
+
+template <int LOGN, int MODE, int AK, int TR>
+__global__ void __launch_bounds__(fp_cols(LOGN) * 3 * (1 << LOGN) / kE) f_pass(PassArgs a) {
+  constexpr int N = 1 << LOGN, TPL = N / kE, BT = bt_of(LOGN), CW = fp_cols(LOGN);
+  constexpr int LINE = Line<LOGN>::PADDED, GT = CW * TPL;  // threads per field
+  constexpr bool FWD = MODE != C_START;
+  constexpr bool INV = MODE != C_NLT && MODE != C_RK4_4 && MODE != C_RK2_2;
+  constexpr bool BOUND = MODE == C_RK4_4S || MODE == C_RK2_2S;
+  constexpr int NOWN = TR ? 2 : 3;           // modes a thread updates
+  constexpr int NLINE = FWD && INV ? 4 : 3;  // A, B, (scratch), stage input
+  static_assert(GT % 64 == 0, "whole waves per field");
+  __shared__ double2 lds[CW * NLINE * LINE];
+  __shared__ double2 famp[BOUND ? CW * kFpForce : 1];
+  __shared__ __align__(16) int frow[BOUND ? CW * kFpForce : 4];
+  const int f = __builtin_amdgcn_readfirstlane(threadIdx.x / GT);
+  const int t = threadIdx.x % GT, cw = t / TPL, j = t % TPL;
+  // one-column workgroups: the two columns of a tile on one XCD
+  const int c = CW == 1 ? xcd_remap(blockIdx.x, gridDim.x) : (int)blockIdx.x * CW + cw;
+  const Rect rc = a.rc;
+  const bool colok = c <= rc.kx;
+  const Phys& ph = a.ph;
+  const double fkx = (double)c * ph.dkx;
+  const double fkxs = fkx * fkx;
+  const unsigned cbase = (unsigned)c * (unsigned)a.kyp;
+  const unsigned colo = ycol_off(c, BT);
+  double2* col = lds + cw * NLINE * LINE;
+  double2* buf = col + f * LINE;
+  double2* sbuf = col + 3 * LINE;  // the column's stage input
+
+  double2 z[kE];
+  if constexpr (FWD) {
+    if (f < 2) {
+      const double2* src = a.y2 + (size_t)f * a.ntiles * N * BT;
+#pragma unroll
+      for (int r = 0; r < kE; ++r)
+        z[r] = colok ? src[yrow_off(j + TPL * r, a.ntiles, BT) + colo] : make_double2(0.0, 0.0);
+    }
+  } else {
+#pragma unroll
+    for (int r = 0; r < kE; ++r) {
+      const int row = row_of(j + TPL * r, rc, N);
+      z[r] = (live_r<TR>(r) && colok && row >= 0) ? a.z[cbase + (unsigned)row]
+                                                   : make_double2(0.0, 0.0);
+    }
+  }
+  const HeldTw<LOGN> tw = held_tw<LOGN>(a.tw, j);
+  // positions this thread updates: r = NOWN f + i of the live ones
+  int pos[NOWN];
+  bool own[NOWN];
+  unsigned qi[NOWN];
+  StageIn in[NOWN];
+  if constexpr (FWD) {
+#pragma unroll
+    for (int i = 0; i < NOWN; ++i) {
+      const int x = NOWN * f + i, r = TR && x >= 3 ? x + 2 : x;
+      pos[i] = j + TPL * r;
+      const int row = r < kE ? row_of(pos[i], rc, N) : -1;
+      own[i] = colok && row >= 0;
+      qi[i] = cbase + (unsigned)row;
+      in[i] = own[i] ? stage_load<MODE, false>(a, qi[i]) : StageIn{};
+    }
+  }
+  double ka[kE];
+  auto load_ka = [&]() {
+#pragma unroll
+    for (int r = 0; r < kE; ++r) {
+      const int row = row_of(j + TPL * r, rc, N);
+      ka[r] = live_r<TR>(r) && colok && row >= 0 && f > 0 ? a.ka[cbase + (unsigned)row] : 1.0;
+    }
+  };
+  // 1024: after the forward transforms (768 threads leave 168 VGPRs)
+  constexpr bool KA_LATE = LOGN >= 10 && FWD;
+  if constexpr (INV && AK == 2 && !KA_LATE) load_ka();
+
+  if constexpr (FWD) {
+    // The column's forcing entries (forcing.f90:25-31), formed by the third
+    // field's waves while the others transform.
+    const bool forced = BOUND && a.fcs != nullptr && colok;
+    int e0 = 0, ne = 0;
+    if constexpr (BOUND) {
+      if (forced) {
+        e0 = a.fcs[c];
+        ne = a.fcs[c + 1] - e0;
+      }
+      if (f == 2) {
+        for (int e = j; e < kFpForce; e += TPL) {
+          int row = -1;
+          if (e < ne) {
+            const FEntry fe = a.fce[e0 + e];
+            const double2 cs = a.fph[fe.k];
+            const double a2 = a.famp * fe.ff2 * cs.y;
+            famp[cw * kFpForce + e] = make_double2(a.famp * fe.ff1 * cs.x, fe.conj ? -a2 : a2);
+            row = fe.row;
+          }
+          frow[cw * kFpForce + e] = row;
+        }
+      }
+    }
+    if (!line_in_wave<LOGN>() || f < 2) fft_held<LOGN, -1>(z, buf, j, tw, f < 2);
+    if (f < 2) {
+#pragma unroll
+      for (int r = 0; r < kE; ++r)
+        if (live_r<TR>(r)) (buf + lpad(j))[lpad_off(TPL * r)] = z[r];
+    }
+    if constexpr (INV && AK == 2 && KA_LATE) load_ka();
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NOWN; ++i) {
+      double2 s = make_double2(0.0, 0.0);
+      if (own[i]) {
+        const int p = pos[i], e = lpad(p);
+        const double fky = (double)kyi_of(p, N) * ph.dky;
+        const double2 k = nl_term(ph, col[e], col[LINE + e], fkx, fkxs, fky);
+        s = stage_update<MODE, false>(a, qi[i], c == 0 && p == 0, k, in[i]);
+        if constexpr (BOUND) {  // in table order
+          const int row = (int)(qi[i] - cbase);
+          const int* fr = frow + cw * kFpForce;
+          for (int n = 0; n < (ne < kFpForce ? ne : kFpForce); n += 8) {
+            const int4 u = *reinterpret_cast<const int4*>(fr + n);
+            const int4 w = *reinterpret_cast<const int4*>(fr + n + 4);
+            if (u.x == row || u.y == row || u.z == row || u.w == row || w.x == row ||
+                w.y == row || w.z == row || w.w == row) {
+              for (int m = n; m < n + 8; ++m) {
+                if (fr[m] == row) {
+                  const double2 d = famp[cw * kFpForce + m];
+                  s = make_double2(s.x + d.x, s.y + d.y);
+                }
+              }
+            }
+          }
+          for (int n = kFpForce; n < ne; ++n) {
+            const FEntry fe = a.fce[e0 + n];
+            if (fe.row == row) {
+              const double2 cs = a.fph[fe.k];
+              const double a2 = a.famp * fe.ff2 * cs.y;
+              s = make_double2(s.x + a.famp * fe.ff1 * cs.x, fe.conj ? s.y - a2 : s.y + a2);
+            }
+          }
+          a.z[qi[i]] = s;
+        }
+        if constexpr (INV) {
+          if (a.sst != nullptr) a.sst[qi[i]] = s;  // kept for the adjoint's recompute
+        }
+      }
+      if constexpr (INV) {
+        if (TR || NOWN * f + i < kE) sbuf[lpad(pos[i])] = s;
+      }
+    }
+    if constexpr (INV) {
+      __syncthreads();
+#pragma unroll
+      for (int r = 0; r < kE; ++r)
+        z[r] = live_r<TR>(r) ? (sbuf + lpad(j))[lpad_off(TPL * r)] : make_double2(0.0, 0.0);
+    }
+  } else if (a.sst != nullptr && f == 0) {
+#pragma unroll
+    for (int r = 0; r < kE; ++r) {
+      const int row = row_of(j + TPL * r, rc, N);
+      if (live_r<TR>(r) && colok && row >= 0) a.sst[cbase + (unsigned)row] = z[r];
+    }
+  }
+
+  if constexpr (INV) {
+#pragma unroll
+    for (int r = 0; r < kE; ++r) {
+      if (!live_r<TR>(r)) continue;
+      const int p = j + TPL * r;
+      const double fky = (double)kyi_of(p, N) * ph.dky;
+      if (c == 0 && p == 0) {  // nlt.f90:25
+        if (f > 0) z[r] = make_double2(0.0, 0.0);
+      } else {
+        z[r] = field_of(f, z[r], fkx, fky, AK == 1 ? fkxs + fky * fky : ka[r]);
+      }
+    }
+    fft_held<LOGN, +1>(z, buf, j, tw);
+    if (colok) {
+      double2* dst = a.y1 + (size_t)f * a.ntiles * N * BT;
+#pragma unroll
+      for (int r = 0; r < kE; ++r) dst[yrow_off(j + TPL * r, a.ntiles, BT) + colo] = z[r];
+    }
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -573,6 +795,66 @@ __device__ __forceinline__ void r_body(const PassArgs& a, int g, int tid,
   split_store<LOGN, TR, BT>(z, buf, j, a.y2, offQ, offQ + fstride, kxm);
 }
 
+// Small grids (see f_pass): a row's two inverse transforms, of q+iv and
+// q+iu, each on its own N/8 threads; the operations are r_body's.  q v
+// crosses to the q u threads through LDS, these run the forward transform of
+// q u + i q v, and both store their half of the split spectrum.
+// Rows per workgroup: 512: two (6.4 us; one 7.2); 1024: one (15.9; two 19.1).
+__host__ __device__ constexpr int fx_rows(int logn) {
+  return logn == 10 ? 1 : logn == 9 ? 2 : logn == 4 ? 16 : 512 >> logn;
+}
+template <int LOGN, int TR>
+__global__ void __launch_bounds__(2 * fx_rows(LOGN) * (1 << LOGN) / kE) fx_pass(PassArgs a) {
+  constexpr int N = 1 << LOGN, TPL = N / kE, BT = bt_of(LOGN), RW = fx_rows(LOGN);
+  constexpr int LINE = Line<LOGN>::PADDED, GT = RW * TPL;
+  __shared__ double2 lds[2 * RW * LINE];
+  int f = threadIdx.x / GT;  // 0: q+iv, 1: q+iu
+  if constexpr (GT % 64 == 0) f = __builtin_amdgcn_readfirstlane(f);
+  const int t = threadIdx.x % GT, rw = t / TPL, j = t % TPL;
+  const int yrow = xcd_remap(blockIdx.x, gridDim.x) * RW + rw;
+  double2* row = lds + 2 * rw * LINE;
+  double2* buf = row + f * LINE;
+  const int kxm = a.rc.kx;
+  const unsigned fstride = (unsigned)a.ntiles * N * BT;
+  const unsigned off = yrow_off(yrow, a.ntiles, BT);
+  double2 z[kE], x0[kE], x1[kE];
+  load_two<LOGN, TR, BT>(x0, x1, j, a.y1, off, off + (f ? fstride : 2 * fstride), kxm);
+  const HeldTw<LOGN> tw = held_tw<LOGN>(a.tw, j);
+  pack_two<LOGN>(z, j, x0, x1);
+  fft_held<LOGN, +1>(z, buf, j, tw);
+  double* qv = reinterpret_cast<double*>(row);  // the q+iv line, free again
+  if (f == 0) {
+#pragma unroll
+    for (int r = 0; r < kE; ++r) qv[j + TPL * r] = z[r].x * z[r].y;  // produ.f90:16
+  }
+  __syncthreads();
+  if (f == 1) {
+#pragma unroll
+    for (int r = 0; r < kE; ++r)
+      z[r] = make_double2(z[r].x * z[r].y, qv[j + TPL * r]);  // produ.f90:15
+  }
+  if (!line_in_wave<LOGN>() || f == 1) fft_held<LOGN, -1>(z, buf, j, tw, f == 1);
+  double2* wl = row + LINE;
+  if (f == 1) {
+#pragma unroll
+    for (int r = 0; r < kE; ++r)
+      if (live_r<TR>(r)) (wl + lpad(j))[lpad_off(TPL * r)] = z[r];
+  }
+  __syncthreads();
+  const double2* pm = wl + lpad(TPL - j);
+  double2* out = a.y2 + off + (f ? 0u : fstride);
+#pragma unroll
+  for (int r = 0; r <= kE / 2; ++r) {  // k <= N/2 (r = kE/2 only for k = N/2)
+    const int k = j + TPL * r;
+    if (live_r<TR>(r) && k <= kxm && k <= N / 2) {
+      const double2 W = (wl + lpad(j))[lpad_off(TPL * r)];
+      const double2 Wc = mirror_at<LOGN>(wl, pm, j, r);
+      out[koff<LOGN, BT>(k)] = f ? make_double2(0.5 * (W.x + Wc.x), 0.5 * (W.y - Wc.y))
+                                 : make_double2(0.5 * (W.y + Wc.y), -0.5 * (W.x - Wc.x));
+    }
+  }
+}
+
 // Row-pair variant: each line of N/8 threads handles rows y0 and y0+1
 // (group g holds pairs g*NL ..).  The complex transform of Q0 + iQ1 gives q
 // of both rows; V0 + iV1 and U0 + iU1 likewise, and the products of the two
@@ -638,19 +920,6 @@ __device__ __forceinline__ void pair_body(const PassArgs& a, int g, int tid,
   for (int r = 0; r < kE; ++r) z[r] = make_double2(qq[r].x * z[r].x, qq[r].y * z[r].y);
   fwd(z);                                                      // (q u)0 + i (q u)1
   split_store<LOGN, TR, BT>(z, buf, j, a.y2, r0, r1, kxm);
-}
-
-// Not launched for N >= 2048 (r_pass_pair there; at 4096 the y passes
-// write y1 in row-pair blocks, which only pair_body reads).
-template <int LOGN, int TR>
-__global__ void __launch_bounds__(rows_of(LOGN) * (1 << LOGN) / kE)
-    r_pass(PassArgs a) {
-  constexpr int RP = rows_of(LOGN);
-  __shared__ double2 lds[RP * Line<LOGN>::PADDED];
-  __shared__ double2 twl[tw_lds_size<LOGN>()];
-  const double2* tw = stage_tw<LOGN>(twl, a.tw, threadIdx.x, blockDim.x);
-  r_body<LOGN, TR, bt_of(LOGN), RP, 0>(a, xcd_remap(blockIdx.x, gridDim.x), threadIdx.x, lds,
-                                       tw);
 }
 
 // N = 8192, one row per workgroup.  A real row x of N points is the
@@ -1170,21 +1439,29 @@ hipError_t ens_r_launch(int ty, const PassArgs* d, const uint32_t* it, int n, in
                         hipStream_t s);
 
 #if defined(GT_INST_LOGN)
+template <int L, int MODE, int AK, int TR>
+static void y_launch(const PassArgs& a, hipStream_t s) {
+  if constexpr (L <= kFpMaxLogn) {
+    constexpr int CW = fp_cols(L);
+    const int g = (a.rc.kc() + CW - 1) / CW;
+    f_pass<L, MODE, AK, TR><<<dim3(g), dim3(CW * 3 * (1 << L) / kE), 0, s>>>(a);
+  } else {
+    c_pass<L, MODE, AK, TR><<<dim3(a.ntiles), dim3(bt_of(L) * (1 << L) / kE), 0, s>>>(a);
+  }
+}
 template <int L, int AK, int TR>
 static hipError_t c_pass_launch_ak(int mode, const PassArgs& a, hipStream_t s) {
-  constexpr int T = bt_of(L) * (1 << L) / kE;
-  dim3 g(a.ntiles), b(T);
   switch (mode) {
-    case C_START: c_pass<L, C_START, AK, TR><<<g, b, 0, s>>>(a); break;
-    case C_NLT: c_pass<L, C_NLT, AK, TR><<<g, b, 0, s>>>(a); break;
-    case C_RK4_1: c_pass<L, C_RK4_1, AK, TR><<<g, b, 0, s>>>(a); break;
-    case C_RK4_2: c_pass<L, C_RK4_2, AK, TR><<<g, b, 0, s>>>(a); break;
-    case C_RK4_3: c_pass<L, C_RK4_3, AK, TR><<<g, b, 0, s>>>(a); break;
-    case C_RK4_4: c_pass<L, C_RK4_4, AK, TR><<<g, b, 0, s>>>(a); break;
-    case C_RK2_1: c_pass<L, C_RK2_1, AK, TR><<<g, b, 0, s>>>(a); break;
-    case C_RK2_2: c_pass<L, C_RK2_2, AK, TR><<<g, b, 0, s>>>(a); break;
-    case C_RK4_4S: c_pass<L, C_RK4_4S, AK, TR><<<g, b, 0, s>>>(a); break;
-    case C_RK2_2S: c_pass<L, C_RK2_2S, AK, TR><<<g, b, 0, s>>>(a); break;
+    case C_START: y_launch<L, C_START, AK, TR>(a, s); break;
+    case C_NLT: y_launch<L, C_NLT, AK, TR>(a, s); break;
+    case C_RK4_1: y_launch<L, C_RK4_1, AK, TR>(a, s); break;
+    case C_RK4_2: y_launch<L, C_RK4_2, AK, TR>(a, s); break;
+    case C_RK4_3: y_launch<L, C_RK4_3, AK, TR>(a, s); break;
+    case C_RK4_4: y_launch<L, C_RK4_4, AK, TR>(a, s); break;
+    case C_RK2_1: y_launch<L, C_RK2_1, AK, TR>(a, s); break;
+    case C_RK2_2: y_launch<L, C_RK2_2, AK, TR>(a, s); break;
+    case C_RK4_4S: y_launch<L, C_RK4_4S, AK, TR>(a, s); break;
+    case C_RK2_2S: y_launch<L, C_RK2_2S, AK, TR>(a, s); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -1200,14 +1477,15 @@ __host__ __device__ inline int rect_tr(const Rect& rc, int n) {
 template <int L>
 hipError_t c_pass_launch(int mode, const PassArgs& a, hipStream_t s) {
   const int tr = rect_tr(a.rc, 1 << L);
+  constexpr int AK = L <= kFpMaxLogn ? 2 : 0;  // alpha != 2: table of ka, or ka in registers
   if (a.ph.akind == 1)
     return tr ? c_pass_launch_ak<L, 1, 1>(mode, a, s) : c_pass_launch_ak<L, 1, 0>(mode, a, s);
-  return tr ? c_pass_launch_ak<L, 0, 1>(mode, a, s) : c_pass_launch_ak<L, 0, 0>(mode, a, s);
+  return tr ? c_pass_launch_ak<L, AK, 1>(mode, a, s) : c_pass_launch_ak<L, AK, 0>(mode, a, s);
 }
 
 template <int L>
 hipError_t r_pass_launch(const PassArgs& a, hipStream_t s) {
-  if constexpr (L >= 11) {  // one row pair per workgroup (8192: one row)
+  if constexpr (L > kFpMaxLogn) {  // one row pair per workgroup (8192: one row)
     constexpr int T = (1 << L) / kE;
     if (rect_tr(a.rc, 1 << L)) {
       if constexpr (L == 13)
@@ -1217,13 +1495,13 @@ hipError_t r_pass_launch(const PassArgs& a, hipStream_t s) {
     } else {
       r_pass_pair<L, 0><<<dim3((1 << L) / 2), dim3(T), 0, s>>>(a);
     }
-    return hipGetLastError();
+  } else {
+    constexpr int RW = fx_rows(L), T = 2 * RW * (1 << L) / kE;
+    if (rect_tr(a.rc, 1 << L))
+      fx_pass<L, 1><<<dim3((1 << L) / RW), dim3(T), 0, s>>>(a);
+    else
+      fx_pass<L, 0><<<dim3((1 << L) / RW), dim3(T), 0, s>>>(a);
   }
-  constexpr int RP = rows_of(L), T = RP * (1 << L) / kE;
-  if (rect_tr(a.rc, 1 << L))
-    r_pass<L, 1><<<dim3((1 << L) / RP), dim3(T), 0, s>>>(a);
-  else
-    r_pass<L, 0><<<dim3((1 << L) / RP), dim3(T), 0, s>>>(a);
   return hipGetLastError();
 }
 

@@ -233,6 +233,27 @@ int rect_tables(gt_ctx* c, const Rect& r, RectTables** out) {
   return GT_OK;
 }
 
+// Table of ka = k2**(alpv/2) of one rectangle for the passes that read it
+// (alpv != 2), built on the device once; null when the passes form ka.
+int rect_ka(gt_ctx* c, const Rect& r, const double** out) {
+  *out = nullptr;
+  if (c->ph.akind == 1 || c->logn > gt::kFpMaxLogn) return GT_OK;
+  RectTables& t = c->tab[rect_kind(c, r)];
+  if (!t.ka) {
+    const int kyp = kyp_of(r);
+    double* p = nullptr;
+    HIPCHK(hipMalloc(&p, sizeof(double) * (size_t)r.kc() * kyp));
+    const hipError_t e = gt::launch_ka_table(c->ph, r, kyp, p, c->stream);
+    if (e != hipSuccess) {
+      (void)hipFree(p);
+      return fail(GT_ERR_HIP, "ka table: %s", hipGetErrorString(e));
+    }
+    t.ka = p;
+  }
+  *out = t.ka;
+  return GT_OK;
+}
+
 int ensure_ybuf(gt_ctx* c, const Rect& r) {
   const int bt = gt::bt_of(c->logn);
   const size_t ntiles = (size_t)(r.kc() + bt - 1) / bt;
@@ -327,7 +348,7 @@ void set_ref_only(Mirror& m) {
   m.cmp_valid = false;
 }
 
-gt::PassArgs pass_args(gt_ctx* c, Mirror& z, RectTables* t) {
+int pass_args(gt_ctx* c, Mirror& z, RectTables* t, gt::PassArgs* out) {
   gt::PassArgs a{};
   a.rc = z.rect;
   a.kyp = z.kyp;
@@ -339,7 +360,9 @@ gt::PassArgs pass_args(gt_ctx* c, Mirror& z, RectTables* t) {
   a.y2 = c->y2;
   a.z = z.dcmp;
   a.emk = t ? t->emk : nullptr;
-  return a;
+  CHK(rect_ka(c, z.rect, &a.ka));
+  *out = a;
+  return GT_OK;
 }
 
 int c_pass(gt_ctx* c, int mode, const gt::PassArgs& a) {
@@ -629,6 +652,7 @@ int gt_destroy(gt_ctx* c) {
   }
   for (auto& t : c->tab) {
     if (t.emk) (void)hipFree(t.emk);
+    if (t.ka) (void)hipFree(t.ka);
     if (t.modes) (void)hipFree(t.modes);
     if (t.fcs) (void)hipFree(t.fcs);
     if (t.fce) (void)hipFree(t.fce);
@@ -926,7 +950,8 @@ int gt_nlt(gt_ctx* c, double* z, double* u, double* v) {
   CHK(lookup(c, v, &mv));
   CHK(ensure_cmp(c, *m));
   CHK(ensure_ybuf(c, m->rect));
-  gt::PassArgs a = pass_args(c, *m, nullptr);
+  gt::PassArgs a;
+  CHK(pass_args(c, *m, nullptr, &a));
   a.out = m->dcmp;
   CHK(c_pass(c, gt::C_START, a));
   CHK(r_pass(c, a));
@@ -948,7 +973,8 @@ int gt_step(gt_ctx* c, double* z, double* znl, double* u, double* v) {
   CHK(ensure_ybuf(c, m->rect));
   RectTables* t;
   CHK(rect_tables(c, m->rect, &t));
-  gt::PassArgs a = pass_args(c, *m, t);
+  gt::PassArgs a;
+  CHK(pass_args(c, *m, t, &a));
   CHK(step_start(c, PEND_RK2, m, nullptr, a));
   CHK(r_pass(c, a));
   CHK(c_pass(c, gt::C_RK2_1, a));
@@ -976,7 +1002,8 @@ int gt_step4(gt_ctx* c, double* z, double* znl, double* znew, double* u, double*
   RectTables* t;
   CHK(rect_tables(c, m->rect, &t));
   CHK(alloc_cmp(c, *mn, m->rect));
-  gt::PassArgs a = pass_args(c, *m, t);
+  gt::PassArgs a;
+  CHK(pass_args(c, *m, t, &a));
   a.znew = mn->dcmp;
   CHK(step_start(c, PEND_RK4, m, mn, a));
   CHK(r_pass(c, a));
