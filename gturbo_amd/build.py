@@ -73,6 +73,9 @@ def build_library(verbose=False, jobs=None):
                           [src_k, f"-DGT_INST_ENS={t}", f"-DGT_ENS_SCHED={sched}"]))
     units.append((os.path.join(OBJ, "kcommon.o"), [src_k, "-DGT_INST_COMMON"]))
     units += [(os.path.join(OBJ, f"k{l}.o"), [src_k, f"-DGT_INST_LOGN={l}"]) for l in LOGNS]
+    # plain C++: the host's own instruction-set attributes
+    units.append((os.path.join(OBJ, "phases.o"),
+                  ["-x", "c++", os.path.join(CSRC, "gturbo_phases.cpp")]))
     units.append((os.path.join(OBJ, "runtime.o"), [os.path.join(CSRC, "gturbo_runtime.cpp")]))
     units.append((os.path.join(OBJ, "ensemble.o"), [os.path.join(CSRC, "gturbo_ensemble.cpp")]))
     units.append((os.path.join(OBJ, "adjoint.o"), [os.path.join(CSRC, "gturbo_adjoint.cpp")]))

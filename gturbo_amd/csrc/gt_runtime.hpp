@@ -11,6 +11,7 @@
 
 #include "gt_internal.hpp"
 #include "gturbo.h"
+#include "gturbo_phases.hpp"
 
 using gt::ForcedMode;
 using gt::Phys;
@@ -38,6 +39,7 @@ int fail(int code, const char* fmt, ...) __attribute__((format(printf, 2, 3)));
 
 constexpr int kNFORC = 2048;  // src/modules.f90:41
 constexpr int kRing = 64;     // forcing-phase slots in flight
+constexpr int kRingSeg = 16;  // slots guarded by one event
 
 struct Mirror {
   void* host = nullptr;
@@ -112,9 +114,11 @@ struct gt_ctx {
 
   // forcing phases
   double2* ph_host = nullptr;  // pinned, kRing * nf
+  // what the kernels read: the pinned slots themselves, or device copies
   double2* ph_dev = nullptr;
-  hipEvent_t ph_ev[gtr::kRing];
-  bool ph_ev_used[gtr::kRing] = {};
+  bool ph_direct = false;
+  hipEvent_t ph_ev[gtr::kRing / gtr::kRingSeg] = {};
+  bool ph_ev_used[gtr::kRing / gtr::kRingSeg] = {};
   unsigned ph_next = 0;
 
   // diagnostics
@@ -155,7 +159,6 @@ void set_ref_only(Mirror& m);
 int pass_args(gt_ctx* c, Mirror& z, RectTables* t, gt::PassArgs* out);
 int c_pass(gt_ctx* c, int mode, const gt::PassArgs& a);
 int r_pass(gt_ctx* c, const gt::PassArgs& a);
-void forcing_phases(int nf, int32_t* seed, double2* out);
 int forcing_on(gt_ctx* c, RectTables* t, double2* z, int32_t* seed);
 void adj_free(gt_ctx* c);  // gturbo_adjoint.cpp
 // Runs the deferred end of the last step (its last stage and forcing), if

@@ -246,7 +246,7 @@ void draw_phases(gt_ens* e, int b, int steps) {
       EnsMember& mb = e->mem[m];
       const int nf = mb.ctx->nf;
       double2* out = e->ph_host[b] + (size_t)mb.first * steps;
-      for (int s = 0; s < steps; ++s) forcing_phases(nf, &mb.seed, out + (size_t)s * nf);
+      for (int s = 0; s < steps; ++s) forcing_phases(nf, &mb.seed, &out[(size_t)s * nf].x);
     }
   };
   std::vector<std::thread> th;

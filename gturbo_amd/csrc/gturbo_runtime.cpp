@@ -381,22 +381,6 @@ int r_pass(gt_ctx* c, const gt::PassArgs& a) {
   return GT_OK;
 }
 
-// Forcing phases of one call: nf draws of rann (src/forcing.f90:40-51),
-// te = pi2*rann with pi2 = 2*3.14159265358979 (src/forcing.f90:10), and
-// (cos te, sin te) evaluated in extended precision and rounded once: the
-// correctly rounded values, identical whichever compiler built the caller.
-void forcing_phases(int nf, int32_t* seed, double2* out) {
-  const double pi2 = 2.0 * 3.14159265358979;
-  uint32_t s = (uint32_t)*seed;
-  for (int k = 0; k < nf; ++k) {
-    s = (69069u * s + 1u) & 0x7FFFFFFFu;
-    const float r = (float)((double)s / (double)0x7FFFFFFF);
-    const double te = pi2 * (double)r;
-    out[k] = make_double2((double)cosl((long double)te), (double)sinl((long double)te));
-  }
-  *seed = (int32_t)s;
-}
-
 int ensure_diag(gt_ctx* c, const Rect& r) {
   const size_t nbin = c->n / 2;
   const size_t need = 2 * (size_t)(r.kc() + 1) * nbin + 2 * nbin + (size_t)r.kc() * 6 + 6;
@@ -444,24 +428,30 @@ int same_rect(gt_ctx* c, Mirror& a, Mirror& b) {
   return GT_OK;
 }
 
-// src/forcing.f90 on a compact field: the phases of this call (host LCG)
-// go through a ring of pinned slots to the device.
 // The next forcing draws (src/forcing.f90:16-24) into a free slot of the
-// phase ring, copied to the device on the stream; the slot is marked used
-// once its reader is launched (slot_read).
+// phase ring.  N <= 1024: the kernels read the pinned slot itself (the
+// readers are one thread per mode or one column's waves, beside their other
+// loads), no copy; a copy command between two passes cost 6-8 us of a step
+// of 55-80 us.  Larger grids, whose step boundary reads phases one after the
+// other, read a device copy made on the stream.  Slots are drawn and read in
+// the same order; an event after the last reader of each run of kRingSeg
+// slots guards its reuse (slot_read).
 int forcing_upload(gt_ctx* c, int32_t* seed, unsigned* slot_out) {
-  const unsigned slot = c->ph_next++ % kRing;
-  if (c->ph_ev_used[slot]) HIPCHK(hipEventSynchronize(c->ph_ev[slot]));
+  const unsigned slot = c->ph_next++ % kRing, seg = slot / kRingSeg;
+  if (slot % kRingSeg == 0 && c->ph_ev_used[seg]) HIPCHK(hipEventSynchronize(c->ph_ev[seg]));
   double2* hp = c->ph_host + (size_t)slot * c->nf;
-  double2* dp = c->ph_dev + (size_t)slot * c->nf;
-  forcing_phases(c->nf, seed, hp);
-  HIPCHK(hipMemcpyAsync(dp, hp, sizeof(double2) * c->nf, hipMemcpyHostToDevice, c->stream));
+  forcing_phases(c->nf, seed, &hp->x);
+  if (!c->ph_direct)
+    HIPCHK(hipMemcpyAsync(c->ph_dev + (size_t)slot * c->nf, hp, sizeof(double2) * c->nf,
+                          hipMemcpyHostToDevice, c->stream));
   *slot_out = slot;
   return GT_OK;
 }
 int slot_read(gt_ctx* c, unsigned slot) {
-  HIPCHK(hipEventRecord(c->ph_ev[slot], c->stream));
-  c->ph_ev_used[slot] = true;
+  if (slot % kRingSeg == kRingSeg - 1) {
+    HIPCHK(hipEventRecord(c->ph_ev[slot / kRingSeg], c->stream));
+    c->ph_ev_used[slot / kRingSeg] = true;
+  }
   return GT_OK;
 }
 int forcing_slot(gt_ctx* c, RectTables* t, double2* z, unsigned slot) {
@@ -472,6 +462,7 @@ int forcing_slot(gt_ctx* c, RectTables* t, double2* z, unsigned slot) {
   }
   return slot_read(c, slot);
 }
+// src/forcing.f90 on a compact field.
 int forcing_on(gt_ctx* c, RectTables* t, double2* z, int32_t* seed) {
   if (c->nf == 0) return GT_OK;
   unsigned slot;
@@ -633,9 +624,17 @@ int gt_create(int32_t n, const double* p, gt_ctx** out) {
   // the allocation-free glob's partial sums on this device (resolved once)
   CREATE_HIP(gt::glob_scratch(&c->glob_scratch, &c->glob_scratch_n));
   const int nfa = c->nf > 0 ? c->nf : 1;
-  CREATE_HIP(hipHostMalloc(&c->ph_host, sizeof(double2) * nfa * kRing, hipHostMallocDefault));
-  CREATE_HIP(hipMalloc(&c->ph_dev, sizeof(double2) * nfa * kRing));
-  for (int i = 0; i < kRing; ++i) CREATE_HIP(hipEventCreateWithFlags(&c->ph_ev[i], hipEventDisableTiming));
+  c->ph_direct = c->logn <= gt::kFpMaxLogn;
+  CREATE_HIP(hipHostMalloc(&c->ph_host, sizeof(double2) * nfa * kRing,
+                           hipHostMallocCoherent | hipHostMallocMapped));
+  if (c->ph_direct) {
+    void* d = nullptr;
+    CREATE_HIP(hipHostGetDevicePointer(&d, c->ph_host, 0));
+    c->ph_dev = static_cast<double2*>(d);
+  } else {
+    CREATE_HIP(hipMalloc(&c->ph_dev, sizeof(double2) * nfa * kRing));
+  }
+  for (auto& e : c->ph_ev) CREATE_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   *out = c;
   return GT_OK;
 }
@@ -663,9 +662,9 @@ int gt_destroy(gt_ctx* c) {
   if (c->flag) (void)hipFree(c->flag);
   if (c->dg) (void)hipFree(c->dg);
   if (c->ph_host) (void)hipHostFree(c->ph_host);
-  if (c->ph_dev) (void)hipFree(c->ph_dev);
-  for (int i = 0; i < kRing; ++i)
-    if (c->ph_ev[i]) (void)hipEventDestroy(c->ph_ev[i]);
+  if (c->ph_dev && !c->ph_direct) (void)hipFree(c->ph_dev);
+  for (hipEvent_t e : c->ph_ev)
+    if (e) (void)hipEventDestroy(e);
   for (auto& t : c->tl) {
     (void)hipEventDestroy(t.a);
     (void)hipEventDestroy(t.b);
