@@ -119,9 +119,8 @@ enum CMode : int {
   C_RK2_2S = 9,
 };
 
-// Column-tile width of the y pass (BT), y rows per workgroup of the x pass,
-// and row pairs per workgroup of the reference-layout transforms, per
-// log2 N.  A line is N/8 threads and (N + N/16) double2 of LDS.  Two
+// Column-tile width of the y pass (BT) and y rows per workgroup of the x
+// pass, per log2 N.  A line is N/8 threads and (N + N/16) double2 of LDS.  Two
 // columns (rows) per workgroup up to N = 4096: a 4-row block of two columns
 // is one 128-byte line, and small grids get as many workgroups as there
 // are column pairs (wider tiles left 256^2 with six y workgroups).
@@ -130,10 +129,6 @@ __host__ __device__ constexpr int rows_of(int logn) { return logn <= 12 ? 2 : 1;
 // Largest log2 N of the single-run passes that run a column's or row's
 // fields side by side (f_pass, fx_pass in gturbo_kernels.hip).
 constexpr int kFpMaxLogn = 10;
-__host__ __device__ constexpr int rp_of(int logn) {
-  return logn <= 6 ? (1 << (logn - 1)) : logn == 7 ? 32 : logn == 8 ? 16
-       : logn == 9 ? 8 : logn == 10 ? 4 : logn == 11 ? 2 : 1;
-}
 
 // Layout of the fields between the passes: rows in groups of kYR; group g
 // of a field holds, tile after tile, a block of kYR rows x BT columns.  The
@@ -218,11 +213,28 @@ struct EnsForce {
 constexpr int kEnsMinLogn = 7, kEnsMaxLogn = 11;
 __host__ __device__ constexpr int ens_lines(int t, int logn) { return t * 8 >> logn; }
 
+// 2D transform of a physical field in the reference layout to (dir < 0, with
+// /NY/NX) or from (dir > 0) a compact spectrum; y: io_size double2 of scratch.
+struct IoArgs {
+  int dir;
+  Phys ph;
+  double* ref;
+  const double2* tw;
+  double2* y;
+  Rect rc;
+  int kyp;
+  double2* cmp;
+  int apply_trunc;  // dir < 0: the mask of src/trunc.f90
+};
+inline size_t io_size(int logn, const Rect& rc) {
+  const int bt = bt_of(logn);
+  return (size_t)((rc.kc() + bt - 1) / bt * bt) << logn;
+}
+
 // Host-side launchers (gturbo_kernels.hip).
 hipError_t launch_c_pass(int logn, int mode, const PassArgs& a, hipStream_t s);
 hipError_t launch_r_pass(int logn, const PassArgs& a, hipStream_t s);
-hipError_t launch_ref_fft(int logn, int dir, double* z, const double2* tw,
-                          hipStream_t s);
+hipError_t launch_io(int logn, const IoArgs& a, hipStream_t s);
 hipError_t launch_j_pass(int logn, int mode, const AdjArgs& a, hipStream_t s);
 hipError_t launch_jr_pass(int logn, const AdjArgs& a, hipStream_t s);
 hipError_t launch_produ(int n, const double* z, double* u, double* v,
@@ -232,6 +244,11 @@ hipError_t launch_trunc_cmp(const Phys& ph, const Rect& rc, int kyp,
                             double2* z, hipStream_t s);
 hipError_t launch_gather(const Phys& ph, const Rect& rc, int kyp,
                          const double* ref, double2* cmp, int apply_trunc,
+                         int* outside_flag, hipStream_t s);
+// Compact rectangle rf -> smaller rectangle rc; with outside_flag, flags a
+// nonzero mode of rf outside rc.
+hipError_t launch_narrow(const Phys& ph, const Rect& rf, int kypf, const double2* src,
+                         const Rect& rc, int kyp, double2* dst, int apply_trunc,
                          int* outside_flag, hipStream_t s);
 hipError_t launch_scatter(const Phys& ph, const Rect& rc, int kyp,
                           const double2* cmp, double* ref, hipStream_t s);

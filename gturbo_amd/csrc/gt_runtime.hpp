@@ -52,6 +52,9 @@ struct Mirror {
   int kyp = 0;
   bool ref_valid = true;
   bool cmp_valid = false;
+  // compact copy on the full rectangle straight from fft_dir: whether its
+  // modes outside the 2/3 rectangle vanish has not been looked at
+  bool wide = false;
 };
 
 struct RectTables {
@@ -109,8 +112,9 @@ struct gt_ctx {
   gtr::RectTables tab[2];  // [0] truncated rect, [1] full rect
   double2* y1 = nullptr;
   double2* y2 = nullptr;
-  size_t ycap = 0;  // double2 per field
+  size_t y1cap = 0, y2cap = 0;  // double2
   int* flag = nullptr;
+  double2* spare = nullptr;  // one full-rectangle compact field (narrow)
 
   // forcing phases
   double2* ph_host = nullptr;  // pinned, kRing * nf
@@ -145,11 +149,17 @@ struct gt_ctx {
 namespace gtr {
 
 int ilog2(int n);
+int ctx_create(int32_t n, const double* params, gt_ctx** out);
 int kyp_of(const Rect& r);
 int rect_kind(const gt_ctx* c, const Rect& r);
 int rect_tables(gt_ctx* c, const Rect& r, RectTables** out);
 int rect_ka(gt_ctx* c, const Rect& r, const double** out);
 int ensure_ybuf(gt_ctx* c, const Rect& r);
+int ensure_io(gt_ctx* c, const Rect& r);
+// fft_dir (with or without trunc) of a physical field into a compact one on
+// rectangle r, and fft_inv of a compact one; scratch is the y1 buffer.
+int io_forward(gt_ctx* c, const double* ref, const Rect& r, double2* cmp, int apply_trunc);
+int io_inverse(gt_ctx* c, const double2* cmp, const Rect& r, double* ref);
 int lookup(gt_ctx* c, const void* host, Mirror** m);
 int alloc_cmp(gt_ctx* c, Mirror& m, const Rect& r);
 int ensure_ref(gt_ctx* c, Mirror& m);

@@ -37,7 +37,6 @@ struct AdjState {
   double2* lacc = nullptr;
   double2* y1 = nullptr;         // 5 fields between the adjoint passes
   double2* y2 = nullptr;         // 3 fields
-  double* tmp = nullptr;         // one reference-layout field
 };
 
 namespace gtr {
@@ -48,7 +47,7 @@ void adj_free(gt_ctx* c) {
   for (double2* p : s->ck)
     if (p) (void)hipFree(p);
   for (void* p : {(void*)s->z, (void*)s->znew, (void*)s->stages, (void*)s->lam,
-                  (void*)s->lacc, (void*)s->y1, (void*)s->y2, (void*)s->tmp})
+                  (void*)s->lacc, (void*)s->y1, (void*)s->y2})
     if (p) (void)hipFree(p);
   delete s;
   c->adj = nullptr;
@@ -87,7 +86,6 @@ int adj_alloc(gt_ctx* c, int nsteps, int kchk) {
     HIPCHK(hipMalloc(&s->lacc, sizeof(double2) * nc));
     HIPCHK(hipMalloc(&s->y1, sizeof(double2) * ycap * 5));
     HIPCHK(hipMalloc(&s->y2, sizeof(double2) * ycap * 3));
-    HIPCHK(hipMalloc(&s->tmp, sizeof(double) * ((size_t)c->n + 2) * c->n));
     for (double2* p : {s->z, s->znew, s->lam, s->lacc})
       HIPCHK(hipMemsetAsync(p, 0, sizeof(double2) * nc, c->stream));
     HIPCHK(hipMemsetAsync(s->stages, 0, sizeof(double2) * nc * nstage * kchk, c->stream));
@@ -107,20 +105,12 @@ int adj_alloc(gt_ctx* c, int nsteps, int kchk) {
 
 // Compact state from a physical field: fft_dir and trunc (src/main.f90:89-92).
 int from_physical(gt_ctx* c, const double* dref, double2* out) {
-  AdjState* s = c->adj;
-  const size_t bytes = sizeof(double) * ((size_t)c->n + 2) * c->n;
-  HIPCHK(hipMemcpyAsync(s->tmp, dref, bytes, hipMemcpyDeviceToDevice, c->stream));
-  HIPCHK(gt::launch_ref_fft(c->logn, -1, s->tmp, c->tw, c->stream));
-  HIPCHK(gt::launch_gather(c->ph, s->rc, s->kyp, s->tmp, out, 1, nullptr, c->stream));
-  return GT_OK;
+  return io_forward(c, dref, c->adj->rc, out, 1);
 }
 
 // Physical field of a compact state: fft_inv (src/main.f90:143).
 int to_physical(gt_ctx* c, const double2* in, double* dref) {
-  AdjState* s = c->adj;
-  HIPCHK(gt::launch_scatter(c->ph, s->rc, s->kyp, in, dref, c->stream));
-  HIPCHK(gt::launch_ref_fft(c->logn, +1, dref, c->tw, c->stream));
-  return GT_OK;
+  return io_inverse(c, in, c->adj->rc, dref);
 }
 
 // One step of src/rkstep.f90 on the working state; with slot >= 0 every

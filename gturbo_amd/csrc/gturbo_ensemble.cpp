@@ -357,7 +357,7 @@ int gt_ens_create(int32_t nmem, const int32_t* n, const double* params, gt_ens**
   int first = 0;
   for (int m = 0; m < nmem; ++m) {
     EnsMember& mb = e->mem[m];
-    ENS_CHK(gt_create(n[m], params + 17 * (size_t)m, &mb.ctx));
+    ENS_CHK(ctx_create(n[m], params + 17 * (size_t)m, &mb.ctx));
     gt_ctx* c = mb.ctx;
     if (m == 0) e->rko = c->rko;
     if (c->rko != e->rko)
@@ -431,12 +431,12 @@ int gt_ens_set_field(gt_ens* e, int32_t m, const double* z, int32_t space) {
   HIPCHK(hipMalloc(&tmp, bytes));
   int flag = 0;
   hipError_t err = hipMemcpyAsync(tmp, z, bytes, hipMemcpyHostToDevice, e->stream);
-  if (err == hipSuccess && space == GT_SPACE_PHYSICAL)
-    err = gt::launch_ref_fft(c->logn, -1, tmp, c->tw, e->stream);  // fft_dir
   if (err == hipSuccess) err = hipMemsetAsync(e->flag, 0, sizeof(int), e->stream);
-  if (err == hipSuccess)  // trunc (physical input) or the rectangle as is
-    err = gt::launch_gather(c->ph, mb.rc, mb.kyp, tmp, mb.z, space == GT_SPACE_PHYSICAL,
-                            space == GT_SPACE_SPECTRAL ? e->flag : nullptr, e->stream);
+  if (err == hipSuccess && space == GT_SPACE_PHYSICAL)  // fft_dir and trunc
+    err = gt::launch_io(c->logn, {-1, c->ph, tmp, c->tw, mb.y1, mb.rc, mb.kyp, mb.z, 1},
+                        e->stream);
+  if (err == hipSuccess && space == GT_SPACE_SPECTRAL)  // the rectangle as is
+    err = gt::launch_gather(c->ph, mb.rc, mb.kyp, tmp, mb.z, 0, e->flag, e->stream);
   if (err == hipSuccess)
     err = hipMemcpyAsync(&flag, e->flag, sizeof(int), hipMemcpyDeviceToHost, e->stream);
   if (err == hipSuccess) err = hipStreamSynchronize(e->stream);
@@ -457,9 +457,11 @@ int gt_ens_get_field(gt_ens* e, int32_t m, double* z, int32_t space) {
   const size_t bytes = ((size_t)c->n + 2) * c->n * sizeof(double);
   double* tmp = nullptr;
   HIPCHK(hipMalloc(&tmp, bytes));
-  hipError_t err = gt::launch_scatter(c->ph, mb.rc, mb.kyp, mb.z, tmp, e->stream);
-  if (err == hipSuccess && space == GT_SPACE_PHYSICAL)
-    err = gt::launch_ref_fft(c->logn, +1, tmp, c->tw, e->stream);  // fft_inv
+  hipError_t err =
+      space == GT_SPACE_PHYSICAL  // fft_inv
+          ? gt::launch_io(c->logn, {1, c->ph, tmp, c->tw, mb.y1, mb.rc, mb.kyp, mb.z, 0},
+                          e->stream)
+          : gt::launch_scatter(c->ph, mb.rc, mb.kyp, mb.z, tmp, e->stream);
   if (err == hipSuccess) err = hipMemcpyAsync(z, tmp, bytes, hipMemcpyDeviceToHost, e->stream);
   if (err == hipSuccess) err = hipStreamSynchronize(e->stream);
   (void)hipFree(tmp);

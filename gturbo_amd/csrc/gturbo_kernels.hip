@@ -1057,80 +1057,82 @@ __global__ void __launch_bounds__((1 << LOGN) / kE, 4)
 }
 
 // ---------------------------------------------------------------------------
-// Reference-layout 2D transforms (src/fft_dir.f90, src/fft_inv.f90):
-// real rows of N+2 doubles, half-spectrum rows of N/2+1 complex.
+// 2D transforms of a physical field in the reference layout (real rows of
+// N+2 doubles; src/fft_dir.f90, src/fft_inv.f90) to and from a spectrum in
+// the compact layout.  The x transforms (io_rows_*) and y transforms
+// (io_cols_*) meet in the passes' block layout: the y part then reads and
+// writes whole blocks on one side and contiguous columns on the other, and
+// only the kept columns travel.  A y transform in place on the reference
+// layout touches 16 or 32 bytes of each row's line.  Both directions with
+// trunc between them, 4096^2: 505 us with transforms in the reference layout
+// and gather/scatter, IO4096_US us; 8192^2: 3040 and IO8192_US us.
 // ---------------------------------------------------------------------------
 
+// Physical row held by slot s of a column: the in-place transforms' order at
+// N = 4096 and 8192 (see c_body), else s.
 template <int LOGN>
-__global__ void __launch_bounds__(rp_of(LOGN) * (1 << LOGN) / kE)
-    ref_rows_fwd(double* z, const double2* __restrict__ tw) {
-  constexpr int N = 1 << LOGN, TPL = N / kE, RP = rp_of(LOGN);
+__device__ __forceinline__ int slot_row(int s) {
+  auto d = [](int j) { return 64 * (j & 7) + 8 * ((j >> 3) & 7) + (j >> 6); };
+  if constexpr (LOGN == 12) return d(s & 511) + (s & ~511);
+  else if constexpr (LOGN == 13) return 2 * (d(s & 511) + 512 * (s >> 10)) + ((s >> 9) & 1);
+  else return s;
+}
+
+// Row pairs per workgroup of the x parts: one wave's worth of short lines.
+__host__ __device__ constexpr int io_pairs(int logn) {
+  return logn >= 9 ? 1 : logn == 4 ? 8 : 512 >> logn;
+}
+template <int LOGN, int S>
+__device__ __forceinline__ void io_fft(double2* w, double2* buf, int j,
+                                       const double2* __restrict__ tw) {
+  if constexpr (line_in_wave<LOGN>()) fft_held<LOGN, S>(w, buf, j, held_tw<LOGN>(tw, j));
+  else fft_reg<LOGN, S>(w, buf, j, tw);
+}
+
+// Slots 2i, 2i+1 (two real rows per complex transform) -> block layout,
+// columns kx <= kxm.
+template <int LOGN>
+__global__ void __launch_bounds__(io_pairs(LOGN) * (1 << LOGN) / kE)
+    io_rows_fwd(const double* __restrict__ z, const double2* __restrict__ tw,
+                double2* __restrict__ y, int ntiles, int kxm) {
+  constexpr int N = 1 << LOGN, TPL = N / kE, RP = io_pairs(LOGN), BT = bt_of(LOGN);
   constexpr int LINE = Line<LOGN>::PADDED;
   __shared__ double2 lds[RP * LINE];
   const int pl = threadIdx.x / TPL, j = threadIdx.x % TPL;
-  const int y0 = 2 * (blockIdx.x * RP + pl);
+  const int s0 = 2 * (xcd_remap(blockIdx.x, gridDim.x) * RP + pl);
   double2* buf = lds + pl * LINE;
   const size_t ld = (size_t)N + 2;
-  const double* r0 = z + ld * y0;
-  const double* r1 = r0 + ld;
+  const double* r0 = z + ld * slot_row<LOGN>(s0);
+  const double* r1 = z + ld * slot_row<LOGN>(s0 + 1);
   double2 w[kE];
 #pragma unroll
   for (int r = 0; r < kE; ++r) {
     const int x = j + TPL * r;
     w[r] = make_double2(r0[x], r1[x]);
   }
-  fft_reg<LOGN, -1>(w, buf, j, tw);
-  double2* pj = buf + lpad(j);
-#pragma unroll
-  for (int r = 0; r < kE; ++r) pj[lpad_off(TPL * r)] = w[r];
-  __syncthreads();  // also orders every read of the real rows before the writes
-  const double2* pm = buf + lpad(TPL - j);
-  double2* c0 = reinterpret_cast<double2*>(z + ld * y0);
-  double2* c1 = c0 + (N / 2 + 1);
-#pragma unroll
-  for (int r = 0; r < kE; ++r) {
-    const int k = j + TPL * r;
-    if (k <= N / 2) {
-      const double2 W = w[r];
-      const double2 Wc = mirror_at<LOGN>(buf, pm, j, r);
-      c0[k] = make_double2(0.5 * (W.x + Wc.x), 0.5 * (W.y - Wc.y));
-      c1[k] = make_double2(0.5 * (W.y + Wc.y), -0.5 * (W.x - Wc.x));
-    }
-  }
+  io_fft<LOGN, -1>(w, buf, j, tw);
+  if constexpr (line_in_wave<LOGN>()) wave_sync();
+  const unsigned off = yrow_off(s0, ntiles, BT);
+  split_store<LOGN, 0, BT>(w, buf, j, y, off, off + BT, kxm);
 }
 
 template <int LOGN>
-__global__ void __launch_bounds__(rp_of(LOGN) * (1 << LOGN) / kE)
-    ref_rows_inv(double* z, const double2* __restrict__ tw) {
-  constexpr int N = 1 << LOGN, TPL = N / kE, RP = rp_of(LOGN);
+__global__ void __launch_bounds__(io_pairs(LOGN) * (1 << LOGN) / kE)
+    io_rows_inv(double* __restrict__ z, const double2* __restrict__ tw,
+                const double2* __restrict__ y, int ntiles, int kxm) {
+  constexpr int N = 1 << LOGN, TPL = N / kE, RP = io_pairs(LOGN), BT = bt_of(LOGN);
   constexpr int LINE = Line<LOGN>::PADDED;
   __shared__ double2 lds[RP * LINE];
   const int pl = threadIdx.x / TPL, j = threadIdx.x % TPL;
-  const int y0 = 2 * (blockIdx.x * RP + pl);
+  const int s0 = 2 * (xcd_remap(blockIdx.x, gridDim.x) * RP + pl);
   double2* buf = lds + pl * LINE;
-  const size_t ld = (size_t)N + 2;
-  const double2* c0 = reinterpret_cast<const double2*>(z + ld * y0);
-  const double2* c1 = c0 + (N / 2 + 1);
+  const unsigned off = yrow_off(s0, ntiles, BT);
   double2 w[kE];
-#pragma unroll
-  for (int r = 0; r < kE; ++r) {
-    const int p = j + TPL * r;
-    double2 v;
-    if (p == 0 || p == N / 2) {
-      v = make_double2(c0[p].x, c1[p].x);
-    } else if (p < N / 2) {
-      const double2 x0 = c0[p], x1 = c1[p];
-      v = make_double2(x0.x - x1.y, x0.y + x1.x);
-    } else {
-      const double2 x0 = c0[N - p], x1 = c1[N - p];
-      v = make_double2(x0.x + x1.y, x1.x - x0.y);
-    }
-    w[r] = v;
-  }
-  __syncthreads();  // every read of the complex rows before any write
-  fft_reg<LOGN, +1>(w, buf, j, tw);
-  double* r0 = z + ld * y0;
-  double* r1 = r0 + ld;
+  build_two<LOGN, 0, BT>(w, j, y, off, off + BT, kxm);
+  io_fft<LOGN, +1>(w, buf, j, tw);
+  const size_t ld = (size_t)N + 2;
+  double* r0 = z + ld * slot_row<LOGN>(s0);
+  double* r1 = z + ld * slot_row<LOGN>(s0 + 1);
 #pragma unroll
   for (int r = 0; r < kE; ++r) {
     const int x = j + TPL * r;
@@ -1143,35 +1145,90 @@ __global__ void __launch_bounds__(rp_of(LOGN) * (1 << LOGN) / kE)
   }
 }
 
-// y transform of every kx column in place; SCALE applies /NY/NX.
-template <int LOGN, int S, int SCALE>
-__global__ void __launch_bounds__(bt_of(LOGN) * (1 << LOGN) / kE)
-    ref_cols(double* z, const double2* __restrict__ tw) {
-  constexpr int N = 1 << LOGN, TPL = N / kE, BT = bt_of(LOGN);
-  constexpr int LINE = Line<LOGN>::PADDED, NH = N / 2 + 1;
-  __shared__ double2 lds[BT * LINE];
-  const int tid = threadIdx.x;
+// Columns per workgroup of the y parts.
+__host__ __device__ constexpr int io_cols(int logn) {
+  return logn <= 8 ? 512 >> logn : bt_of(logn);
+}
+template <int LOGN>
+__host__ __device__ constexpr int io_line() {
+  return LOGN == 12 ? kIpLine : LOGN == 13 ? 2 * kIpLine : Line<LOGN>::PADDED;
+}
+// Thread -> (column in workgroup, index in line); each line whole waves (or
+// a wave's share) as the in-place transforms need.
+template <int LOGN>
+__device__ __forceinline__ void io_map(int tid, int& b, int& j) {
+  constexpr int TPL = (1 << LOGN) / kE;
+  if constexpr (LOGN == 12) {
+    b = (tid >> 6) & 1;
+    j = ((tid >> 7) << 6) | (tid & 63);
+  } else {
+    b = tid / TPL;
+    j = tid % TPL;
+  }
+}
+
+// Block layout -> compact column, /NY/NX (src/fft_dir.f90:19; a power of
+// two: exact), with the mask of src/trunc.f90 when apply_trunc is set.
+template <int LOGN>
+__global__ void __launch_bounds__(io_cols(LOGN) * (1 << LOGN) / kE)
+    io_cols_fwd(Phys ph, const double2* __restrict__ tw, const double2* __restrict__ y,
+                int ntiles, Rect rc, int kyp, double2* __restrict__ cmp, int apply_trunc) {
+  constexpr int N = 1 << LOGN, TPL = N / kE, CW = io_cols(LOGN), BT = bt_of(LOGN);
+  __shared__ double2 lds[CW * io_line<LOGN>()];
   int b, j;
-  line_map<TPL, BT>(tid, b, j);
-  const int kx = blockIdx.x * BT + b;
-  const bool ok = kx < NH;
-  double2* zc = reinterpret_cast<double2*>(z);
+  io_map<LOGN>(threadIdx.x, b, j);
+  const int wg = LOGN == 13 ? xcd_remap(blockIdx.x, gridDim.x) : (int)blockIdx.x;
+  const int c = wg * CW + b;
+  const bool ok = c <= rc.kx;
+  double2* buf = lds + b * io_line<LOGN>();
+  const unsigned colo = ycol_off(c, BT);
   double2 w[kE];
 #pragma unroll
   for (int r = 0; r < kE; ++r)
-    w[r] = ok ? zc[kx + (size_t)NH * (j + TPL * r)] : make_double2(0.0, 0.0);
-  fft_reg<LOGN, S>(w, lds + b * LINE, j, tw);
-  if (ok) {
+    w[r] = ok ? y[yrow_off(j + TPL * r, ntiles, BT) + colo] : make_double2(0.0, 0.0);
+  if constexpr (LOGN == 12) fft_dit<-1>(w, buf, j, tw);
+  else if constexpr (LOGN == 13) fft_dit2<-1>(w, buf, j, tw);
+  else io_fft<LOGN, -1>(w, buf, j, tw);
+  if (!ok) return;
+  const double fkx = (double)c * ph.dkx;
 #pragma unroll
-    for (int r = 0; r < kE; ++r) {
-      double2 v = w[r];
-      if (SCALE) {
-        v.x = v.x / (double)N / (double)N;
-        v.y = v.y / (double)N / (double)N;
-      }
-      zc[kx + (size_t)NH * (j + TPL * r)] = v;
-    }
+  for (int r = 0; r < kE; ++r) {
+    const int p = j + TPL * r, row = row_of(p, rc, N);
+    if (row < 0) continue;
+    double2 v = make_double2(w[r].x * ph.inv_n2, w[r].y * ph.inv_n2);
+    const double fky = (double)kyi_of(p, N) * ph.dky;
+    if (apply_trunc && (cut_mode(ph, fkx * fkx, fky * fky) || (c == 0 && p == 0)))
+      v = make_double2(0.0, 0.0);
+    cmp[(size_t)c * kyp + row] = v;
   }
+}
+
+// Compact column (zero outside the rectangle) -> block layout.
+template <int LOGN>
+__global__ void __launch_bounds__(io_cols(LOGN) * (1 << LOGN) / kE)
+    io_cols_inv(const double2* __restrict__ tw, double2* __restrict__ y, int ntiles, Rect rc,
+                int kyp, const double2* __restrict__ cmp) {
+  constexpr int N = 1 << LOGN, TPL = N / kE, CW = io_cols(LOGN), BT = bt_of(LOGN);
+  __shared__ double2 lds[CW * io_line<LOGN>()];
+  int b, j;
+  io_map<LOGN>(threadIdx.x, b, j);
+  const int wg = LOGN == 13 ? xcd_remap(blockIdx.x, gridDim.x) : (int)blockIdx.x;
+  const int c = wg * CW + b;
+  const bool ok = c <= rc.kx;
+  double2* buf = lds + b * io_line<LOGN>();
+  double2 w[kE];
+#pragma unroll
+  for (int r = 0; r < kE; ++r) {
+    const int row = row_of(j + TPL * r, rc, N);
+    w[r] = ok && row >= 0 ? cmp[(size_t)c * kyp + row] : make_double2(0.0, 0.0);
+  }
+  if constexpr (LOGN == 12) fft_dif<+1>(w, buf, j, tw, false);
+  else if constexpr (LOGN == 13) fft_dif2<+1>(w, buf, j, tw, false);
+  else io_fft<LOGN, +1>(w, buf, j, tw);
+  if (!ok) return;
+  const unsigned colo = ycol_off(c, BT);
+#pragma unroll
+  for (int r = 0; r < kE; ++r) y[yrow_off(j + TPL * r, ntiles, BT) + colo] = w[r];
 }
 
 // ---------------------------------------------------------------------------
@@ -1426,7 +1483,7 @@ hipError_t c_pass_launch(int mode, const PassArgs& a, hipStream_t s);
 template <int L>
 hipError_t r_pass_launch(const PassArgs& a, hipStream_t s);
 template <int L>
-hipError_t ref_fft_launch(int dir, double* z, const double2* tw, hipStream_t s);
+hipError_t io_launch(const IoArgs& a, hipStream_t s);
 template <int L>
 hipError_t j_pass_launch(int mode, const AdjArgs& a, hipStream_t s);
 template <int L>
@@ -1506,16 +1563,17 @@ hipError_t r_pass_launch(const PassArgs& a, hipStream_t s) {
 }
 
 template <int L>
-hipError_t ref_fft_launch(int dir, double* z, const double2* tw, hipStream_t s) {
-  constexpr int N = 1 << L, RP = rp_of(L), BT = bt_of(L);
-  const dim3 gr(N / 2 / RP), br(RP * N / kE);
-  const dim3 gc((N / 2 + 1 + BT - 1) / BT), bc(BT * N / kE);
-  if (dir < 0) {  // fft_dir: rows R2C, columns forward, /NY/NX
-    ref_rows_fwd<L><<<gr, br, 0, s>>>(z, tw);
-    ref_cols<L, -1, 1><<<gc, bc, 0, s>>>(z, tw);
-  } else {  // fft_inv: columns inverse, rows C2R
-    ref_cols<L, +1, 0><<<gc, bc, 0, s>>>(z, tw);
-    ref_rows_inv<L><<<gr, br, 0, s>>>(z, tw);
+hipError_t io_launch(const IoArgs& a, hipStream_t s) {
+  constexpr int N = 1 << L, RP = io_pairs(L), CW = io_cols(L), BT = bt_of(L);
+  const dim3 gr(N / 2 / RP), br(RP * N / kE), bc(CW * N / kE);
+  const dim3 gc((a.rc.kc() + CW - 1) / CW);
+  const int nt = (a.rc.kc() + BT - 1) / BT;
+  if (a.dir < 0) {
+    io_rows_fwd<L><<<gr, br, 0, s>>>(a.ref, a.tw, a.y, nt, a.rc.kx);
+    io_cols_fwd<L><<<gc, bc, 0, s>>>(a.ph, a.tw, a.y, nt, a.rc, a.kyp, a.cmp, a.apply_trunc);
+  } else {
+    io_cols_inv<L><<<gc, bc, 0, s>>>(a.tw, a.y, nt, a.rc, a.kyp, a.cmp);
+    io_rows_inv<L><<<gr, br, 0, s>>>(a.ref, a.tw, a.y, nt, a.rc.kx);
   }
   return hipGetLastError();
 }
@@ -1557,7 +1615,7 @@ template hipError_t j_pass_launch<GT_INST_LOGN>(int, const AdjArgs&, hipStream_t
 template hipError_t jr_pass_launch<GT_INST_LOGN>(const AdjArgs&, hipStream_t);
 template hipError_t c_pass_launch<GT_INST_LOGN>(int, const PassArgs&, hipStream_t);
 template hipError_t r_pass_launch<GT_INST_LOGN>(const PassArgs&, hipStream_t);
-template hipError_t ref_fft_launch<GT_INST_LOGN>(int, double*, const double2*, hipStream_t);
+template hipError_t io_launch<GT_INST_LOGN>(const IoArgs&, hipStream_t);
 #endif  // GT_INST_LOGN
 
 #if defined(GT_INST_ENS)
@@ -1757,6 +1815,32 @@ __global__ void gather_k(Phys ph, Rect rc, int kyp, const double2* __restrict__ 
     }
     cmp[(size_t)c * kyp + r] = v;
   }
+}
+
+// Compact rectangle rf -> the smaller rectangle rc (optionally truncated):
+// one workgroup row per column, both sides contiguous.
+__global__ void narrow_k(Phys ph, Rect rf, int kypf, const double2* __restrict__ src, Rect rc,
+                         int kyp, double2* __restrict__ dst, int apply_trunc) {
+  const int n = ph.n, ky = rc.ky(), c = blockIdx.y;
+  const int r = blockIdx.x * blockDim.x + threadIdx.x;
+  if (r >= ky) return;
+  const int p = fft_of(r, rc, n);
+  double2 v = src[(size_t)c * kypf + row_of(p, rf, n)];
+  if (apply_trunc) {
+    const double fkx = (double)c * ph.dkx, fky = (double)kyi_of(p, n) * ph.dky;
+    if (cut_mode(ph, fkx * fkx, fky * fky) || (c == 0 && p == 0)) v = make_double2(0.0, 0.0);
+  }
+  dst[(size_t)c * kyp + r] = v;
+}
+
+// Flags a nonzero mode of compact rectangle rf outside rc.
+__global__ void outside_cmp_k(Phys ph, Rect rf, int kypf, const double2* __restrict__ src,
+                              Rect rc, int* flag) {
+  const int n = ph.n, c = blockIdx.y;
+  const int r = blockIdx.x * blockDim.x + threadIdx.x;
+  if (r >= rf.ky() || (c <= rc.kx && row_of(fft_of(r, rf, n), rc, n) >= 0)) return;
+  const double2 v = src[(size_t)c * kypf + r];
+  if (v.x != 0.0 || v.y != 0.0) atomicOr(flag, 1);
 }
 
 // ka = k2**(alpv/2) over the compact rectangle, with the expressions of the
@@ -2206,9 +2290,8 @@ hipError_t launch_jr_pass(int logn, const AdjArgs& a, hipStream_t s) {
   return hipSuccess;
 }
 
-hipError_t launch_ref_fft(int logn, int dir, double* z, const double2* tw,
-                          hipStream_t s) {
-  GT_LOGN_SWITCH(logn, return ref_fft_launch<L>(dir, z, tw, s));
+hipError_t launch_io(int logn, const IoArgs& a, hipStream_t s) {
+  GT_LOGN_SWITCH(logn, return io_launch<L>(a, s));
   return hipSuccess;
 }
 
@@ -2239,6 +2322,17 @@ hipError_t launch_gather(const Phys& ph, const Rect& rc, int kyp, const double* 
   if (outside_flag)
     outside_k<<<grid_for((size_t)(ph.n / 2 + 1) * ph.n, 256), 256, 0, s>>>(
         ph, rc, rc2, outside_flag);
+  return hipGetLastError();
+}
+
+hipError_t launch_narrow(const Phys& ph, const Rect& rf, int kypf, const double2* src,
+                         const Rect& rc, int kyp, double2* dst, int apply_trunc,
+                         int* outside_flag, hipStream_t s) {
+  if (outside_flag)
+    outside_cmp_k<<<dim3((rf.ky() + 255) / 256, rf.kc()), 256, 0, s>>>(ph, rf, kypf, src, rc,
+                                                                      outside_flag);
+  narrow_k<<<dim3((rc.ky() + 255) / 256, rc.kc()), 256, 0, s>>>(ph, rf, kypf, src, rc, kyp, dst,
+                                                               apply_trunc);
   return hipGetLastError();
 }
 

@@ -2,6 +2,7 @@
 // table of device copies, host tables and the C entry points of gturbo.h.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -254,22 +255,49 @@ int rect_ka(gt_ctx* c, const Rect& r, const double** out) {
   return GT_OK;
 }
 
-int ensure_ybuf(gt_ctx* c, const Rect& r) {
+// Never cleared: what a pass reads of a field it or the pass before wrote,
+// but for the column that fills up the last tile, whose values go nowhere.
+static int grow(double2** p, size_t* cap, size_t need) {
+  if (need <= *cap) return GT_OK;
+  if (*p) (void)hipFree(*p);
+  *p = nullptr;
+  *cap = 0;
+  HIPCHK(hipMalloc(p, sizeof(double2) * need));
+  *cap = need;
+  return GT_OK;
+}
+
+// double2 of one field between the passes: the tiles' columns (y1, y2), or
+// the y1 blocks' at N = 4096.
+static size_t yfield(const gt_ctx* c, const Rect& r) {
   const int bt = gt::bt_of(c->logn);
   const size_t ntiles = (size_t)(r.kc() + bt - 1) / bt;
-  // columns of a field: the tiles' (y1, y2), or the y1 blocks' at N = 4096
-  const size_t cols = std::max(ntiles * bt, (size_t)gt::y1_cols(r.kc()));
-  const size_t need = cols * (size_t)c->n;
-  if (need <= c->ycap) return GT_OK;
-  if (c->y1) (void)hipFree(c->y1);
-  if (c->y2) (void)hipFree(c->y2);
-  c->y1 = c->y2 = nullptr;
-  c->ycap = 0;
-  HIPCHK(hipMalloc(&c->y1, sizeof(double2) * need * 3));
-  HIPCHK(hipMalloc(&c->y2, sizeof(double2) * need * 2));
-  HIPCHK(hipMemsetAsync(c->y1, 0, sizeof(double2) * need * 3, c->stream));
-  HIPCHK(hipMemsetAsync(c->y2, 0, sizeof(double2) * need * 2, c->stream));
-  c->ycap = need;
+  return std::max(ntiles * bt, (size_t)gt::y1_cols(r.kc())) * (size_t)c->n;
+}
+
+int ensure_ybuf(gt_ctx* c, const Rect& r) {
+  CHK(grow(&c->y1, &c->y1cap, 3 * yfield(c, r)));
+  return grow(&c->y2, &c->y2cap, 2 * yfield(c, r));
+}
+
+// y1 as the scratch of a 2D transform on rectangle r, at the size the steps
+// will want.
+int ensure_io(gt_ctx* c, const Rect& r) {
+  return grow(&c->y1, &c->y1cap, std::max(gt::io_size(c->logn, r), 3 * yfield(c, c->rtr)));
+}
+
+int io_forward(gt_ctx* c, const double* ref, const Rect& r, double2* cmp, int apply_trunc) {
+  CHK(ensure_io(c, r));
+  const gt::IoArgs a{-1, c->ph, const_cast<double*>(ref), c->tw, c->y1, r, kyp_of(r), cmp,
+                     apply_trunc};
+  HIPCHK(gt::launch_io(c->logn, a, c->stream));
+  return GT_OK;
+}
+
+int io_inverse(gt_ctx* c, const double2* cmp, const Rect& r, double* ref) {
+  CHK(ensure_io(c, r));
+  const gt::IoArgs a{1, c->ph, ref, c->tw, c->y1, r, kyp_of(r), const_cast<double2*>(cmp), 0};
+  HIPCHK(gt::launch_io(c->logn, a, c->stream));
   return GT_OK;
 }
 
@@ -311,12 +339,57 @@ int ensure_ref(gt_ctx* c, Mirror& m) {
   return GT_OK;
 }
 
+static bool has_tr(const gt_ctx* c) {  // a truncated rectangle of its own
+  return c->truncate == 1 &&
+         (c->rtr.kx != c->rfull.kx || c->rtr.p != c->rfull.p || c->rtr.q != c->rfull.q);
+}
+
+static size_t full_size(const gt_ctx* c) {  // double2 of a full-rectangle compact field
+  return (size_t)c->rfull.kc() * kyp_of(c->rfull);
+}
+static int ensure_spare(gt_ctx* c) {
+  if (!has_tr(c) || c->spare) return GT_OK;
+  HIPCHK(hipMalloc(&c->spare, sizeof(double2) * full_size(c)));
+  return GT_OK;
+}
+
+// A full-rectangle compact field onto the truncated rectangle: with the mask
+// of trunc, or as it is if its modes outside vanish (else it stays).  The
+// result goes to the context's spare field, which the old one replaces.
+static int narrow(gt_ctx* c, Mirror& m, int apply_trunc) {
+  const Rect r = c->rtr;
+  if (!has_tr(c) || rect_kind(c, m.rect) == 0) return GT_OK;
+  const size_t full = full_size(c);
+  CHK(ensure_spare(c));
+  if (!apply_trunc) HIPCHK(hipMemsetAsync(c->flag, 0, sizeof(int), c->stream));
+  {
+    Timer t(c, GT_K_OTHER);
+    HIPCHK(gt::launch_narrow(c->ph, m.rect, m.kyp, m.dcmp, r, kyp_of(r), c->spare, apply_trunc,
+                             apply_trunc ? nullptr : c->flag, c->stream));
+  }
+  if (!apply_trunc) {
+    int flag = 0;
+    HIPCHK(hipMemcpyAsync(&flag, c->flag, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(hipStreamSynchronize(c->stream));
+    if (flag) return GT_OK;
+  }
+  std::swap(m.dcmp, c->spare);
+  m.cmp_cap = full;  // a full-rectangle field has exactly this capacity
+  m.rect = r;
+  m.kyp = kyp_of(r);
+  return GT_OK;
+}
+
 // Compact copy of a spectral field.  With the 2/3 rule on, the truncated
 // rectangle is used unless the field has nonzero modes outside it.
 int ensure_cmp(gt_ctx* c, Mirror& m) {
+  if (m.cmp_valid && m.wide) {
+    m.wide = false;
+    return narrow(c, m, 0);
+  }
   if (m.cmp_valid) return GT_OK;
   Rect r = c->rtr;
-  if (c->truncate == 1 && (r.kx != c->rfull.kx || r.p != c->rfull.p || r.q != c->rfull.q)) {
+  if (has_tr(c)) {
     HIPCHK(hipMemsetAsync(c->flag, 0, sizeof(int), c->stream));
     CHK(alloc_cmp(c, m, r));
     {
@@ -342,10 +415,12 @@ int ensure_cmp(gt_ctx* c, Mirror& m) {
 void set_cmp_only(Mirror& m) {
   m.cmp_valid = true;
   m.ref_valid = false;
+  m.wide = false;
 }
 void set_ref_only(Mirror& m) {
   m.ref_valid = true;
   m.cmp_valid = false;
+  m.wide = false;
 }
 
 int pass_args(gt_ctx* c, Mirror& z, RectTables* t, gt::PassArgs* out) {
@@ -514,19 +589,8 @@ static int step_start(gt_ctx* c, int kind, Mirror* m, Mirror* mn, const gt::Pass
   return c_pass(c, gt::C_START, a);
 }
 
-}  // namespace gtr
-
-// ===========================================================================
-// C ABI
-// ===========================================================================
-
-using namespace gtr;
-
-extern "C" {
-
-const char* gt_last_error(void) { return g_err.c_str(); }
-
-int gt_create(int32_t n, const double* p, gt_ctx** out) {
+// Tables and stream of one simulation, without field workspaces.
+int ctx_create(int32_t n, const double* p, gt_ctx** out) {
   if (!out || !p) return fail(GT_ERR_ARG, "null argument");
   *out = nullptr;
   if (n < 16 || n > 8192 || (n & (n - 1)))
@@ -639,6 +703,33 @@ int gt_create(int32_t n, const double* p, gt_ctx** out) {
   return GT_OK;
 }
 
+}  // namespace gtr
+
+// ===========================================================================
+// C ABI
+// ===========================================================================
+
+using namespace gtr;
+
+extern "C" {
+
+const char* gt_last_error(void) { return g_err.c_str(); }
+
+int gt_create(int32_t n, const double* p, gt_ctx** out) {
+  CHK(ctx_create(n, p, out));
+  gt_ctx* c = *out;
+  // the workspaces that a first fft_dir, trunc and step would otherwise allocate
+  int rc = ensure_io(c, c->rfull);
+  if (rc == GT_OK) rc = ensure_spare(c);
+  if (rc != GT_OK) {
+    std::string keep = g_err;
+    gt_destroy(c);
+    g_err = keep;
+    *out = nullptr;
+  }
+  return rc;
+}
+
 int gt_destroy(gt_ctx* c) {
   if (!c) return GT_OK;
   c->pend = Pending{};  // a deferred step end is dropped with the context
@@ -660,6 +751,7 @@ int gt_destroy(gt_ctx* c) {
   if (c->y1) (void)hipFree(c->y1);
   if (c->y2) (void)hipFree(c->y2);
   if (c->flag) (void)hipFree(c->flag);
+  if (c->spare) (void)hipFree(c->spare);
   if (c->dg) (void)hipFree(c->dg);
   if (c->ph_host) (void)hipHostFree(c->ph_host);
   if (c->ph_dev && !c->ph_direct) (void)hipFree(c->ph_dev);
@@ -849,6 +941,7 @@ int gt_copy(gt_ctx* c, void* dst, const void* src) {
     HIPCHK(hipMemcpyAsync(d->dcmp, s->dcmp, sizeof(double2) * (size_t)s->rect.kc() * s->kyp,
                           hipMemcpyDeviceToDevice, c->stream));
     d->cmp_valid = true;
+    d->wide = s->wide;
     d->ref_valid = false;
     if (s->ref_valid) {
       HIPCHK(hipMemcpyAsync(d->dref, s->dref, ((size_t)c->n + 2) * c->n * sizeof(double),
@@ -880,9 +973,12 @@ int gt_fft_dir(gt_ctx* c, double* z, int32_t plan) {
   Mirror* m;
   CHK(lookup(c, z, &m));
   CHK(ensure_ref(c, *m));
+  // the spectrum stays in the compact layout, every mode of it
+  CHK(alloc_cmp(c, *m, c->rfull));
   Timer t(c, GT_K_OTHER);
-  HIPCHK(gt::launch_ref_fft(c->logn, -1, m->dref, c->tw, c->stream));
-  set_ref_only(*m);
+  CHK(io_forward(c, m->dref, c->rfull, m->dcmp, 0));
+  set_cmp_only(*m);
+  m->wide = has_tr(c);
   return GT_OK;
 }
 
@@ -893,9 +989,14 @@ int gt_fft_inv(gt_ctx* c, double* z, int32_t plan) {
   if (plan != GT_PLAN_Z2D) return fail(GT_ERR_ARG, "fft_inv needs a Z2D plan (got %d)", plan);
   Mirror* m;
   CHK(lookup(c, z, &m));
-  CHK(ensure_ref(c, *m));
+  if (!m->ref_valid && !m->cmp_valid)
+    return fail(GT_ERR_ARG, "array %p has no valid device data", m->host);
+  if (m->ref_valid) {  // a spectrum in the reference layout, all of it
+    CHK(alloc_cmp(c, *m, c->rfull));
+    HIPCHK(gt::launch_gather(c->ph, m->rect, m->kyp, m->dref, m->dcmp, 0, nullptr, c->stream));
+  }
   Timer t(c, GT_K_OTHER);
-  HIPCHK(gt::launch_ref_fft(c->logn, +1, m->dref, c->tw, c->stream));
+  CHK(io_inverse(c, m->dcmp, m->rect, m->dref));
   set_ref_only(*m);
   return GT_OK;
 }
@@ -926,7 +1027,11 @@ int gt_trunc(gt_ctx* c, double* z) {
   CHK(lookup(c, z, &m));
   Timer t(c, GT_K_OTHER);
   if (m->cmp_valid) {
-    HIPCHK(gt::launch_trunc_cmp(c->ph, m->rect, m->kyp, m->dcmp, c->stream));
+    if (m->wide) {
+      CHK(narrow(c, *m, 1));
+    } else {
+      HIPCHK(gt::launch_trunc_cmp(c->ph, m->rect, m->kyp, m->dcmp, c->stream));
+    }
     set_cmp_only(*m);
     return GT_OK;
   }

@@ -53,3 +53,50 @@ def test_forcing_phase_ring_wraps(oracle_mod):
     """150 forced steps: every slot of the phase ring is used again.  A step
     adds round-off of order 1e-16; 1e-12 over 150 steps."""
     assert _steps(oracle_mod, params_for(64), 150) < 1e-12
+
+
+@pytest.mark.parametrize("n", [16, 128, 2048])
+def test_consumers_of_fft_dir(oracle_mod, n):
+    """fft_dir leaves its spectrum on the whole half-spectrum: trunc of it, a
+    step of it without trunc (modes outside the 2/3 rectangle), the same of a
+    copy, fft_inv of each, and trunc of an array that was transformed before
+    it served as the accumulator.  1e-12 as for the other comparisons."""
+    p = params_for(n)
+    s, o = Solver(p), oracle_mod.Oracle(p)
+    rng = np.random.default_rng(n)
+    w = np.zeros((n, n + 2))
+    w[:, :n] = rng.standard_normal((n, n)) * (4.0 / n)
+    a, b, c = w.copy(), w.copy(), w.copy()
+    ag, bg, cg = w.copy(), s.field(), w.copy()
+    znl, u, v = (s.field() for _ in range(3))
+    for x in (ag, bg, cg, znl, u, v):
+        s.enter_data(x)
+
+    def same(xg, x):
+        s.update_host(xg)
+        assert _rel(xg, x) < 1e-12
+
+    for x in (a, b, c):
+        o.fft_dir(x)
+    s.fft_dir(ag)
+    s.copy(bg, ag)
+    s.trunc(ag)
+    o.trunc(a)
+    s.fft_dir(cg)
+    s.step4(bg, znl, cg, u, v)  # cg: accumulator from here on
+    o.step4(b)
+    same(ag, a)
+    same(bg, b)
+    s.step4(ag, znl, cg, u, v)
+    o.step4(a)
+    s.synchronize()
+    s.trunc(cg)
+    s.update_host(cg)
+    assert cg[0, 0] == 0.0 and cg[0, 1] == 0.0
+    kc = s.rect[0]
+    assert not np.any(np.ascontiguousarray(cg).view(np.complex128)[:, kc + 1:])
+    for xg, x in ((ag, a), (bg, b)):
+        s.fft_inv(xg)
+        o.fft_inv(x)
+        same(xg, x)
+    s.close()
