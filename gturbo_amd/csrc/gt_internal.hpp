@@ -91,6 +91,7 @@ struct AdjArgs {
   double2* lam;          // adjoint state: lambda' in, lambda out (J_END)
   double2* lacc;         // the step's adjoint accumulator
   const double* emk;
+  const double* ka;      // k2**(alpv/2) (compact), N <= 512 with alpv != 2
   const double2* snext;  // stage state of the next transposed term
 };
 
@@ -102,6 +103,8 @@ enum JMode : int {
   J_END = 4,     // a_s1 in: lambda = lacc + a_s1
   J_START2 = 5,  // RK2: lacc = E^2 mu, a = dt E mu (s2)
   J_RK2_1 = 6,   // a_s2 in: lacc += E a_s2, a = dt/2 E a_s2 (s1)
+  J_BOUND4 = 7,  // J_END of one step and J_START4 of the step before it
+  J_BOUND2 = 8,  // J_END and J_START2 likewise
 };
 
 enum CMode : int {
@@ -129,6 +132,8 @@ __host__ __device__ constexpr int rows_of(int logn) { return logn <= 12 ? 2 : 1;
 // Largest log2 N of the single-run passes that run a column's or row's
 // fields side by side (f_pass, fx_pass in gturbo_kernels.hip).
 constexpr int kFpMaxLogn = 10;
+// The same for the adjoint passes (fj_pass, fjr_pass; measured there).
+constexpr int kFjMaxLogn = 9;
 
 // Layout of the fields between the passes: rows in groups of kYR; group g
 // of a field holds, tile after tile, a block of kYR rows x BT columns.  The

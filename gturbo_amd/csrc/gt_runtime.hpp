@@ -170,6 +170,8 @@ int pass_args(gt_ctx* c, Mirror& z, RectTables* t, gt::PassArgs* out);
 int c_pass(gt_ctx* c, int mode, const gt::PassArgs& a);
 int r_pass(gt_ctx* c, const gt::PassArgs& a);
 int forcing_on(gt_ctx* c, RectTables* t, double2* z, int32_t* seed);
+// The fused step boundary `mode` with one draw of the forcing.
+int step_boundary(gt_ctx* c, int mode, gt::PassArgs a, RectTables* t, int32_t* seed);
 void adj_free(gt_ctx* c);  // gturbo_adjoint.cpp
 // Runs the deferred end of the last step (its last stage and forcing), if
 // any: every entry point that reads or writes device data calls it first.

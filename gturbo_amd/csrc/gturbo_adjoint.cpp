@@ -113,9 +113,14 @@ int to_physical(gt_ctx* c, const double2* in, double* dref) {
   return io_inverse(c, in, c->adj->rc, dref);
 }
 
-// One step of src/rkstep.f90 on the working state; with slot >= 0 every
-// stage input is kept in the stage store.
-int fwd_step(gt_ctx* c, RectTables* t, int slot) {
+// Steps n0 .. n1-1 of src/rkstep.f90 with their forcing (src/main.f90:136) on
+// the working state.  Between two steps the last stage, the forcing and the
+// next step's first pass run as one y pass, as gt_step4 and gt_step fuse
+// them.  keep: every stage input goes to the stage store (slot n - n0) and
+// the run ends with the last stage input, the last step's end and forcing
+// not being needed; else the state is checkpointed every kchk steps and the
+// last step ends.
+int fwd_steps(gt_ctx* c, RectTables* t, int n0, int n1, int32_t* seed, bool keep) {
   AdjState* s = c->adj;
   CHK(ensure_ybuf(c, s->rc));
   gt::PassArgs a{};
@@ -131,38 +136,41 @@ int fwd_step(gt_ctx* c, RectTables* t, int slot) {
   a.znew = s->znew;
   a.emk = t->emk;
   CHK(rect_ka(c, s->rc, &a.ka));
-  auto st = [&](int k) { return slot >= 0 ? stage_ptr(s, slot, k) : nullptr; };
-  if (c->rko == 4) {
+  const bool rk4 = c->rko == 4;
+  const std::vector<int> stages = rk4 ? std::vector<int>{gt::C_RK4_1, gt::C_RK4_2, gt::C_RK4_3}
+                                      : std::vector<int>{gt::C_RK2_1};
+  for (int n = n0; n < n1; ++n) {
+    auto st = [&](int k) { return keep ? stage_ptr(s, n - n0, k) : nullptr; };
     a.sst = st(0);
-    CHK(c_pass(c, gt::C_START, a));
-    CHK(r_pass(c, a));
-    a.sst = st(1);
-    CHK(c_pass(c, gt::C_RK4_1, a));
-    CHK(r_pass(c, a));
-    a.sst = st(2);
-    CHK(c_pass(c, gt::C_RK4_2, a));
-    CHK(r_pass(c, a));
-    a.sst = st(3);
-    CHK(c_pass(c, gt::C_RK4_3, a));
-    CHK(r_pass(c, a));
-    a.sst = nullptr;
-    CHK(c_pass(c, gt::C_RK4_4, a));
-  } else {
-    a.sst = st(0);
-    CHK(c_pass(c, gt::C_START, a));
-    CHK(r_pass(c, a));
-    a.sst = st(1);
-    CHK(c_pass(c, gt::C_RK2_1, a));
-    CHK(r_pass(c, a));
-    a.sst = nullptr;
-    CHK(c_pass(c, gt::C_RK2_2, a));
+    if (n == n0) {
+      CHK(c_pass(c, gt::C_START, a));
+    } else {
+      CHK(step_boundary(c, rk4 ? gt::C_RK4_4S : gt::C_RK2_2S, a, t, seed));
+    }
+    if (!keep && n % s->kchk == 0) {
+      HIPCHK(hipMemcpyAsync(s->ck[n / s->kchk], s->z, sizeof(double2) * s->nc,
+                            hipMemcpyDeviceToDevice, c->stream));
+      s->ckseed[n / s->kchk] = *seed;
+    }
+    for (size_t k = 0; k < stages.size(); ++k) {
+      CHK(r_pass(c, a));
+      a.sst = st((int)k + 1);
+      CHK(c_pass(c, stages[k], a));
+    }
+    if (!keep || n + 1 < n1) CHK(r_pass(c, a));
   }
-  return GT_OK;
+  if (keep) return GT_OK;
+  a.sst = nullptr;
+  CHK(c_pass(c, rk4 ? gt::C_RK4_4 : gt::C_RK2_2, a));
+  return forcing_on(c, t, s->z, seed);
 }
 
-// The adjoint of one step: lam (adjoint of the step's output) -> lam
-// (adjoint of its input), with the step's stage inputs in slot.
-int adj_step(gt_ctx* c, RectTables* t, int slot) {
+// The adjoint of one step: lam (adjoint of the step's output) -> lam (adjoint
+// of its input), with the step's stage inputs in slot.  The end of a step
+// runs with the start of the step before it (first = false: the step after
+// this one, if any, has left its end to this one; last: this one's end is
+// run here).
+int adj_step(gt_ctx* c, RectTables* t, int slot, bool first, bool last) {
   AdjState* s = c->adj;
   gt::AdjArgs j{};
   j.rc = s->rc;
@@ -176,11 +184,13 @@ int adj_step(gt_ctx* c, RectTables* t, int slot) {
   j.lam = s->lam;
   j.lacc = s->lacc;
   j.emk = t->emk;
+  CHK(rect_ka(c, s->rc, &j.ka));
   auto yp = [&](int mode, int stage) -> int {
     j.snext = stage >= 0 ? stage_ptr(s, slot, stage) : nullptr;
-    Timer tm(c, mode == gt::J_START4 || mode == gt::J_START2 ? GT_K_YSTART
-                : mode == gt::J_END                        ? GT_K_YFINAL
-                                                           : GT_K_YSTAGE);
+    Timer tm(c, mode == gt::J_START4 || mode == gt::J_START2   ? GT_K_YSTART
+                : mode == gt::J_END                            ? GT_K_YFINAL
+                : mode == gt::J_BOUND4 || mode == gt::J_BOUND2 ? GT_K_YBOUND
+                                                               : GT_K_YSTAGE);
     HIPCHK(gt::launch_j_pass(c->logn, mode, j, c->stream));
     return GT_OK;
   };
@@ -190,7 +200,7 @@ int adj_step(gt_ctx* c, RectTables* t, int slot) {
     return GT_OK;
   };
   if (c->rko == 4) {
-    CHK(yp(gt::J_START4, 3));
+    CHK(yp(first ? gt::J_START4 : gt::J_BOUND4, 3));
     CHK(xp());
     CHK(yp(gt::J_RK4_3, 2));
     CHK(xp());
@@ -198,15 +208,13 @@ int adj_step(gt_ctx* c, RectTables* t, int slot) {
     CHK(xp());
     CHK(yp(gt::J_RK4_1, 0));
     CHK(xp());
-    CHK(yp(gt::J_END, -1));
   } else {
-    CHK(yp(gt::J_START2, 1));
+    CHK(yp(first ? gt::J_START2 : gt::J_BOUND2, 1));
     CHK(xp());
     CHK(yp(gt::J_RK2_1, 0));
     CHK(xp());
-    CHK(yp(gt::J_END, -1));
   }
-  return GT_OK;
+  return last ? yp(gt::J_END, -1) : GT_OK;
 }
 
 int adj_check(gt_ctx* c) {
@@ -239,15 +247,7 @@ int gt_adj_forward(gt_ctx* c, const double* w0, double* wT, int32_t nsteps, int3
   RectTables* t;
   CHK(rect_tables(c, s->rc, &t));
   CHK(from_physical(c, m0->dref, s->z));
-  for (int n = 0; n < nsteps; ++n) {
-    if (n % kchk == 0) {
-      HIPCHK(hipMemcpyAsync(s->ck[n / kchk], s->z, sizeof(double2) * s->nc,
-                            hipMemcpyDeviceToDevice, c->stream));
-      s->ckseed[n / kchk] = *seed;
-    }
-    CHK(fwd_step(c, t, -1));
-    CHK(forcing_on(c, t, s->z, seed));  // src/main.f90:136
-  }
+  CHK(fwd_steps(c, t, 0, nsteps, seed, false));
   CHK(to_physical(c, s->z, mT->dref));
   set_ref_only(*mT);
   s->ready = true;
@@ -272,11 +272,9 @@ int gt_adj_backward(gt_ctx* c, const double* gT, double* g0) {
     HIPCHK(hipMemcpyAsync(s->z, s->ck[seg], sizeof(double2) * s->nc, hipMemcpyDeviceToDevice,
                           c->stream));
     int32_t seed = s->ckseed[seg];
-    for (int n = n0; n < n1; ++n) {
-      CHK(fwd_step(c, t, n - n0));
-      if (n + 1 < n1) CHK(forcing_on(c, t, s->z, &seed));
-    }
-    for (int n = n1 - 1; n >= n0; --n) CHK(adj_step(c, t, n - n0));
+    CHK(fwd_steps(c, t, n0, n1, &seed, true));
+    for (int n = n1 - 1; n >= n0; --n)
+      CHK(adj_step(c, t, n - n0, n == s->nsteps - 1, n == 0));
   }
   CHK(to_physical(c, s->lam, m0->dref));
   set_ref_only(*m0);

@@ -1245,6 +1245,85 @@ __global__ void __launch_bounds__(io_cols(LOGN) * (1 << LOGN) / kE)
 // the products.
 // ---------------------------------------------------------------------------
 
+// What the reversed stage of an adjoint y pass reads of one mode.
+struct JIn {
+  double E;
+  double2 mu, l;
+};
+template <int MODE>
+__device__ __forceinline__ JIn j_load(const AdjArgs& a, unsigned q, bool mean) {
+  JIn in{};
+  if constexpr (MODE != J_END) in.E = a.emk[q];
+  if constexpr (MODE != J_START4 && MODE != J_START2) in.l = a.lacc[q];
+  if constexpr (MODE != J_END && MODE != J_BOUND4 && MODE != J_BOUND2)
+    in.mu = mean ? make_double2(0.0, 0.0) : a.lam[q];
+  return in;
+}
+// The transposed term of one mode from the forward transforms C = F(q
+// lambda_x), Z = F(q lambda_y) (j_oper) and D = F(u lambda_x + v lambda_y),
+// with fft_dir's 1/N^2.
+__device__ __forceinline__ double2 j_oper(double2 C, double2 Z, double fkx, double fky,
+                                          double kar) {
+  return make_double2((fky * C.y - fkx * Z.y) / kar, (fkx * Z.x - fky * C.x) / kar);
+}
+__device__ __forceinline__ double2 j_term(const Phys& ph, double2 D, double2 v, double fkxs,
+                                          double fky, bool mean) {
+  if (mean || (ph.truncate == 1 && cut_mode(ph, fkxs, fky * fky))) return make_double2(0.0, 0.0);
+  return make_double2((D.x + v.x) * ph.inv_n2, (D.y + v.y) * ph.inv_n2);
+}
+// The reversed stage (JMode) with transposed term t: stores lam / lacc and
+// returns the adjoint input of the next transposed term.
+template <int MODE>
+__device__ __forceinline__ double2 j_update(const AdjArgs& a, unsigned q, bool mean, double2 t,
+                                            const JIn& in) {
+  const Phys& ph = a.ph;
+  const double E = in.E;
+  const double2 mu = in.mu;
+  double2 l = in.l;
+  if constexpr (MODE == J_END || MODE == J_BOUND4 || MODE == J_BOUND2) {
+    double2 m = make_double2(l.x + t.x, l.y + t.y);
+    a.lam[q] = m;
+    if constexpr (MODE == J_END) return m;
+    if (mean) m = make_double2(0.0, 0.0);
+    const double EE = E * E;
+    a.lacc[q] = make_double2(EE * m.x, EE * m.y);
+    if constexpr (MODE == J_BOUND4) return make_double2(ph.dt6 * m.x, ph.dt6 * m.y);
+    else return make_double2(ph.dt * E * m.x, ph.dt * E * m.y);
+  } else if constexpr (MODE == J_START4 || MODE == J_START2) {
+    const double EE = E * E;
+    a.lacc[q] = make_double2(EE * mu.x, EE * mu.y);
+    if constexpr (MODE == J_START4) return make_double2(ph.dt6 * mu.x, ph.dt6 * mu.y);
+    else return make_double2(ph.dt * E * mu.x, ph.dt * E * mu.y);
+  } else {
+    double2 av;
+    if constexpr (MODE == J_RK4_3) {
+      const double EE = E * E;
+      l = make_double2(l.x + EE * t.x, l.y + EE * t.y);
+      av = make_double2(ph.dt3 * E * mu.x + ph.dt * E * t.x, ph.dt3 * E * mu.y + ph.dt * E * t.y);
+    } else if constexpr (MODE == J_RK4_2) {
+      l = make_double2(l.x + E * t.x, l.y + E * t.y);
+      av = make_double2(ph.dt3 * E * mu.x + ph.dt2 * t.x, ph.dt3 * E * mu.y + ph.dt2 * t.y);
+    } else if constexpr (MODE == J_RK4_1) {
+      const double EE = E * E;
+      l = make_double2(l.x + E * t.x, l.y + E * t.y);
+      av = make_double2(ph.dt6 * EE * mu.x + ph.dt2 * E * t.x,
+                        ph.dt6 * EE * mu.y + ph.dt2 * E * t.y);
+    } else {  // J_RK2_1
+      l = make_double2(l.x + E * t.x, l.y + E * t.y);
+      av = make_double2(ph.dt2 * E * t.x, ph.dt2 * E * t.y);
+    }
+    a.lacc[q] = l;
+    return av;
+  }
+}
+// Value of one mode in inverse transform f of an adjoint y pass: i kx a, i ky
+// a of the adjoint input, then q, u, v of the stage state.
+__device__ __forceinline__ double2 j_field(int f, double2 v, double fkx, double fky, double kar) {
+  if (f == 0) return make_double2(-fkx * v.y, fkx * v.x);
+  if (f == 1) return make_double2(-fky * v.y, fky * v.x);
+  return field_of(f - 2, v, fkx, fky, kar);
+}
+
 template <int LOGN, int MODE, int AK, int TR>
 __global__ void __launch_bounds__(bt_of(LOGN) * (1 << LOGN) / kE, AK == 1 ? 4 : 1)
     j_pass(AdjArgs a) {
@@ -1291,9 +1370,7 @@ __global__ void __launch_bounds__(bt_of(LOGN) * (1 << LOGN) / kE, AK == 1 ? 4 : 
       if (live_r<TR>(r) && colok && row_of(p, rc, N) >= 0 && !(c == 0 && p == 0)) {
         const double fky = (double)kyi_of(p, N) * ph.dky;
         const double k2 = fkxs + fky * fky;
-        const double kar = AK == 1 ? k2 : kalpha(ph, k2);
-        v = make_double2((fky * C[r].y - fkx * z[r].y) / kar,
-                         (fkx * z[r].x - fky * C[r].x) / kar);
+        v = j_oper(C[r], z[r], fkx, fky, AK == 1 ? k2 : kalpha(ph, k2));
       }
       C[r] = v;
     }
@@ -1310,38 +1387,9 @@ __global__ void __launch_bounds__(bt_of(LOGN) * (1 << LOGN) / kE, AK == 1 ? 4 : 
       if (live_r<TR>(r) && colok && row >= 0) {
         const double fky = (double)kyi_of(p, N) * ph.dky;
         const bool mean = (c == 0 && p == 0);
-        // the transposed term (fft_dir's 1/N^2 on the forward transforms)
-        double2 t = make_double2((z[r].x + C[r].x) * ph.inv_n2, (z[r].y + C[r].y) * ph.inv_n2);
-        if ((ph.truncate == 1 && cut_mode(ph, fkxs, fky * fky)) || mean)
-          t = make_double2(0.0, 0.0);
         const unsigned q = cbase + (unsigned)row;
-        const double E = a.emk[q];
-        if constexpr (MODE == J_END) {
-          const double2 l = a.lacc[q];
-          a.lam[q] = make_double2(l.x + t.x, l.y + t.y);
-        } else {
-          const double2 mu = mean ? make_double2(0.0, 0.0) : a.lam[q];
-          double2 l = a.lacc[q];
-          if constexpr (MODE == J_RK4_3) {
-            const double EE = E * E;
-            l = make_double2(l.x + EE * t.x, l.y + EE * t.y);
-            av[r] = make_double2(ph.dt3 * E * mu.x + ph.dt * E * t.x,
-                                 ph.dt3 * E * mu.y + ph.dt * E * t.y);
-          } else if constexpr (MODE == J_RK4_2) {
-            l = make_double2(l.x + E * t.x, l.y + E * t.y);
-            av[r] = make_double2(ph.dt3 * E * mu.x + ph.dt2 * t.x,
-                                 ph.dt3 * E * mu.y + ph.dt2 * t.y);
-          } else if constexpr (MODE == J_RK4_1) {
-            const double EE = E * E;
-            l = make_double2(l.x + E * t.x, l.y + E * t.y);
-            av[r] = make_double2(ph.dt6 * EE * mu.x + ph.dt2 * E * t.x,
-                                 ph.dt6 * EE * mu.y + ph.dt2 * E * t.y);
-          } else if constexpr (MODE == J_RK2_1) {
-            l = make_double2(l.x + E * t.x, l.y + E * t.y);
-            av[r] = make_double2(ph.dt2 * E * t.x, ph.dt2 * E * t.y);
-          }
-          a.lacc[q] = l;
-        }
+        const double2 t = j_term(ph, z[r], C[r], fkxs, fky, mean);
+        av[r] = j_update<MODE>(a, q, mean, t, j_load<MODE>(a, q, mean));
       }
     }
   } else {
@@ -1352,12 +1400,8 @@ __global__ void __launch_bounds__(bt_of(LOGN) * (1 << LOGN) / kE, AK == 1 ? 4 : 
       av[r] = make_double2(0.0, 0.0);
       if (live_r<TR>(r) && colok && row >= 0) {
         const unsigned q = cbase + (unsigned)row;
-        const double2 mu = (c == 0 && p == 0) ? make_double2(0.0, 0.0) : a.lam[q];
-        const double E = a.emk[q];
-        const double EE = E * E;
-        a.lacc[q] = make_double2(EE * mu.x, EE * mu.y);
-        if constexpr (MODE == J_START4) av[r] = make_double2(ph.dt6 * mu.x, ph.dt6 * mu.y);
-        else av[r] = make_double2(ph.dt * E * mu.x, ph.dt * E * mu.y);
+        const bool mean = c == 0 && p == 0;
+        av[r] = j_update<MODE>(a, q, mean, av[r], j_load<MODE>(a, q, mean));
       }
     }
   }
@@ -1374,26 +1418,10 @@ __global__ void __launch_bounds__(bt_of(LOGN) * (1 << LOGN) / kE, AK == 1 ? 4 : 
         double2 v = make_double2(0.0, 0.0);
         if (live_r<TR>(r) && colok && row >= 0) {
           const double fky = (double)kyi_of(p, N) * ph.dky;
-          if (f == 0) {
-            v = make_double2(-fkx * av[r].y, fkx * av[r].x);  // i kx a
-          } else if (f == 1) {
-            v = make_double2(-fky * av[r].y, fky * av[r].x);  // i ky a
-          } else {
-            const double2 sv = a.snext[cbase + (unsigned)row];
-            if (f == 2) {
-              v = sv;
-            } else if (!(c == 0 && p == 0)) {  // u, v as src/nlt.f90:25-34
-              const double k2 = fkxs + fky * fky;
-              const double kar = AK == 1 ? k2 : kalpha(ph, k2);
-              if (f == 3) {
-                const double kyn = fky / kar;
-                v = make_double2(-kyn * sv.y, kyn * sv.x);
-              } else {
-                const double kxn = fkx / kar;
-                v = make_double2(kxn * sv.y, -kxn * sv.x);
-              }
-            }
-          }
+          const double k2 = fkxs + fky * fky;
+          if (f < 3 || !(c == 0 && p == 0))  // u, v: src/nlt.f90:25-34
+            v = j_field(f, f < 2 ? av[r] : a.snext[cbase + (unsigned)row], fkx, fky,
+                        AK == 1 || f < 3 ? k2 : kalpha(ph, k2));
         }
         z[r] = v;
       }
@@ -1469,6 +1497,194 @@ __global__ void __launch_bounds__(rows_of(LOGN) * (1 << LOGN) / kE)
   for (int r = 0; r <= kE / 2; ++r) {
     const int k = j + TPL * r;
     if (live_r<TR>(r) && k <= kxm && k <= N / 2) a.y2[off + koff<LOGN, BT>(k)] = z[r];
+  }
+}
+
+// Small grids (see f_pass): the adjoint passes with a column's three forward
+// and five inverse transforms, and a row's three inverse and two forward
+// ones, on their own threads: two transforms deep instead of eight and five.
+// 512^2, alpha 1: y stage 25.2 -> 10.0 us, x pass 12.0 -> 9.0, and a step's
+// end and the next one's start (10.0 + 18.1 us) in one pass, 10.1; results
+// bit-identical.  At 1024^2 a column fills 104 KB of LDS and the passes in
+// turn stay ahead: a gradient step 541 us, 582 with these.
+template <int LOGN, int MODE, int AK>
+__global__ void __launch_bounds__(fp_cols(LOGN) * 5 * (1 << LOGN) / kE) fj_pass(AdjArgs a) {
+  constexpr int N = 1 << LOGN, TPL = N / kE, BT = bt_of(LOGN), CW = fp_cols(LOGN);
+  constexpr int LINE = Line<LOGN>::PADDED, GT = CW * TPL;
+  constexpr bool FWD = MODE != J_START4 && MODE != J_START2;
+  constexpr bool INV = MODE != J_END;
+  constexpr int NLINE = INV ? 6 : 3;  // a line per field, the adjoint input
+  static_assert(GT % 64 == 0 && line_in_wave<LOGN>(), "whole waves per field");
+  __shared__ double2 lds[CW * NLINE * LINE];
+  const int f = __builtin_amdgcn_readfirstlane(threadIdx.x / GT);
+  const int t = threadIdx.x % GT, cw = t / TPL, j = t % TPL;
+  const int c = CW == 1 ? xcd_remap(blockIdx.x, gridDim.x) : (int)blockIdx.x * CW + cw;
+  const Rect rc = a.rc;
+  const bool colok = c <= rc.kx;
+  const Phys& ph = a.ph;
+  const double fkx = (double)c * ph.dkx;
+  const double fkxs = fkx * fkx;
+  const unsigned cbase = (unsigned)c * (unsigned)a.kyp;
+  const unsigned colo = ycol_off(c, BT);
+  const size_t fs = (size_t)a.ntiles * N * BT;
+  double2* col = lds + cw * NLINE * LINE;
+  double2* buf = col + (NLINE == 6 || f < 3 ? f : 0) * LINE;
+  double2* abuf = col + 5 * LINE;
+
+  double2 z[kE], sv[kE];
+  double ka[kE];
+  if constexpr (FWD) {
+    if (f < 3) {  // F(q lambda_x), F(q lambda_y), F(u lambda_x + v lambda_y)
+      const double2* src = a.y2 + (f == 2 ? 0 : (f + 1) * fs);
+#pragma unroll
+      for (int r = 0; r < kE; ++r)
+        z[r] = colok ? src[yrow_off(j + TPL * r, a.ntiles, BT) + colo] : make_double2(0.0, 0.0);
+    }
+  }
+  const HeldTw<LOGN> tw = held_tw<LOGN>(a.tw, j);
+  int pos[2];
+  bool own[2];
+  unsigned qi[2];
+  JIn in[2];
+  double kao[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {  // modes this thread updates (fields 0-2)
+    const int x = 2 * f + i, r = x >= 3 ? x + 2 : x;
+    pos[i] = j + TPL * r;
+    const int row = f < 3 ? row_of(pos[i], rc, N) : -1;
+    own[i] = colok && row >= 0;
+    qi[i] = cbase + (unsigned)row;
+    in[i] = own[i] ? j_load<MODE>(a, qi[i], c == 0 && pos[i] == 0) : JIn{};
+    kao[i] = AK == 2 && FWD && own[i] ? a.ka[qi[i]] : 1.0;
+  }
+  if constexpr (INV) {
+#pragma unroll
+    for (int r = 0; r < kE; ++r) {  // the stage state of the next transposed term
+      const int row = row_of(j + TPL * r, rc, N);
+      const bool ok = f >= 2 && live_r<1>(r) && colok && row >= 0;
+      sv[r] = ok ? a.snext[cbase + (unsigned)row] : make_double2(0.0, 0.0);
+      ka[r] = AK == 2 && ok && f > 2 ? a.ka[cbase + (unsigned)row] : 1.0;
+    }
+  }
+  if constexpr (FWD) {
+    if (f < 3) {
+      fft_held<LOGN, -1>(z, buf, j, tw);
+#pragma unroll
+      for (int r = 0; r < kE; ++r)
+        if (live_r<1>(r)) (buf + lpad(j))[lpad_off(TPL * r)] = z[r];
+    }
+    __syncthreads();
+  }
+  if (f < 3) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      double2 v = make_double2(0.0, 0.0);
+      if (own[i]) {
+        const int p = pos[i], e = lpad(p);
+        const bool mean = c == 0 && p == 0;
+        double2 tm = v;
+        if constexpr (FWD) {
+          const double fky = (double)kyi_of(p, N) * ph.dky;
+          if (!mean)
+            tm = j_oper(col[e], col[LINE + e], fkx, fky, AK == 1 ? fkxs + fky * fky : kao[i]);
+          tm = j_term(ph, col[2 * LINE + e], tm, fkxs, fky, mean);
+        }
+        v = j_update<MODE>(a, qi[i], mean, tm, in[i]);
+      }
+      if constexpr (INV) abuf[lpad(pos[i])] = v;
+    }
+  }
+  if constexpr (INV) {
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kE; ++r) {
+      z[r] = make_double2(0.0, 0.0);
+      if (!live_r<1>(r)) continue;
+      const int p = j + TPL * r;
+      const double fky = (double)kyi_of(p, N) * ph.dky;
+      const double2 av = (abuf + lpad(j))[lpad_off(TPL * r)];
+      const double2 v = make_double2(f < 2 ? av.x : sv[r].x, f < 2 ? av.y : sv[r].y);
+      if (f < 3 || !(c == 0 && p == 0))
+        z[r] = j_field(f, v, fkx, fky, AK == 1 || f < 3 ? fkxs + fky * fky : ka[r]);
+    }
+    fft_held<LOGN, +1>(z, buf, j, tw);
+    if (colok) {
+      double2* dst = a.y1 + f * fs;
+#pragma unroll
+      for (int r = 0; r < kE; ++r) dst[yrow_off(j + TPL * r, a.ntiles, BT) + colo] = z[r];
+    }
+  }
+}
+
+template <int LOGN>
+__global__ void __launch_bounds__(3 * fx_rows(LOGN) * (1 << LOGN) / kE) fjr_pass(AdjArgs a) {
+  constexpr int N = 1 << LOGN, TPL = N / kE, BT = bt_of(LOGN), RW = fx_rows(LOGN);
+  constexpr int LINE = Line<LOGN>::PADDED, GT = RW * TPL;
+  static_assert(line_in_wave<LOGN>(), "a line inside a wave");
+  __shared__ double2 lds[4 * RW * LINE];
+  int f = threadIdx.x / GT;  // 0: lambda_x + i lambda_y, 1: q + iu, 2: v
+  if constexpr (GT % 64 == 0) f = __builtin_amdgcn_readfirstlane(f);
+  const int t = threadIdx.x % GT, rw = t / TPL, j = t % TPL;
+  const int yrow = xcd_remap(blockIdx.x, gridDim.x) * RW + rw;
+  double2* row = lds + 4 * rw * LINE;
+  double2* buf = row + f * LINE;
+  double* ub = reinterpret_cast<double*>(row + 3 * LINE);
+  const int kxm = a.rc.kx;
+  const unsigned fs = (unsigned)a.ntiles * N * BT;
+  const unsigned off = yrow_off(yrow, a.ntiles, BT);
+  double2 z[kE];
+  {
+    double2 x0[kE], x1[kE];
+    const unsigned of = off + 2 * f * fs;
+    load_two<LOGN, 1, BT>(x0, x1, j, a.y1, of, f == 2 ? of : of + fs, kxm);
+    if (f == 2) {
+#pragma unroll
+      for (int r = 0; r < kE; ++r) x1[r] = make_double2(0.0, 0.0);
+    }
+    pack_two<LOGN>(z, j, x0, x1);
+  }
+  const HeldTw<LOGN> tw = held_tw<LOGN>(a.tw, j);
+  fft_held<LOGN, +1>(z, buf, j, tw);
+  if (f == 0) {
+#pragma unroll
+    for (int r = 0; r < kE; ++r) (buf + lpad(j))[lpad_off(TPL * r)] = z[r];
+  } else if (f == 1) {
+#pragma unroll
+    for (int r = 0; r < kE; ++r) ub[j + TPL * r] = z[r].y;
+  }
+  __syncthreads();
+  if (f > 0) {
+#pragma unroll
+    for (int r = 0; r < kE; ++r) {
+      const double2 l = (row + lpad(j))[lpad_off(TPL * r)];
+      z[r] = f == 1 ? make_double2(z[r].x * l.x, z[r].x * l.y)  // q lambda_x + i q lambda_y
+                    : make_double2(ub[j + TPL * r] * l.x + z[r].x * l.y, 0.0);
+    }
+    fft_held<LOGN, -1>(z, buf, j, tw);
+  }
+  if (f == 1) {
+#pragma unroll
+    for (int r = 0; r < kE; ++r)
+      if (live_r<1>(r)) (buf + lpad(j))[lpad_off(TPL * r)] = z[r];
+  }
+  __syncthreads();
+  double2* wl = row + LINE;
+  const double2* pm = wl + lpad(TPL - j);
+  double2* out = a.y2 + off + (f == 2 ? 0u : (f + 1) * fs);
+#pragma unroll
+  for (int r = 0; r <= kE / 2; ++r) {
+    const int k = j + TPL * r;
+    if (live_r<1>(r) && k <= kxm && k <= N / 2) {
+      if (f == 2) {  // F(u lambda_x + v lambda_y)
+        out[koff<LOGN, BT>(k)] = z[r];
+      } else {
+        const double2 W = (wl + lpad(j))[lpad_off(TPL * r)];
+        const double2 Wc = mirror_at<LOGN>(wl, pm, j, r);
+        out[koff<LOGN, BT>(k)] = f == 0
+                                     ? make_double2(0.5 * (W.x + Wc.x), 0.5 * (W.y - Wc.y))
+                                     : make_double2(0.5 * (W.y + Wc.y), -0.5 * (W.x - Wc.x));
+      }
+    }
   }
 }
 
@@ -1578,18 +1794,28 @@ hipError_t io_launch(const IoArgs& a, hipStream_t s) {
   return hipGetLastError();
 }
 
+template <int L, int MODE, int AK>
+static void j_launch(const AdjArgs& a, hipStream_t s) {
+  if constexpr (L <= kFjMaxLogn) {
+    constexpr int CW = fp_cols(L);
+    const int g = (a.rc.kc() + CW - 1) / CW;
+    fj_pass<L, MODE, AK><<<dim3(g), dim3(CW * 5 * (1 << L) / kE), 0, s>>>(a);
+  } else {
+    j_pass<L, MODE, AK, 1><<<dim3(a.ntiles), dim3(bt_of(L) * (1 << L) / kE), 0, s>>>(a);
+  }
+}
 template <int L, int AK>
 static hipError_t j_pass_launch_ak(int mode, const AdjArgs& a, hipStream_t s) {
-  constexpr int T = bt_of(L) * (1 << L) / kE;
-  const dim3 g(a.ntiles), b(T);
   switch (mode) {
-    case J_START4: j_pass<L, J_START4, AK, 1><<<g, b, 0, s>>>(a); break;
-    case J_RK4_3: j_pass<L, J_RK4_3, AK, 1><<<g, b, 0, s>>>(a); break;
-    case J_RK4_2: j_pass<L, J_RK4_2, AK, 1><<<g, b, 0, s>>>(a); break;
-    case J_RK4_1: j_pass<L, J_RK4_1, AK, 1><<<g, b, 0, s>>>(a); break;
-    case J_END: j_pass<L, J_END, AK, 1><<<g, b, 0, s>>>(a); break;
-    case J_START2: j_pass<L, J_START2, AK, 1><<<g, b, 0, s>>>(a); break;
-    case J_RK2_1: j_pass<L, J_RK2_1, AK, 1><<<g, b, 0, s>>>(a); break;
+    case J_START4: j_launch<L, J_START4, AK>(a, s); break;
+    case J_RK4_3: j_launch<L, J_RK4_3, AK>(a, s); break;
+    case J_RK4_2: j_launch<L, J_RK4_2, AK>(a, s); break;
+    case J_RK4_1: j_launch<L, J_RK4_1, AK>(a, s); break;
+    case J_END: j_launch<L, J_END, AK>(a, s); break;
+    case J_START2: j_launch<L, J_START2, AK>(a, s); break;
+    case J_RK2_1: j_launch<L, J_RK2_1, AK>(a, s); break;
+    case J_BOUND4: j_launch<L, J_BOUND4, AK>(a, s); break;
+    case J_BOUND2: j_launch<L, J_BOUND2, AK>(a, s); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -1598,16 +1824,22 @@ static hipError_t j_pass_launch_ak(int mode, const AdjArgs& a, hipStream_t s) {
 // The adjoint needs the 2/3 rectangle (TR = 1).
 template <int L>
 hipError_t j_pass_launch(int mode, const AdjArgs& a, hipStream_t s) {
+  constexpr int AK = L <= kFjMaxLogn ? 2 : 0;
   if (!rect_tr(a.rc, 1 << L)) return hipErrorInvalidValue;
   return a.ph.akind == 1 ? j_pass_launch_ak<L, 1>(mode, a, s)
-                         : j_pass_launch_ak<L, 0>(mode, a, s);
+                         : j_pass_launch_ak<L, AK>(mode, a, s);
 }
 
 template <int L>
 hipError_t jr_pass_launch(const AdjArgs& a, hipStream_t s) {
   if (!rect_tr(a.rc, 1 << L)) return hipErrorInvalidValue;
-  constexpr int RP = rows_of(L), T = RP * (1 << L) / kE;
-  jr_pass<L, 1><<<dim3((1 << L) / RP), dim3(T), 0, s>>>(a);
+  if constexpr (L <= kFjMaxLogn) {
+    constexpr int RW = fx_rows(L);
+    fjr_pass<L><<<dim3((1 << L) / RW), dim3(3 * RW * (1 << L) / kE), 0, s>>>(a);
+  } else {
+    constexpr int RP = rows_of(L), T = RP * (1 << L) / kE;
+    jr_pass<L, 1><<<dim3((1 << L) / RP), dim3(T), 0, s>>>(a);
+  }
   return hipGetLastError();
 }
 

@@ -557,6 +557,22 @@ int flush_pending(gt_ctx* c) {
   return GT_OK;
 }
 
+// A fused step boundary with the forcing draws of a slot.
+static int boundary_pass(gt_ctx* c, int mode, gt::PassArgs a, RectTables* t, unsigned slot) {
+  a.fcs = t->fcs;
+  a.fce = t->fce;
+  a.fph = c->ph_dev + (size_t)slot * c->nf;
+  a.famp = c->sdt * c->famp;
+  CHK(c_pass(c, mode, a));
+  return slot_read(c, slot);
+}
+int step_boundary(gt_ctx* c, int mode, gt::PassArgs a, RectTables* t, int32_t* seed) {
+  if (c->nf == 0) return c_pass(c, mode, a);
+  unsigned slot;
+  CHK(forcing_upload(c, seed, &slot));
+  return boundary_pass(c, mode, a, t, slot);
+}
+
 // Whether the deferred end can be fused into a step of the same kind on
 // the same arrays (state z, and for RK4 the accumulator of the deferred
 // step, which its last stage reads).
@@ -574,15 +590,8 @@ static int step_start(gt_ctx* c, int kind, Mirror* m, Mirror* mn, const gt::Pass
   if (pending_fuses(c, kind, m, mn)) {
     const Pending q = c->pend;
     c->pend = Pending{};
-    gt::PassArgs b = q.a;
-    if (q.forced) {
-      b.fcs = q.t->fcs;
-      b.fce = q.t->fce;
-      b.fph = c->ph_dev + (size_t)q.slot * c->nf;
-      b.famp = c->sdt * c->famp;
-    }
-    CHK(c_pass(c, kind == PEND_RK4 ? gt::C_RK4_4S : gt::C_RK2_2S, b));
-    if (q.forced) CHK(slot_read(c, q.slot));
+    const int mode = kind == PEND_RK4 ? gt::C_RK4_4S : gt::C_RK2_2S;
+    CHK(q.forced ? boundary_pass(c, mode, q.a, q.t, q.slot) : c_pass(c, mode, q.a));
     return GT_OK;
   }
   CHK(flush_pending(c));

@@ -4,9 +4,12 @@ rectangles, and columns with more forced modes than a workgroup stages."""
 import numpy as np
 import pytest
 
+from gturbo_amd import ic
+from gturbo_amd.adjoint import Adjoint
+from gturbo_amd.params import InitialSpectrum
 from gturbo_amd.solver import Solver
-
 from helpers import params_for, random_spectral
+from test_gpu_adjoint import _tlm
 
 pytestmark = pytest.mark.gpu
 
@@ -100,3 +103,22 @@ def test_consumers_of_fft_dir(oracle_mod, n):
         o.fft_inv(x)
         same(xg, x)
     s.close()
+
+
+@pytest.mark.parametrize("n,alpv,rko,nsteps,kchk", [
+    (16, 2.0, 4, 5, 2), (32, 1.5, 2, 6, 4), (512, 1.5, 4, 3, 2), (1024, 2.0, 4, 3, 3)])
+def test_adjoint_dot_product(oracle_mod, n, alpv, rko, nsteps, kchk):
+    """Adjoint passes at the ends of their sizes, with a partial last segment
+    (5 = 2 + 2 + 1): <gT, M' dw0> = <M'^T gT, dw0> as in test_gpu_adjoint."""
+    p = params_for(n, alpv=alpv, rko=rko, famp=1.0)
+    rng = np.random.default_rng(n + nsteps)
+    w0 = ic.physical_field(p, InitialSpectrum(seed=11, p=4.0, k0=max(n / 16.0, 2.0), energy=0.5))
+    dw0, gT = rng.standard_normal((n, n)), rng.standard_normal((n, n))
+    o = oracle_mod.Oracle(p)
+    wT_o, dwT = _tlm(o, w0.astype(np.float64), dw0, nsteps, 481929)
+    with Adjoint(p, nsteps, kchk) as adj:
+        wT, _ = adj.forward(w0.astype(np.float64), 481929)
+        g0 = adj.backward(gT)
+    assert _rel(wT, wT_o) < 1e-11
+    lhs, rhs = float(np.sum(gT * dwT)), float(np.sum(g0 * dw0))
+    assert abs(lhs - rhs) <= 1e-10 * abs(lhs)
