@@ -190,9 +190,10 @@ struct DiagArgs {
   const double2* znl;
   double* part1;  // (kx+1) x NBIN partial sums
   double* part2;
+  int2* lohi;     // kx+1: first and last shell of each column
   double* out1;   // NBIN
   double* out2;
-  double* gpart;  // (kx+1) x 6
+  double* gpart;  // 6 x (kx+1)
   double* gout;   // 6
 };
 

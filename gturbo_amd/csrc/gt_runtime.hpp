@@ -128,6 +128,8 @@ struct gt_ctx {
   // diagnostics
   double* dg = nullptr;
   size_t dg_cap = 0;
+  double* dg_out = nullptr;  // results, pinned: 2 NBIN sums, 6 of glob
+  double* dg_dev = nullptr;  // their device address
   // device address of the static partial sums of gt_glob_noalloc on this
   // context's device, and their count in doubles
   double* glob_scratch = nullptr;

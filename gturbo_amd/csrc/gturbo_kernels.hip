@@ -2170,21 +2170,24 @@ __global__ void ens_forcing_k(const EnsForce* __restrict__ f, int nmem, int tota
 __global__ void ens_tick_k(int* step) { step[0] = step[0] + 1; }
 
 // ---------------------------------------------------------------------------
-// Diagnostics (src/diagnostics.f90), deterministic, in two launches each.
+// Diagnostics (src/diagnostics.f90), deterministic: the order of every sum is
+// fixed, so the results do not change from run to run (the reference's
+// accumulations on the GPU are unprotected, diagnostics.f90:25-39,84-101).
 //
 // Spectrum and fluxes: one workgroup (4 waves) per kx column bins the
 // column's modes into LDS bins, one per shell.  In each half of a column
-// (ky >= 0: rows 0..p; ky < 0: rows p+1..) the shell index is monotone in
-// the row, so a chunk of 64 consecutive rows of one wave holds runs of equal
-// shells: a segmented wavefront scan (lane shuffles, a fixed tree) sums each
-// run, the run's last lane carries the sum, and runs continued across the
-// four waves of a 256-row chunk are joined in wave order by the run's first
-// lane, which alone adds it to the shell's LDS bin.  The column's bins then
-// go to part[c][b].  A second launch sums part[.][b] over the columns, one
-// wavefront per shell: lanes take columns c = lane, lane + 64, ... in
-// order, then a fixed shuffle tree.  The order of every sum is fixed, so
-// the result does not change from run to run; it replaces the reference's
-// unprotected accumulations on the GPU (diagnostics.f90:25-39,84-101).
+// (ky >= 0: rows 0..p; ky < 0: rows p+1..) the shell index is monotone in the
+// row.  Each wave takes a quarter of the half in chunks of 64 rows, whose
+// runs of equal shells a segmented wavefront scan sums (a fixed tree); a run
+// that a chunk leaves open is carried in registers to the next.  A shell then
+// belongs to one wave, except where a wave's first run continues the one
+// before: first runs go to a slot per wave, added in wave order after the
+// half.  One barrier per half instead of two per chunk, and the next chunk's
+// loads are issued before this one is summed.  The column's bins go to
+// part[c][b]; a second launch sums part[.][b] over the columns.  4096^2
+// spectrum: bins 42 us (54 with a barrier pair per chunk and hypot; 60 MB,
+// bound by the instructions of the root, the division and the scan), columns
+// 10 us (27 with one shell's column of part per wavefront).
 // ---------------------------------------------------------------------------
 
 __host__ __device__ __forceinline__ int shell_of(const Phys& ph, double fkxs, int p) {
@@ -2210,44 +2213,46 @@ __host__ __device__ __forceinline__ void column_shells(const Phys& ph, const Rec
 
 constexpr int kDiagT = 256;  // threads of a diagnostics workgroup (4 waves)
 
-// Inclusive sums of v1, v2 over each run of equal keys in the wave (runs
-// are contiguous); returns true on a run's last lane.
-__device__ __forceinline__ bool wave_runs(int key, double& v1, double& v2) {
-  const int lane = (int)(threadIdx.x & 63);
-  const int kprev = __shfl_up(key, 1);
-  const bool head = lane == 0 || kprev != key;
-  const unsigned long long heads = __ballot(head);
-  // run number: heads at or below this lane
-  const int run = __popcll(heads & (~0ull >> (63 - lane)));
+// Inclusive sums of v1, v2 over each run of equal keys in the wave (runs are
+// contiguous, heads the ballot of their first lanes).
+__device__ __forceinline__ void wave_runs(unsigned long long heads, int lane, double& v1,
+                                          double& v2) {
+  // lanes of the run at or below this one
+  const int back = lane - (63 - __clzll((long long)(heads & (~0ull >> (63 - lane)))));
 #pragma unroll
   for (int d = 1; d < 64; d <<= 1) {
     const double t1 = __shfl_up(v1, d), t2 = __shfl_up(v2, d);
-    const int rr = __shfl_up(run, d);
-    if (lane >= d && rr == run) {
+    if (d <= back) {
       v1 = v1 + t1;
       v2 = v2 + t2;
     }
   }
-  const bool next_head = lane == 63 ? true : ((heads >> (lane + 1)) & 1ull) != 0;
-  return next_head;
 }
 
-// which = 0: spectrum (sp, sz);  which = 1: fluxes (flzm, flem)
+__device__ __forceinline__ double lane_value(double v, int lane) {
+  const int lo = __builtin_amdgcn_readlane(__double2loint(v), lane);
+  const int hi = __builtin_amdgcn_readlane(__double2hiint(v), lane);
+  return __hiloint2double(hi, lo);
+}
+
+// WHICH = 0: spectrum (sp, sz);  WHICH = 1: fluxes (flzm, flem)
 // nbl: the most shells of any column (LDS bins per sum).
-__global__ void __launch_bounds__(kDiagT) shell_bin_k(DiagArgs d, int which, int nbl) {
+template <int WHICH>
+__global__ void __launch_bounds__(kDiagT) shell_bin_k(DiagArgs d, int nbl) {
   extern __shared__ double dsm[];
+  constexpr int NW = kDiagT / 64;
   const Phys& ph = d.ph;
   const Rect rc = d.rc;
   const int n = ph.n, nbin = n / 2, c = blockIdx.x, tid = threadIdx.x;
-  const int wave = tid >> 6, lane = tid & 63;
-  double* bin1 = dsm;                  // shell b of the column in bin b - lo
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  double* bin1 = dsm;         // shell b of the column in bin b - lo
   double* bin2 = bin1 + nbl;
-  double* sv1 = bin2 + nbl;            // per-lane run sums of a chunk
-  double* sv2 = sv1 + kDiagT;
-  int* skey = reinterpret_cast<int*>(sv2 + kDiagT);  // key on a run's last lane, else -1
-  int* ftail = skey + kDiagT;                        // each wave's first run end
+  __shared__ double edge1[NW], edge2[NW];  // each wave's first run
+  __shared__ int ekey[NW];
   const double fkx = (double)c * ph.dkx, fkxs = fkx * fkx;
-  const bool edge = (c == 0 || c == n / 2);
+  const double fac = (c == 0 || c == n / 2) ? (WHICH ? 1.0 : 0.5)   // diagnostics.f90:29-30
+                                            : (WHICH ? 2.0 : 1.0);  // :89-90
   const size_t cq = (size_t)c * d.kyp;
   int blo, bhi;
   column_shells(ph, rc, c, blo, bhi);
@@ -2256,12 +2261,34 @@ __global__ void __launch_bounds__(kDiagT) shell_bin_k(DiagArgs d, int which, int
     bin1[b - blo] = 0.0;
     bin2[b - blo] = 0.0;
   }
-  __syncthreads();
   const int P = rc.p, Ky = rc.ky();
   for (int half = 0; half < 2; ++half) {
-    const int r0 = half ? P + 1 : 0, r1 = half ? Ky : P + 1;  // rows [r0, r1)
-    for (int base = r0; base < r1; base += kDiagT) {
-      const int r = base + tid;
+    const int h0 = half ? P + 1 : 0, h1 = half ? Ky : P + 1;  // rows [h0, h1)
+    const int per = ((h1 - h0 + NW - 1) / NW + 63) & ~63;
+    const int r0 = h0 + wave * per, r1 = r0 + per < h1 ? r0 + per : h1;
+    __syncthreads();  // bins cleared; the half before added up
+    if (lane == 0) ekey[wave] = -1;
+    const double2 zero = make_double2(0.0, 0.0);
+    double2 zn = r0 + lane < r1 ? d.z[cq + r0 + lane] : zero;
+    double2 nn = WHICH && r0 + lane < r1 ? d.znl[cq + r0 + lane] : zero;
+    int first = -2, ck = -1;       // the wave's first key; the carried run
+    double c1 = 0.0, c2 = 0.0;
+    // adds a finished run: the wave's first one to its slot
+    auto put = [&](int key, double v1, double v2) {
+      if (key == first) {
+        ekey[wave] = key;
+        edge1[wave] = v1;
+        edge2[wave] = v2;
+      } else {
+        bin1[key - blo] = bin1[key - blo] + v1;
+        bin2[key - blo] = bin2[key - blo] + v2;
+      }
+    };
+    for (int base = r0; base < r1; base += 64) {
+      const int r = base + lane, rn = r + 64;
+      const double2 zv = zn, nv = nn;
+      zn = rn < r1 ? d.z[cq + rn] : zero;
+      if (WHICH) nn = rn < r1 ? d.znl[cq + rn] : zero;
       int key = -1;
       double v1 = 0.0, v2 = 0.0;
       if (r < r1 && !(c == 0 && r == 0)) {  // diagnostics.f90:28
@@ -2269,59 +2296,59 @@ __global__ void __launch_bounds__(kDiagT) shell_bin_k(DiagArgs d, int which, int
         const double fky = (double)kyi_of(p, n) * ph.dky;
         const double k2 = fkxs + fky * fky;
         const double k = sqrt(k2);
-        const int ib = (int)(k / ph.dkx) + 1;  // diagnostics.f90:34
+        const int ib = (int)(ph.dkx == 1.0 ? k : k / ph.dkx) + 1;  // diagnostics.f90:34
         if (ib < nbin && ib >= blo && ib <= bhi) {
           key = ib;
           const double ka = kalpha(ph, k2);
-          const double2 zv = d.z[cq + r];
-          if (which == 0) {
-            const double fac = edge ? 0.5 : 1.0;  // diagnostics.f90:29-30
-            const double am = hypot(zv.x, zv.y);
-            const double a2 = am * am;
+          if (WHICH == 0) {
+            const double a2 = zv.x * zv.x + zv.y * zv.y;
             v1 = fac * a2 / ka;  // sp, diagnostics.f90:36
             v2 = fac * a2;       // sz, :37
           } else {
-            const double fac = edge ? 1.0 : 2.0;  // diagnostics.f90:89-90
-            const double2 nv = d.znl[cq + r];
             const double fz = zv.x * nv.x + zv.y * nv.y;  // :93
             v1 = fac * fz;          // flzm, :98
             v2 = fac * (fz / ka);   // flem, :95,99
           }
         }
       }
-      const bool last = wave_runs(key, v1, v2);
-      const unsigned long long lasts = __ballot(last);
-      skey[tid] = last ? key : -1;
-      sv1[tid] = v1;
-      sv2[tid] = v2;
-      if (lane == 0) ftail[wave] = (wave << 6) + __builtin_ctzll(lasts);
-      __syncthreads();
-      if (last && key >= 0) {
-        // A wave's first run continues the previous wave's last run when the
-        // keys agree: that run belongs to the lane that ends its first piece.
-        const bool cont = wave > 0 && tid == ftail[wave] && skey[(wave << 6) - 1] == key;
-        if (!cont) {
-          double a1 = v1, a2 = v2;
-          if (lane == 63) {
-            for (int w2 = wave + 1; w2 < kDiagT / 64; ++w2) {
-              const int t = ftail[w2];
-              if (skey[t] != key) break;
-              a1 = a1 + sv1[t];
-              a2 = a2 + sv2[t];
-              if ((t & 63) != 63) break;
-            }
-          }
-          bin1[key - blo] = bin1[key - blo] + a1;
-          bin2[key - blo] = bin2[key - blo] + a2;
+      const int kprev = __shfl_up(key, 1);
+      const bool head = lane == 0 || kprev != key;
+      const unsigned long long heads = __ballot(head);
+      wave_runs(heads, lane, v1, v2);
+      const int k0 = __builtin_amdgcn_readfirstlane(key);
+      if (base == r0) first = k0;
+      if (ck == k0 && ck >= 0) {  // the carried run goes on in this chunk's first
+        if ((heads & (~0ull >> (63 - lane))) == 1ull) {
+          v1 = c1 + v1;
+          v2 = c2 + v2;
+        }
+      } else if (ck >= 0 && lane == 0) {
+        put(ck, c1, c2);
+      }
+      // runs that end inside the chunk (one lane each)
+      if (lane < 63 && ((heads >> (lane + 1)) & 1ull) != 0 && key >= 0) put(key, v1, v2);
+      ck = __builtin_amdgcn_readlane(key, 63);
+      c1 = lane_value(v1, 63);
+      c2 = lane_value(v2, 63);
+    }
+    if (ck >= 0 && lane == 0) put(ck, c1, c2);
+    __syncthreads();
+    if (tid == 0) {
+      for (int w = 0; w < NW; ++w) {
+        const int key = ekey[w];
+        if (key >= 0) {
+          bin1[key - blo] = bin1[key - blo] + edge1[w];
+          bin2[key - blo] = bin2[key - blo] + edge2[w];
         }
       }
-      __syncthreads();
     }
   }
+  __syncthreads();
   for (int b = blo + tid; b <= bhi; b += kDiagT) {
     d.part1[(size_t)c * nbin + (b - 1)] = bin1[b - blo];
     d.part2[(size_t)c * nbin + (b - 1)] = bin2[b - blo];
   }
+  if (tid == 0) d.lohi[c] = make_int2(blo, bhi);
 }
 
 // Sum of a wavefront's values in a fixed tree order; lane 0 holds the total.
@@ -2331,76 +2358,109 @@ __device__ __forceinline__ double wave_sum(double v) {
   return v;
 }
 
-// One wavefront per shell: the columns' bins of shell b, over the columns in
-// a fixed order.
-__global__ void __launch_bounds__(kDiagT) shell_sum_k(DiagArgs d, int which) {
+// The columns' bins summed over the columns: a workgroup takes 16 shells,
+// its 64 rows of 16 threads the columns c = g, g + 64, ... in order (128
+// contiguous bytes of part each), then a fixed tree over the rows.
+constexpr int kSumT = 1024, kSumB = 16, kSumG = kSumT / kSumB;
+__global__ void __launch_bounds__(kSumT) shell_sum_k(DiagArgs d, int which) {
+  __shared__ double s1[kSumG][kSumB + 1], s2[kSumG][kSumB + 1];
+  __shared__ int2 lh[8192 / 2 + 1];
   const Phys& ph = d.ph;
-  const Rect rc = d.rc;
-  const int n = ph.n, nbin = n / 2;
-  const int b = (int)((blockIdx.x * kDiagT + threadIdx.x) >> 6) + 1;  // shell 1..NBIN
-  const int lane = threadIdx.x & 63;
-  if (b > nbin) return;
-  double s1 = 0.0, s2 = 0.0;
-  for (int c = lane; c <= rc.kx; c += 64) {
-    int lo, hi;
-    column_shells(ph, rc, c, lo, hi);
-    if (b >= lo && b <= hi) {
-      s1 = s1 + d.part1[(size_t)c * nbin + (b - 1)];
-      s2 = s2 + d.part2[(size_t)c * nbin + (b - 1)];
+  const int nbin = ph.n / 2, kx = d.rc.kx;
+  const int o = threadIdx.x % kSumB, g = threadIdx.x / kSumB;
+  const int b = blockIdx.x * kSumB + o + 1;  // shell 1..NBIN
+  for (int c = threadIdx.x; c <= kx; c += kSumT) lh[c] = d.lohi[c];
+  __syncthreads();
+  double a1 = 0.0, a2 = 0.0;
+  for (int c0 = g; c0 <= kx; c0 += 8 * kSumG) {
+    double t1[8], t2[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {  // all in flight together
+      const int c = c0 + i * kSumG;
+      const bool in = c <= kx && b <= nbin && b >= lh[c].x && b <= lh[c].y;
+      t1[i] = in ? d.part1[(size_t)c * nbin + (b - 1)] : 0.0;
+      t2[i] = in ? d.part2[(size_t)c * nbin + (b - 1)] : 0.0;
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      a1 = a1 + t1[i];
+      a2 = a2 + t2[i];
     }
   }
-  s1 = wave_sum(s1);
-  s2 = wave_sum(s2);
-  if (lane != 0) return;
+  s1[g][o] = a1;
+  s2[g][o] = a2;
+  __syncthreads();
+#pragma unroll
+  for (int h = kSumG / 2; h > 0; h >>= 1) {
+    if (g < h) {
+      s1[g][o] = s1[g][o] + s1[g + h][o];
+      s2[g][o] = s2[g][o] + s2[g + h][o];
+    }
+    __syncthreads();
+  }
+  if (g != 0 || b > nbin) return;
   if (which == 0) {  // diagnostics.f90:42-45
-    d.out1[b - 1] = s1 / ph.dkx;
-    d.out2[b - 1] = s2 / ph.dkx;
+    d.out1[b - 1] = s1[0][o] / ph.dkx;
+    d.out2[b - 1] = s2[0][o] / ph.dkx;
   } else {
-    d.part1[(size_t)(rc.kx + 1) * nbin + (b - 1)] = s1;  // flzm
-    d.part2[(size_t)(rc.kx + 1) * nbin + (b - 1)] = s2;  // flem
+    d.part1[(size_t)(kx + 1) * nbin + (b - 1)] = s1[0][o];  // flzm
+    d.part2[(size_t)(kx + 1) * nbin + (b - 1)] = s2[0][o];  // flem
   }
 }
 
-// flz(i) = sum(flzm(i:NBIN)) in the reference's order (diagnostics.f90:104-109):
-// each thread sums its own suffix in increasing q, from LDS (workgroup g
-// stages flzm and flem from its first i on).
-__global__ void __launch_bounds__(kDiagT) suffix_k(DiagArgs d) {
-  extern __shared__ double ssm[];
-  const int nbin = d.ph.n / 2;
-  const int i0 = blockIdx.x * kDiagT, len = nbin - i0;
+// flz(i) = sum(flzm(i:NBIN)) and fle likewise (diagnostics.f90:104-109): a
+// scan from the last shell down in one workgroup, four shells a thread, a
+// fixed order (4.6 us at 4096^2; 36 with each thread adding its own suffix).
+// NBIN <= 4096.
+__global__ void __launch_bounds__(1024) suffix_k(DiagArgs d) {
+  __shared__ double w1[16], w2[16];
+  const int nbin = d.ph.n / 2, t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const double* flzm = d.part1 + (size_t)(d.rc.kx + 1) * nbin;
   const double* flem = d.part2 + (size_t)(d.rc.kx + 1) * nbin;
-  double* lz = ssm;
-  double* le = ssm + len;
-  for (int t = threadIdx.x; t < len; t += kDiagT) {
-    lz[t] = flzm[i0 + t];
-    le[t] = flem[i0 + t];
+  // thread t: the reversed positions 4t .. 4t+3, i.e. shells nbin-1-4t down
+  double z[4], e[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int q = nbin - 1 - (4 * t + i);
+    z[i] = q >= 0 ? flzm[q] : 0.0;
+    e[i] = q >= 0 ? flem[q] : 0.0;
+  }
+#pragma unroll
+  for (int i = 1; i < 4; ++i) {
+    z[i] = z[i] + z[i - 1];
+    e[i] = e[i] + e[i - 1];
+  }
+  double tz = z[3], te = e[3];  // inclusive scan of the threads' totals
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const double uz = __shfl_up(tz, o), ue = __shfl_up(te, o);
+    if (lane >= o) {
+      tz = tz + uz;
+      te = te + ue;
+    }
+  }
+  if (lane == 63) {
+    w1[wave] = tz;
+    w2[wave] = te;
   }
   __syncthreads();
-  const int i = i0 + (int)threadIdx.x;
-  if (i >= nbin) return;
-  double sz = 0.0, se = 0.0;
-  int q = i - i0;
-  // sixteen terms loaded together, then added one after the other in q order
-  for (; q + 16 <= len; q += 16) {
-    double tz[16], te[16];
+  double bz = __shfl_up(tz, 1), be = __shfl_up(te, 1);
+  if (lane == 0) bz = be = 0.0;
+  double pz = 0.0, pe = 0.0;  // the waves before, in order
+  for (int w = 0; w < wave; ++w) {
+    pz = pz + w1[w];
+    pe = pe + w2[w];
+  }
+  bz = pz + bz;
+  be = pe + be;
 #pragma unroll
-    for (int t = 0; t < 16; ++t) {
-      tz[t] = lz[q + t];
-      te[t] = le[q + t];
-    }
-#pragma unroll
-    for (int t = 0; t < 16; ++t) {
-      sz = sz + tz[t];
-      se = se + te[t];
+  for (int i = 0; i < 4; ++i) {
+    const int q = nbin - 1 - (4 * t + i);
+    if (q >= 0) {
+      d.out1[q] = be + e[i];  // fle
+      d.out2[q] = bz + z[i];  // flz
     }
   }
-  for (; q < len; ++q) {
-    sz = sz + lz[q];
-    se = se + le[q];
-  }
-  d.out1[i] = se;  // fle
-  d.out2[i] = sz;  // flz
 }
 
 // k2**a for the dissipation exponents of glob: repeated products for the
@@ -2419,32 +2479,41 @@ __device__ __forceinline__ double pow_k2(double k2, double a) {
 }
 
 // src/diagnostics.f90:147-163: one workgroup per column; each thread sums
-// its rows in order, then a fixed wavefront tree and the four waves in
-// order.  dise_* use k2**alpnu / ka for k2**(alpnu - alpv/2).
+// its rows in order (four loads ahead), then a fixed wavefront tree and the
+// four waves in order.  dise_* use k2**alpnu / ka for k2**(alpnu - alpv/2).
 __global__ void __launch_bounds__(kDiagT) glob_col_k(DiagArgs d) {
   const Phys& ph = d.ph;
   const Rect rc = d.rc;
   const int n = ph.n, c = blockIdx.x, Ky = rc.ky();
   const double fkx = (double)c * ph.dkx, fkxs = fkx * fkx;
   const double fac = (c == 0 || c == n / 2) ? 0.5 : 1.0;
+  const double2* z = d.z + (size_t)c * d.zcs;
   double acc[6] = {0, 0, 0, 0, 0, 0};
-  for (int r = threadIdx.x; r < Ky; r += kDiagT) {
-    if (c == 0 && r == 0) continue;
-    const int p = fft_of(r, rc, n);
-    const double fky = (double)kyi_of(p, n) * ph.dky;
-    const double k2 = fkxs + fky * fky;
-    const double ka = kalpha(ph, k2);
-    const double2 zv = d.z[(size_t)c * d.zcs + (size_t)r * d.zrs];
-    const double am = hypot(zv.x, zv.y);
-    const double scra = am * am;
-    const double dnu = 2.0 * fac * ph.nu * pow_k2(k2, ph.alpnu) * scra;
-    const double dmu = 2.0 * fac * ph.mu * pow_k2(k2, ph.alpmu) * scra;
-    acc[0] = acc[0] + fac * scra / ka;  // ee
-    acc[1] = acc[1] + fac * scra;       // zz
-    acc[2] = acc[2] + dnu;              // disz_nu
-    acc[3] = acc[3] + dmu;              // disz_mu
-    acc[4] = acc[4] + dnu / ka;         // dise_nu
-    acc[5] = acc[5] + dmu / ka;         // dise_mu
+  for (int rb = threadIdx.x; rb < Ky; rb += 4 * kDiagT) {
+    double2 zv[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int r = rb + i * kDiagT;
+      zv[i] = r < Ky ? z[(size_t)r * d.zrs] : make_double2(0.0, 0.0);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int r = rb + i * kDiagT;
+      if (r >= Ky || (c == 0 && r == 0)) continue;
+      const int p = fft_of(r, rc, n);
+      const double fky = (double)kyi_of(p, n) * ph.dky;
+      const double k2 = fkxs + fky * fky;
+      const double ka = kalpha(ph, k2);
+      const double a2 = fac * (zv[i].x * zv[i].x + zv[i].y * zv[i].y), ae = a2 / ka;
+      const double gnu = 2.0 * ph.nu * pow_k2(k2, ph.alpnu);
+      const double gmu = 2.0 * ph.mu * pow_k2(k2, ph.alpmu);
+      acc[0] = acc[0] + ae;        // ee
+      acc[1] = acc[1] + a2;        // zz
+      acc[2] = acc[2] + gnu * a2;  // disz_nu
+      acc[3] = acc[3] + gmu * a2;  // disz_mu
+      acc[4] = acc[4] + gnu * ae;  // dise_nu
+      acc[5] = acc[5] + gmu * ae;  // dise_mu
+    }
   }
   __shared__ double red[6][kDiagT / 64];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -2458,17 +2527,27 @@ __global__ void __launch_bounds__(kDiagT) glob_col_k(DiagArgs d) {
     const int q = threadIdx.x;
     double v = red[q][0];
     for (int w = 1; w < kDiagT / 64; ++w) v = v + red[q][w];
-    d.gpart[(size_t)c * 6 + q] = v;
+    d.gpart[(size_t)q * rc.kc() + c] = v;
   }
 }
 
-// One wavefront per quantity, over the columns in a fixed order.
-__global__ void __launch_bounds__(6 * 64) glob_sum_k(DiagArgs d) {
-  const int q = threadIdx.x >> 6, lane = threadIdx.x & 63;
+// Two wavefronts per quantity, over the columns in a fixed order.
+__global__ void __launch_bounds__(12 * 64) glob_sum_k(DiagArgs d) {
+  __shared__ double red[12];
+  const int q = threadIdx.x / 128, t = threadIdx.x % 128, kc = d.rc.kc();
+  const double* g = d.gpart + (size_t)q * kc;
   double s = 0.0;
-  for (int c = lane; c <= d.rc.kx; c += 64) s = s + d.gpart[(size_t)c * 6 + q];
+  for (int c0 = t; c0 < kc; c0 += 8 * 128) {
+    double v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = c0 + 128 * i < kc ? g[c0 + 128 * i] : 0.0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) s = s + v[i];
+  }
   s = wave_sum(s);
-  if (lane == 0) d.gout[q] = s;
+  if (t % 64 == 0) red[threadIdx.x / 64] = s;
+  __syncthreads();
+  if (t == 0) d.gout[q] = red[2 * q] + red[2 * q + 1];
 }
 
 __global__ void shell_index_k(Phys ph, int* ib) {
@@ -2633,38 +2712,26 @@ hipError_t launch_spectrum(const DiagArgs& d, int which, hipStream_t s) {
     column_shells(d.ph, d.rc, c, lo, hi);
     nbl = hi - lo + 1 > nbl ? hi - lo + 1 : nbl;
   }
-  // LDS: two sums per shell of a column, the chunk's run sums and keys, and
-  // one slot per wave
-  const size_t lds = sizeof(double) * (2 * (size_t)nbl + 2 * kDiagT) +
-                     sizeof(int) * (kDiagT + kDiagT / 64);
-  static bool attr = false;  // once per process: more than 64 KB of LDS at N = 8192
-  if (!attr && lds > 48 * 1024) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&shell_bin_k),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize,
-                                             (int)lds);
+  // LDS: two sums per shell of a column; 44 KB at N = 8192, 65,520 bytes (with
+  // the static part above the 64 KB a launch gets by itself) untruncated
+  const size_t lds = 2 * sizeof(double) * (size_t)nbl;
+  if (lds > 60 * 1024) {
+    const hipError_t e = hipFuncSetAttribute(
+        which == 0 ? reinterpret_cast<const void*>(&shell_bin_k<0>)
+                   : reinterpret_cast<const void*>(&shell_bin_k<1>),
+        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return e;
-    attr = true;
   }
-  shell_bin_k<<<d.rc.kc(), kDiagT, lds, s>>>(d, which, nbl);
-  shell_sum_k<<<(nbin * 64 + kDiagT - 1) / kDiagT, kDiagT, 0, s>>>(d, which);
-  if (which == 1) {
-    const size_t slds = 2 * sizeof(double) * (size_t)nbin;  // the first workgroup's
-    static bool sattr = false;
-    if (!sattr && slds > 48 * 1024) {
-      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&suffix_k),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize,
-                                               (int)slds);
-      if (e != hipSuccess) return e;
-      sattr = true;
-    }
-    suffix_k<<<(nbin + kDiagT - 1) / kDiagT, kDiagT, slds, s>>>(d);
-  }
+  if (which == 0) shell_bin_k<0><<<d.rc.kc(), kDiagT, lds, s>>>(d, nbl);
+  else shell_bin_k<1><<<d.rc.kc(), kDiagT, lds, s>>>(d, nbl);
+  shell_sum_k<<<(nbin + kSumB - 1) / kSumB, kSumT, 0, s>>>(d, which);
+  if (which == 1) suffix_k<<<1, 1024, 0, s>>>(d);
   return hipGetLastError();
 }
 
 hipError_t launch_glob(const DiagArgs& d, hipStream_t s) {
   glob_col_k<<<d.rc.kc(), kDiagT, 0, s>>>(d);
-  glob_sum_k<<<1, 6 * 64, 0, s>>>(d);
+  glob_sum_k<<<1, 12 * 64, 0, s>>>(d);
   return hipGetLastError();
 }
 

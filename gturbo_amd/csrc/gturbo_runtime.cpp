@@ -456,9 +456,18 @@ int r_pass(gt_ctx* c, const gt::PassArgs& a) {
   return GT_OK;
 }
 
+// Partial sums on the device, results in pinned memory that the kernels write
+// (at most 64 KB) and the entry points read after the stream.
 int ensure_diag(gt_ctx* c, const Rect& r) {
   const size_t nbin = c->n / 2;
-  const size_t need = 2 * (size_t)(r.kc() + 1) * nbin + 2 * nbin + (size_t)r.kc() * 6 + 6;
+  if (!c->dg_out) {
+    void* d = nullptr;
+    HIPCHK(hipHostMalloc(&c->dg_out, sizeof(double) * (2 * nbin + 6),
+                         hipHostMallocCoherent | hipHostMallocMapped));
+    HIPCHK(hipHostGetDevicePointer(&d, c->dg_out, 0));
+    c->dg_dev = static_cast<double*>(d);
+  }
+  const size_t need = 2 * (size_t)(r.kc() + 1) * nbin + (size_t)r.kc() * 7;
   if (need <= c->dg_cap) return GT_OK;
   if (c->dg) (void)hipFree(c->dg);
   c->dg = nullptr;
@@ -479,10 +488,11 @@ gt::DiagArgs diag_args(gt_ctx* c, const Mirror& z) {
   const size_t nbin = c->n / 2, kc = z.rect.kc();
   d.part1 = c->dg;
   d.part2 = d.part1 + (kc + 1) * nbin;
-  d.out1 = d.part2 + (kc + 1) * nbin;
+  d.gpart = d.part2 + (kc + 1) * nbin;
+  d.lohi = reinterpret_cast<int2*>(d.gpart + kc * 6);
+  d.out1 = c->dg_dev;
   d.out2 = d.out1 + nbin;
-  d.gpart = d.out2 + nbin;
-  d.gout = d.gpart + kc * 6;
+  d.gout = d.out2 + nbin;
   return d;
 }
 
@@ -762,6 +772,7 @@ int gt_destroy(gt_ctx* c) {
   if (c->flag) (void)hipFree(c->flag);
   if (c->spare) (void)hipFree(c->spare);
   if (c->dg) (void)hipFree(c->dg);
+  if (c->dg_out) (void)hipHostFree(c->dg_out);
   if (c->ph_host) (void)hipHostFree(c->ph_host);
   if (c->ph_dev && !c->ph_direct) (void)hipFree(c->ph_dev);
   for (hipEvent_t e : c->ph_ev)
@@ -1172,9 +1183,9 @@ int gt_spectrum(gt_ctx* c, const double* z, double* sp, double* sz) {
     HIPCHK(gt::launch_spectrum(d, 0, c->stream));
   }
   const size_t nbin = c->n / 2;
-  HIPCHK(hipMemcpyAsync(sp, d.out1, sizeof(double) * nbin, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipMemcpyAsync(sz, d.out2, sizeof(double) * nbin, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(hipStreamSynchronize(c->stream));
+  std::memcpy(sp, c->dg_out, sizeof(double) * nbin);
+  std::memcpy(sz, c->dg_out + nbin, sizeof(double) * nbin);
   return GT_OK;
 }
 
@@ -1196,9 +1207,9 @@ int gt_fluxes(gt_ctx* c, const double* z, const double* znl, double* fle, double
     HIPCHK(gt::launch_spectrum(d, 1, c->stream));
   }
   const size_t nbin = c->n / 2;
-  HIPCHK(hipMemcpyAsync(fle, d.out1, sizeof(double) * nbin, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipMemcpyAsync(flz, d.out2, sizeof(double) * nbin, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(hipStreamSynchronize(c->stream));
+  std::memcpy(fle, c->dg_out, sizeof(double) * nbin);
+  std::memcpy(flz, c->dg_out + nbin, sizeof(double) * nbin);
   return GT_OK;
 }
 
@@ -1215,8 +1226,8 @@ int gt_glob(gt_ctx* c, const double* z, double* out) {
     Timer t(c, GT_K_OTHER);
     HIPCHK(gt::launch_glob(d, c->stream));
   }
-  HIPCHK(hipMemcpyAsync(out, d.gout, sizeof(double) * 6, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(hipStreamSynchronize(c->stream));
+  std::memcpy(out, c->dg_out + c->n, sizeof(double) * 6);
   return GT_OK;
 }
 

@@ -122,3 +122,39 @@ def test_adjoint_dot_product(oracle_mod, n, alpv, rko, nsteps, kchk):
     assert _rel(wT, wT_o) < 1e-11
     lhs, rhs = float(np.sum(gT * dwT)), float(np.sum(g0 * dw0))
     assert abs(lhs - rhs) <= 1e-10 * abs(lhs)
+
+
+@pytest.mark.parametrize("n,truncate,lx", [(32, 1, 1), (64, 0, 2), (2048, 1, 1), (8192, 0, 1)])
+def test_shell_sums(n, truncate, lx):
+    """Spectrum and fluxes of a random spectrum against numpy: runs of shells
+    across chunks and waves, several columns per shell, the most LDS bins
+    (8192 untruncated).  Sums of up to 1e5 terms a shell: 1e-12 of each sum's
+    absolute terms."""
+    p = params_for(n, truncate=truncate, xlx=2 * np.pi * lx, ring=(3.0, 5.0))
+    s = Solver(p)
+    nh, nb = n // 2 + 1, n // 2
+    z, q = (random_spectral(n, k, truncated=bool(truncate)) for k in (1, 2))
+    s.enter_data(z)
+    s.enter_data(q)
+    sp, sz = s.spectrum(z)
+    fle, flz = s.fluxes(z, q)
+    ib = s.shell_index()
+    s.close()
+    zc, qc = (np.ascontiguousarray(a).view(np.complex128).reshape(n, nh) for a in (z, q))
+    kx = np.arange(nh) * s.dkx
+    ky = np.where(np.arange(n) <= n // 2, np.arange(n), np.arange(n) - n) * s.dky
+    k2 = kx[None, :] ** 2 + ky[:, None] ** 2
+    k2[0, 0] = 1.0
+    ok = (ib < nb) & (ib > 0)
+    fac = np.ones((1, nh))
+    fac[0, 0] = fac[0, -1] = 0.5
+
+    def bins(v):
+        return np.bincount(ib[ok] - 1, weights=v[ok], minlength=nb)
+
+    a2 = fac * np.abs(zc) ** 2
+    fz = 2 * fac * (zc.real * qc.real + zc.imag * qc.imag)
+    for got, v in ((sp, a2 / k2 / s.dkx), (sz, a2 / s.dkx)):
+        assert np.all(np.abs(got - bins(v)) <= 1e-12 * bins(np.abs(v)))
+    for got, v in ((fle, fz / k2), (flz, fz)):
+        assert np.max(np.abs(got - np.cumsum(bins(v)[::-1])[::-1])) <= 1e-12 * np.abs(v[ok]).sum()
