@@ -365,17 +365,18 @@ __device__ __forceinline__ void fft_held(double2* a, double2* buf, int j,
 }
 
 // ---------------------------------------------------------------------------
-// In-place radix-8 transforms of a 4096-point line over 512 threads (eight
-// whole waves, thread j = lane + 64 wave).  The first pass combines the
-// elements j + 512 r that thread j holds; its outputs go to LDS, and each
+// In-place radix-8 transforms of a 2048- or 4096-point line over T = N/8
+// threads (whole waves, thread j = lane + 64 wave).  The first pass combines
+// the elements j + T r that thread j holds; its outputs go to LDS, and each
 // later pass reads, transforms and writes back one run of the line that
-// belongs to a single wave (stride 64: wave j/64's 512 elements; stride 8
-// and 1: runs inside them).  Only the first exchange crosses waves, so a
-// transform needs one workgroup barrier plus one before its first write
+// belongs to a single wave (strides T/8 and T/64: runs inside the wave's 512
+// elements; the last pass eight consecutive ones, as one radix-8 butterfly at
+// 4096 and two radix-4 ones at 2048).  Only the first exchange crosses waves,
+// so a transform needs one workgroup barrier plus one before its first write
 // (when LDS may still be read by another wave), instead of two per pass.
 //   fft_dif: natural order in, out of order: thread j, register r holds
-//            X[D(j) + 512 r], D(j) = 64 (j mod 8) + 8 (j/8 mod 8) + j/64
-//            (the octal digits of j reversed).
+//            X[ip_row(j, r)] (the digits of 8 j + r reversed; at 4096
+//            D(j) + 512 r with D the octal digit reversal of j).
 //   fft_dit: the transposed algorithm (same twiddles, applied before each
 //            radix-8 DFT, passes in reverse): input in that order, natural
 //            order out.
@@ -383,9 +384,21 @@ __device__ __forceinline__ void fft_held(double2* a, double2* buf, int j,
 // thread plus constants, and a wave's accesses at stride 8 or 9 spread over
 // the banks.
 // ---------------------------------------------------------------------------
-constexpr int kIpLine = 4096 + 4096 / 8;  // double2 per line in LDS
+template <int LOGN>
+constexpr int ip_line() { return (1 << LOGN) + (1 << LOGN) / 8; }  // double2 in LDS
+constexpr int kIpLine = ip_line<12>();
 
 __device__ __forceinline__ int ip_pad(int e) { return e + (e >> 3); }
+
+// Output index of fft_dif in thread j, register r.
+template <int LOGN>
+__host__ __device__ __forceinline__ int ip_row(int j, int r) {
+  static_assert(LOGN == 11 || LOGN == 12, "in-place lines of 2048 or 4096 points");
+  if constexpr (LOGN == 12)
+    return 64 * (j & 7) + 8 * ((j >> 3) & 7) + (j >> 6) + 512 * r;
+  else
+    return (j >> 5) + 8 * ((j >> 2) & 7) + 128 * (j & 3) + 64 * (r >> 2) + 512 * (r & 3);
+}
 
 // t[r] *= W^(k r) (conjugated for S > 0), from w1 = W^k; each power is
 // applied as soon as it is formed (at most four live at a time).
@@ -404,28 +417,31 @@ __device__ __forceinline__ void apply_tw8(double2* t, double2 w1) {
   ap(t[7], cmul(w3, w4));
 }
 
-// Twiddles of the three twiddled passes of a 4096-point in-place transform
-// in thread j: W^j (stride 512), W^(8 (j % 64)) (stride 64), W^(64 (j % 8))
-// (stride 8), from the table read at stride TS.  The same for every
-// transform a thread runs, so a kernel running several may load them once.
+// Twiddles of the three twiddled passes of an in-place transform in thread
+// j: W^j (stride T), W^(8 (j % (T/8))), W^(64 (j % (T/64))), from the table
+// read at stride TS.  The same for every transform a thread runs, so a kernel
+// running several may load them once.
 struct IpTw {
   double2 w1, w2, w3;
 };
-template <int TS = 1>
-__device__ __forceinline__ IpTw ip_tw(const double2* __restrict__ tw, int j) {
-  return {tw[TS * j], tw[TS * 8 * (j & 63)], tw[TS * 64 * (j & 7)]};
-}
-// Twiddle sources for fft_dif / fft_dit: operator()(P) gives the twiddle of
-// pass P (1-3), called where the transform first needs it in flight.
-template <int TS>
+// Twiddle sources for fft_dif / fft_dit: at<P>() gives the twiddle of pass P
+// (1-3), called where the transform first needs it in flight.
+template <int LOGN, int TS>
 struct TwFromTable {
+  static constexpr int T = (1 << LOGN) / 8;
   const double2* __restrict__ tw;
   int j;
   template <int P>
   __device__ __forceinline__ double2 at() const {
-    return P == 1 ? tw[TS * j] : P == 2 ? tw[TS * 8 * (j & 63)] : tw[TS * 64 * (j & 7)];
+    return P == 1 ? tw[TS * j] : P == 2 ? tw[TS * 8 * (j & (T / 8 - 1))]
+                                        : tw[TS * 64 * (j & (T / 64 - 1))];
   }
 };
+template <int LOGN, int TS = 1>
+__device__ __forceinline__ IpTw ip_tw(const double2* __restrict__ tw, int j) {
+  const TwFromTable<LOGN, TS> t{tw, j};
+  return {t.template at<1>(), t.template at<2>(), t.template at<3>()};
+}
 struct TwHeld {
   const IpTw& w;
   template <int P>
@@ -434,11 +450,38 @@ struct TwHeld {
   }
 };
 
+// Runs of passes 2 and 3 in LDS: thread j's first element and the padded
+// distance of its r-th one.
+template <int LOGN>
+struct IpRun {
+  static constexpr int T = (1 << LOGN) / 8, S2 = T / 8, S3 = T / 64;
+  static __device__ __forceinline__ int base2(int j) {
+    return ip_pad((j / S2) * T + (j & (S2 - 1)));
+  }
+  static __device__ __forceinline__ int base3(int j) {
+    return ip_pad((j / S3) * S2 + (j & (S3 - 1)));
+  }
+  static constexpr int off1(int r) { return T * r + T * r / 8; }
+  static constexpr int off2(int r) { return S2 * r + S2 * r / 8; }
+  static constexpr int off3(int r) { return S3 * r + S3 * r / 8; }
+};
+// Last (stride 1) pass on the thread's eight consecutive elements.
+template <int LOGN, int S>
+__device__ __forceinline__ void ip_last(double2* a) {
+  if constexpr (LOGN == 12) {
+    dft<8, S>(a);
+  } else {
+    dft<4, S>(a);
+    dft<4, S>(a + 4);
+  }
+}
+
 // bar: barrier before the first LDS write (another wave may still read
 // LDS); a uniform run-time flag, so that a loop holds one copy of the code.
-template <int S, class TW>
+template <int LOGN, int S, class TW>
 __device__ __forceinline__ void fft_dif_t(double2* a, double2* buf, int j, const TW& T,
                                           bool bar) {
+  using R = IpRun<LOGN>;
   double2 wn = T.template at<1>();  // pass 1: W^(j r)
   dft<8, S>(a);
   apply_tw8<S>(a, wn);
@@ -447,42 +490,42 @@ __device__ __forceinline__ void fft_dif_t(double2* a, double2* buf, int j, const
   {
     double2* p = buf + ip_pad(j);
 #pragma unroll
-    for (int r = 0; r < 8; ++r) p[576 * r] = a[r];  // ip_pad(j + 512 r)
+    for (int r = 0; r < 8; ++r) p[R::off1(r)] = a[r];
   }
   __syncthreads();
-  {  // pass 2, stride 64: wave j/64's elements
-    double2* p = buf + ip_pad((j >> 6) * 512 + (j & 63));
+  {  // pass 2
+    double2* p = buf + R::base2(j);
 #pragma unroll
-    for (int r = 0; r < 8; ++r) a[r] = p[72 * r];
+    for (int r = 0; r < 8; ++r) a[r] = p[R::off2(r)];
     dft<8, S>(a);
     apply_tw8<S>(a, wn);
     wn = T.template at<3>();
 #pragma unroll
-    for (int r = 0; r < 8; ++r) p[72 * r] = a[r];
+    for (int r = 0; r < 8; ++r) p[R::off2(r)] = a[r];
   }
   wave_sync();
-  {  // pass 3, stride 8
-    double2* p = buf + ip_pad((j >> 3) * 64 + (j & 7));
+  {  // pass 3
+    double2* p = buf + R::base3(j);
 #pragma unroll
-    for (int r = 0; r < 8; ++r) a[r] = p[9 * r];
+    for (int r = 0; r < 8; ++r) a[r] = p[R::off3(r)];
     dft<8, S>(a);
     apply_tw8<S>(a, wn);
 #pragma unroll
-    for (int r = 0; r < 8; ++r) p[9 * r] = a[r];
+    for (int r = 0; r < 8; ++r) p[R::off3(r)] = a[r];
   }
   wave_sync();
   {  // pass 4, stride 1
     const double2* p = buf + 9 * j;  // ip_pad(8 j)
 #pragma unroll
     for (int r = 0; r < 8; ++r) a[r] = p[r];
-    dft<8, S>(a);
+    ip_last<LOGN, S>(a);
   }
 }
-template <int S, int TS = 1>
+template <int S, int TS = 1, int LOGN = 12>
 __device__ __forceinline__ void fft_dif(double2* a, double2* buf, int j,
                                         const double2* __restrict__ tw, bool bar) {
   asm volatile("" : "+v"(j));
-  fft_dif_t<S>(a, buf, j, TwFromTable<TS>{tw, j}, bar);
+  fft_dif_t<LOGN, S>(a, buf, j, TwFromTable<LOGN, TS>{tw, j}, bar);
 }
 // Held twiddles enter each transform opaque, so that the compiler keeps
 // forming the powers inside it rather than holding them across transforms.
@@ -491,12 +534,12 @@ __device__ __forceinline__ IpTw opaque(IpTw w) {
                "+v"(w.w3.y));
   return w;
 }
-template <int S>
-__device__ __forceinline__ void fft_dif(double2* a, double2* buf, int j, const IpTw& w,
-                                        bool bar) {
+template <int LOGN, int S>
+__device__ __forceinline__ void fft_dif_held(double2* a, double2* buf, int j, const IpTw& w,
+                                             bool bar) {
   asm volatile("" : "+v"(j));
   const IpTw lw = opaque(w);
-  fft_dif_t<S>(a, buf, j, TwHeld{lw}, bar);
+  fft_dif_t<LOGN, S>(a, buf, j, TwHeld{lw}, bar);
 }
 
 // Input as fft_dif leaves it; the thread's own LDS run is free to write
@@ -504,10 +547,11 @@ __device__ __forceinline__ void fft_dif(double2* a, double2* buf, int j, const I
 // elements: a barrier must precede the next LDS write.
 // BAR: start with a workgroup barrier (another wave may still read this
 // wave's run of LDS, e.g. after a preceding fft_dit).
-template <int S, bool BAR, class TW>
+template <int LOGN, int S, bool BAR, class TW>
 __device__ __forceinline__ void fft_dit_t(double2* a, double2* buf, int j, const TW& T) {
+  using R = IpRun<LOGN>;
   double2 wn = T.template at<3>();
-  dft<8, S>(a);  // pass 4, stride 1
+  ip_last<LOGN, S>(a);  // pass 4, stride 1
   if constexpr (BAR) __syncthreads();
   {
     double2* p = buf + 9 * j;
@@ -515,47 +559,47 @@ __device__ __forceinline__ void fft_dit_t(double2* a, double2* buf, int j, const
     for (int r = 0; r < 8; ++r) p[r] = a[r];
   }
   wave_sync();
-  {  // pass 3, stride 8
-    double2* p = buf + ip_pad((j >> 3) * 64 + (j & 7));
+  {  // pass 3
+    double2* p = buf + R::base3(j);
 #pragma unroll
-    for (int r = 0; r < 8; ++r) a[r] = p[9 * r];
+    for (int r = 0; r < 8; ++r) a[r] = p[R::off3(r)];
     apply_tw8<S>(a, wn);
     wn = T.template at<2>();
     dft<8, S>(a);
 #pragma unroll
-    for (int r = 0; r < 8; ++r) p[9 * r] = a[r];
+    for (int r = 0; r < 8; ++r) p[R::off3(r)] = a[r];
   }
   wave_sync();
-  {  // pass 2, stride 64
-    double2* p = buf + ip_pad((j >> 6) * 512 + (j & 63));
+  {  // pass 2
+    double2* p = buf + R::base2(j);
 #pragma unroll
-    for (int r = 0; r < 8; ++r) a[r] = p[72 * r];
+    for (int r = 0; r < 8; ++r) a[r] = p[R::off2(r)];
     apply_tw8<S>(a, wn);
     wn = T.template at<1>();
     dft<8, S>(a);
 #pragma unroll
-    for (int r = 0; r < 8; ++r) p[72 * r] = a[r];
+    for (int r = 0; r < 8; ++r) p[R::off2(r)] = a[r];
   }
   __syncthreads();
-  {  // pass 1, stride 512: natural order out
+  {  // pass 1: natural order out
     const double2* p = buf + ip_pad(j);
 #pragma unroll
-    for (int r = 0; r < 8; ++r) a[r] = p[576 * r];
+    for (int r = 0; r < 8; ++r) a[r] = p[R::off1(r)];
     apply_tw8<S>(a, wn);
     dft<8, S>(a);
   }
 }
-template <int S, bool BAR = false, int TS = 1>
+template <int S, bool BAR = false, int TS = 1, int LOGN = 12>
 __device__ __forceinline__ void fft_dit(double2* a, double2* buf, int j,
                                         const double2* __restrict__ tw) {
   asm volatile("" : "+v"(j));
-  fft_dit_t<S, BAR>(a, buf, j, TwFromTable<TS>{tw, j});
+  fft_dit_t<LOGN, S, BAR>(a, buf, j, TwFromTable<LOGN, TS>{tw, j});
 }
-template <int S, bool BAR = false>
-__device__ __forceinline__ void fft_dit(double2* a, double2* buf, int j, const IpTw& w) {
+template <int LOGN, int S, bool BAR = false>
+__device__ __forceinline__ void fft_dit_held(double2* a, double2* buf, int j, const IpTw& w) {
   asm volatile("" : "+v"(j));
   const IpTw lw = opaque(w);
-  fft_dit_t<S, BAR>(a, buf, j, TwHeld{lw});
+  fft_dit_t<LOGN, S, BAR>(a, buf, j, TwHeld{lw});
 }
 
 // 8192-point lines over 1024 threads (thread t holds x[t + 1024 r]): a

@@ -55,8 +55,9 @@ struct PassArgs {
   double2* znew;      // RK4 accumulator (compact)
   const double* emk;  // integrating factor (compact, real)
   double2* out;       // nonlinear term (compact), NLT mode
-  const double* ka;   // k2**(alpv/2) (compact); read by the batched passes and at
-                      // N <= 1024 when alpv != 2
+  const double* ka;   // k2**(alpv/2) (compact); read when alpv != 2 by the batched
+                      // passes, at N <= 1024, and for powers
+                      // other than roots
   double2* sst;       // if set: the stage input formed by this y pass is
                       // also stored here (compact), for the adjoint's recompute
   // batched ensemble passes only: x-pass packing (0 = one row per line,

@@ -49,19 +49,6 @@ __device__ __forceinline__ double kalpha(const Phys& ph, double k2) {
   }
 }
 
-// ka in a y pass specialised on the alpha kind: AK = 1 when alpv = 2 (ka =
-// k2, nothing else in the kernel), AK = 0 a per-thread table of ka built
-// once per column, AK = 2 ka where it is used (the batched passes, whose
-// members differ in alpha): k2 for alpv = 2, else the member's table of ka
-// in the compact layout, built on the host with the same expressions as
-// kalpha (no power or root code in those kernels).
-template <int AK>
-__device__ __forceinline__ double kalpha_t(const PassArgs& a, double k2, unsigned q) {
-  if constexpr (AK == 1) return k2;
-  else if constexpr (AK == 0) return kalpha(a.ph, k2);
-  else return a.ph.akind == 1 ? k2 : a.ka[q];
-}
-
 // With the 2/3 rule the kept rectangle stays below |k| = 3N/8, so of a
 // thread's positions p = j + r*N/8 the ones with r = 3, 4 are never kept:
 // those inputs are zero and those outputs unused.  TR = 1 makes that a
@@ -113,27 +100,17 @@ __device__ __forceinline__ void st_state(double2* p, double2 v) {
   }
 }
 
-template <int LOGN, int BT>
-__device__ __forceinline__ void load_tile(double2* lds,
-                                          const double2* __restrict__ src,
-                                          int tid) {
-  constexpr int N = 1 << LOGN, NTHR = BT * (N / 16), LINE = Line<LOGN>::PADDED;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    int e = tid + NTHR * i;
-    lds[(e % BT) * LINE + lpad(e / BT)] = src[e];
-  }
-}
-
-template <int LOGN, int BT>
-__device__ __forceinline__ void store_tile(double2* __restrict__ dst,
-                                           const double2* lds, int tid) {
-  constexpr int N = 1 << LOGN, NTHR = BT * (N / 16), LINE = Line<LOGN>::PADDED;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    int e = tid + NTHR * i;
-    dst[e] = lds[(e % BT) * LINE + lpad(e / BT)];
-  }
+// ka in a y pass specialised on the alpha kind, where it is used: AK = 1
+// when alpv = 2 (ka = k2, nothing else in the kernel); AK = 2 (the batched
+// passes, whose members differ in alpha) k2 for alpv = 2, else the member's
+// table of ka in the compact layout, built with the same expressions as
+// kalpha (no power or root code in those kernels); AK = 3 (alpv != 2, N >=
+// 2048) square roots for alpv = 1 and 1/2, else the table.
+template <int AK>
+__device__ __forceinline__ double kalpha_t(const PassArgs& a, double k2, unsigned q) {
+  if constexpr (AK == 1) return k2;
+  else if constexpr (AK == 2) return a.ph.akind == 1 ? k2 : a.ka[q];
+  else return a.ph.akind == 2 ? sqrt(k2) : a.ph.akind == 3 ? sqrt(sqrt(k2)) : a.ka[q];
 }
 
 // Workgroup -> tile remap so that consecutive tiles run on one XCD
@@ -277,27 +254,36 @@ __device__ __forceinline__ double2 field_of(int f, double2 s, double fkx, double
   return make_double2(kxn * s.y, -kxn * s.x);
 }
 
+// double2 of LDS of an in-place line (8192: two 4096-point problems).
+template <int LOGN>
+__host__ __device__ constexpr int ip_lds() {
+  return LOGN == 13 ? 2 * kIpLine : LOGN == 11 ? ip_line<11>() : kIpLine;
+}
+
 // One tile of BT kx-columns; lds holds BT padded lines.  SCHED is the radix
 // order of the transforms (fft_reg).
-// IP (4096-point lines only): the y buffers hold the rows of a column in
-// the order the in-place transforms use (slot j + 512 r holds physical row
-// D(j) + 512 r, D the octal digit reversal of j); the forward transforms
-// (fft_dit) take the loaded slots and return natural ky order, the inverse
-// ones (fft_dif) return slot order for the stores.  Each line is eight
-// whole waves: line b = wave mod 2, j = 64 (wave / 2) + lane.  The x pass
-// transforms rows, whichever rows a slot pair holds.
+// IP (N >= 2048): the y buffers hold the rows of a column in the order the
+// in-place transforms use (slot j + N/8 r holds physical row ip_row(j, r));
+// the forward transforms (fft_dit) take the loaded slots and return natural
+// ky order, the inverse ones (fft_dif) return slot order for the stores.
+// Each line is whole waves: of two lines, line b = wave mod 2, j = 64 (wave
+// / 2) + lane.  The x pass transforms rows, whichever rows a slot pair holds.
 template <int LOGN, int MODE, int AK, int TR, int BT, int SCHED, bool IP = false>
 __device__ __forceinline__ void c_body(const PassArgs& a, int tile, int tid,
                                        double2* lds, const double2* tw) {
   constexpr int N = 1 << LOGN, TPL = N / kE;
-  constexpr int LINE = IP ? (LOGN == 13 ? 2 : 1) * kIpLine : Line<LOGN>::PADDED;
-  static_assert(!IP || (LOGN == 12 && BT == 2) || (LOGN == 13 && BT == 1),
-                "in-place y pass: two 4096-point lines or one 8192-point line");
+  constexpr int LINE = IP ? ip_lds<LOGN>() : Line<LOGN>::PADDED;
+  static_assert(!IP || (LOGN == 13 && BT == 1) || ((LOGN == 11 || LOGN == 12) && BT <= 2),
+                "in-place y pass: up to two lines, or one 8192-point line");
   constexpr bool FWD = MODE != C_START;
   constexpr bool INV = MODE == C_START || MODE == C_RK4_1 || MODE == C_RK4_2 ||
                        MODE == C_RK4_3 || MODE == C_RK2_1 || MODE == C_RK4_4S ||
                        MODE == C_RK2_2S;
   constexpr bool NT = LOGN >= 12;    // state accesses that bypass the caches
+  // ka formed or read once for u and v, not at each of them (below; alpha 1.5
+  // at 4096 1332 -> 1290 us a step, at 8192 5928 -> 5829; the batched sizes
+  // keep the rounding they share with f_pass)
+  constexpr bool ONCE = LOGN >= 12;
   constexpr bool NT2 = LOGN == 12;   // Y2 reads likewise, at 4096 only
   int b, j;
   if constexpr (IP && BT == 2) {
@@ -319,9 +305,13 @@ __device__ __forceinline__ void c_body(const PassArgs& a, int tile, int tid,
   const unsigned cbase = (unsigned)c * (unsigned)a.kyp;
   double2 s[kE];
   double2 z[kE];
-  // 4096-point in-place transforms: their three twiddles, loaded once.
+  // the batched passes loop over items: another wave may still read the last
+  // one's LDS
+  constexpr bool LOOP = AK == 2;
+  // in-place transforms up to 4096 points: their three twiddles, loaded once.
+  constexpr bool HELD = IP && LOGN <= 12 && !LOOP;
   IpTw ytw{};
-  if constexpr (IP && LOGN == 12) ytw = ip_tw(tw, j);
+  if constexpr (HELD) ytw = ip_tw<LOGN>(tw, j);
 
   if constexpr (FWD) {
     double2 A[kE];
@@ -329,7 +319,8 @@ __device__ __forceinline__ void c_body(const PassArgs& a, int tile, int tid,
     const double2* srcA = a.y2;
 #pragma unroll
     for (int r = 0; r < kE; ++r) z[r] = ld_state<NT2>(&srcA[yrow_off(j + TPL * r, a.ntiles, BT) + colo]);
-    if constexpr (IP && LOGN == 12) fft_dit<-1, false>(z, buf, j, ytw);
+    if constexpr (HELD) fft_dit_held<LOGN, -1>(z, buf, j, ytw);
+    else if constexpr (IP && LOOP) fft_dit<-1, true, 1, LOGN>(z, buf, j, tw);
     else if constexpr (IP) fft_dit2<-1, false>(z, buf, j, tw);
     else fft_reg<LOGN, -1, SCHED>(z, buf, j, tw);
 #pragma unroll
@@ -337,7 +328,8 @@ __device__ __forceinline__ void c_body(const PassArgs& a, int tile, int tid,
     const double2* srcB = a.y2 + (size_t)a.ntiles * N * BT;
 #pragma unroll
     for (int r = 0; r < kE; ++r) z[r] = ld_state<NT2>(&srcB[yrow_off(j + TPL * r, a.ntiles, BT) + colo]);
-    if constexpr (IP && LOGN == 12) fft_dit<-1, true>(z, buf, j, ytw);
+    if constexpr (HELD) fft_dit_held<LOGN, -1, true>(z, buf, j, ytw);
+    else if constexpr (IP && LOOP) fft_dit<-1, true, 1, LOGN>(z, buf, j, tw);
     else if constexpr (IP) fft_dit2<-1, true>(z, buf, j, tw);
     else fft_reg<LOGN, -1, SCHED>(z, buf, j, tw);
     int je = j;
@@ -384,18 +376,6 @@ __device__ __forceinline__ void c_body(const PassArgs& a, int tile, int tid,
         if (live_r<TR>(r) && colok && row >= 0) a.sst[cbase + (unsigned)row] = s[r];
       }
     }
-    // ka is tabled only for AK = 0; for AK = 1 it is k2 and for AK = 2 it is
-    // evaluated where needed.
-    double ka[AK == 0 ? kE : 1];
-    if constexpr (AK == 0) {
-#pragma unroll
-      for (int r = 0; r < kE; ++r) {
-        const int p = j + TPL * r;
-        const double fky = (double)kyi_of(p, N) * ph.dky;
-        const bool use = live_r<TR>(r) && colok && row_of(p, rc, N) >= 0 && !(c == 0 && p == 0);
-        ka[r] = use ? kalpha(ph, fkxs + fky * fky) : 1.0;
-      }
-    }
 #pragma unroll 1
     for (int f = 0; f < 3; ++f) {
       int jo = j;
@@ -409,17 +389,30 @@ __device__ __forceinline__ void c_body(const PassArgs& a, int tile, int tid,
             v = s[r];
           } else if (!(c == 0 && p == 0)) {  // nlt.f90:25
             const double fky = (double)kyi_of(p, N) * ph.dky;
-            const double kar =
-                AK == 0 ? ka[AK == 0 ? r : 0]
-                        : kalpha_t<AK>(a, fkxs + fky * fky, cbase + (unsigned)row_of(p, rc, N));
-            v = field_of(f, s[r], fkx, fky, kar);
+            if constexpr (ONCE) {
+              // q is not needed any more: q/ka in its place, ka formed (or
+              // read) once for both velocity components
+              if (f == 1) {
+                const double kar = kalpha_t<AK>(a, fkxs + fky * fky,
+                                                cbase + (unsigned)row_of(p, rc, N));
+                s[r] = make_double2(s[r].x / kar, s[r].y / kar);
+                v = make_double2(-fky * s[r].y, fky * s[r].x);
+              } else {
+                v = make_double2(fkx * s[r].y, -fkx * s[r].x);
+              }
+            } else {
+              v = field_of(f, s[r], fkx, fky,
+                           kalpha_t<AK>(a, fkxs + fky * fky,
+                                        cbase + (unsigned)row_of(p, rc, N)));
+            }
           }
         }
         z[r] = v;
       }
       if constexpr (IP) {
         // a barrier first unless nothing has used LDS since the table staging
-        if constexpr (LOGN == 12) fft_dif<+1>(z, buf, j, ytw, FWD || f > 0);
+        if constexpr (HELD) fft_dif_held<LOGN, +1>(z, buf, j, ytw, FWD || f > 0);
+        else if constexpr (LOOP) fft_dif<+1, 1, LOGN>(z, buf, j, tw, true);
         else fft_dif2<+1>(z, buf, j, tw, FWD || f > 0);
       } else {
         fft_reg<LOGN, +1, SCHED>(z, buf, j, tw);
@@ -439,18 +432,25 @@ __device__ __forceinline__ void c_body(const PassArgs& a, int tile, int tid,
   }
 }
 
+// Which y passes use the in-place transforms, for any alpha: on the 2/3
+// rectangle RK4 steps at 2048 304 (alpha 2), 356 (1), 382 (1.5) -> 292, 297,
+// 301 us, at 4096 alpha 1 1252 -> 1143, at 8192 alpha 1 6228 -> 5545, 1.5
+// 6397 -> 5829 (Stockham passes with ka in registers, which spilled).  On the
+// full one only at 8192 (9784 -> 9324); at 4096 its eight live values a field
+// leave no registers for the held twiddles (1887 -> 2080), at 2048 no change.
+template <int LOGN, int AK, int TR>
+__host__ __device__ constexpr bool c_pass_ip() { return TR == 1 || LOGN == 13; }
 template <int LOGN, int MODE, int AK, int TR>
-__global__ void __launch_bounds__(bt_of(LOGN) * (1 << LOGN) / kE, AK == 1 ? 4 : 1)
-    c_pass(PassArgs a) {
+__global__ void __launch_bounds__(bt_of(LOGN) * (1 << LOGN) / kE, 4) c_pass(PassArgs a) {
   constexpr int BT = bt_of(LOGN);
-  // Row slots in transform order (in-place transforms) for alpha = 2 on the
-  // 2/3 rectangle; every y pass of a run has the same AK and TR, so the
-  // buffers' row order is the same in all of them.
-  constexpr bool IP = (LOGN == 12 || LOGN == 13) && AK == 1 && TR == 1;
-  // 4096-point in-place transforms hold their three twiddles in registers
-  // (read once from memory): no table in LDS.
-  constexpr bool HELD = IP && LOGN == 12;
-  __shared__ double2 lds[IP ? 2 * kIpLine : BT * Line<LOGN>::PADDED];
+  // Row slots in transform order (in-place transforms) on the 2/3 rectangle;
+  // every y pass of a run has the same AK and TR, so the buffers' row order is
+  // the same in all of them.
+  constexpr bool IP = c_pass_ip<LOGN, AK, TR>();
+  // The in-place transforms up to 4096 points hold their three twiddles in
+  // registers (read once from memory): no table in LDS.
+  constexpr bool HELD = IP && LOGN <= 12;
+  __shared__ double2 lds[BT * (IP ? ip_lds<LOGN>() : Line<LOGN>::PADDED)];
   __shared__ double2 twl[HELD ? 1 : tw_lds_size<LOGN>()];
   const double2* tw = HELD ? a.tw : stage_tw<LOGN>(twl, a.tw, threadIdx.x, blockDim.x);
   // 8192: a one-column workgroup shares each line of Y1 and Y2 with the next
@@ -864,9 +864,19 @@ template <int LOGN, int TR, int BT, int NL, int SCHED, bool TWPF = false>
 __device__ __forceinline__ void pair_body(const PassArgs& a, int g, int tid,
                                           double2* lds, const double2* tw) {
   constexpr int N = 1 << LOGN, TPL = N / kE;
-  constexpr int LINE = Line<LOGN>::PADDED;
+  // 2048- and 4096-point lines use the in-place transforms (lines of whole
+  // waves): the inverse ones leave x out of order, which the pointwise
+  // products do not mind, and the forward ones restore natural order for
+  // split_store.
+  constexpr bool IP = (LOGN == 11 && NL <= 2) || (LOGN == 12 && NL == 1);
+  constexpr int LINE = IP ? ip_lds<LOGN>() : Line<LOGN>::PADDED;
   int pl, j;
-  line_map<TPL, NL>(tid, pl, j);
+  if constexpr (IP && NL == 2) {
+    pl = (tid >> 6) & 1;
+    j = ((tid >> 7) << 6) | (tid & 63);
+  } else {
+    line_map<TPL, NL>(tid, pl, j);
+  }
   double2* buf = lds + pl * LINE;
   const int y0 = 2 * (g * NL + pl);
   const int kxm = a.rc.kx;
@@ -879,24 +889,23 @@ __device__ __forceinline__ void pair_body(const PassArgs& a, int g, int tid,
   const unsigned i0 = Y1 ? y1_off(y0, 0, cols) : r0, i1 = Y1 ? y1_off(y0 + 1, 0, cols) : r1;
   const unsigned fq = 0, fu = fs1, fv = 2 * fs1;
 
-  // 4096-point lines of a one-pair workgroup use the in-place transforms:
-  // the inverse ones leave x out of order, which the pointwise products do
-  // not mind, and the forward ones restore natural order for split_store.
-  constexpr bool IP = LOGN == 12 && NL == 1 && TWPF;
   constexpr bool IP2 = LOGN == 13 && NL == 1 && TWPF;  // 8192: radix 2, then two 4096s
-  // 4096: the three twiddles every transform of the thread uses, loaded once.
+  // the three twiddles every transform of the thread uses, loaded once (from
+  // memory; a table in LDS is read where it is needed)
   IpTw w{};
-  if constexpr (IP) w = ip_tw(tw, j);
+  if constexpr (IP && TWPF) w = ip_tw<LOGN>(tw, j);
   // bar: another wave may still read LDS (ignored by the Stockham transforms,
   // which synchronise on every transpose)
   auto inv = [&](double2* v, bool bar) {
-    if constexpr (IP) fft_dif<+1>(v, buf, j, w, bar);
+    if constexpr (IP && TWPF) fft_dif_held<LOGN, +1>(v, buf, j, w, bar);
+    else if constexpr (IP) fft_dif<+1, 1, LOGN>(v, buf, j, tw, bar);
     else if constexpr (IP2) fft_dif2<+1>(v, buf, j, tw, bar);
     else fft_reg<LOGN, +1, SCHED, TWPF>(v, buf, j, tw);
   };
   auto fwd = [&](double2* v) {
     if constexpr (IP || IP2) {
-      if constexpr (IP) fft_dit<-1>(v, buf, j, w);
+      if constexpr (IP && TWPF) fft_dit_held<LOGN, -1>(v, buf, j, w);
+      else if constexpr (IP) fft_dit<-1, false, 1, LOGN>(v, buf, j, tw);
       else fft_dit2<-1>(v, buf, j, tw);
       __syncthreads();  // every wave's reads done before split_store writes
     } else {
@@ -1051,7 +1060,7 @@ __global__ void __launch_bounds__((1 << LOGN) / kE, 4)
     r_pass_pair(PassArgs a) {
   // Twiddles from memory: these workgroups are short-lived (one row pair),
   // and staging the table in LDS measured slower here.
-  __shared__ double2 lds[LOGN == 12 ? kIpLine : LOGN == 13 ? 2 * kIpLine : Line<LOGN>::PADDED];
+  __shared__ double2 lds[ip_lds<LOGN>()];
   pair_body<LOGN, TR, bt_of(LOGN), 1, 0, true>(a, xcd_remap(blockIdx.x, gridDim.x),
                                                threadIdx.x, lds, a.tw);
 }
@@ -1072,9 +1081,8 @@ __global__ void __launch_bounds__((1 << LOGN) / kE, 4)
 // N = 4096 and 8192 (see c_body), else s.
 template <int LOGN>
 __device__ __forceinline__ int slot_row(int s) {
-  auto d = [](int j) { return 64 * (j & 7) + 8 * ((j >> 3) & 7) + (j >> 6); };
-  if constexpr (LOGN == 12) return d(s & 511) + (s & ~511);
-  else if constexpr (LOGN == 13) return 2 * (d(s & 511) + 512 * (s >> 10)) + ((s >> 9) & 1);
+  if constexpr (LOGN == 12) return ip_row<12>(s & 511, s >> 9);
+  else if constexpr (LOGN == 13) return 2 * ip_row<12>(s & 511, s >> 10) + ((s >> 9) & 1);
   else return s;
 }
 
@@ -1750,7 +1758,7 @@ __host__ __device__ inline int rect_tr(const Rect& rc, int n) {
 template <int L>
 hipError_t c_pass_launch(int mode, const PassArgs& a, hipStream_t s) {
   const int tr = rect_tr(a.rc, 1 << L);
-  constexpr int AK = L <= kFpMaxLogn ? 2 : 0;  // alpha != 2: table of ka, or ka in registers
+  constexpr int AK = L <= kFpMaxLogn ? 2 : 3;
   if (a.ph.akind == 1)
     return tr ? c_pass_launch_ak<L, 1, 1>(mode, a, s) : c_pass_launch_ak<L, 1, 0>(mode, a, s);
   return tr ? c_pass_launch_ak<L, AK, 1>(mode, a, s) : c_pass_launch_ak<L, AK, 0>(mode, a, s);
@@ -1883,14 +1891,14 @@ __device__ __forceinline__ const double2* ens_stage_tw(double2* twl, const PassA
 template <int T, int MODE, int SCHED, int L>
 __device__ __forceinline__ void ens_c_one(const PassArgs& a, int tile, int tid,
                                           double2* lds, const double2* tw) {
-  c_body<L, MODE, 2, 1, ens_lines(T, L), SCHED>(a, tile, tid, lds, tw);
+  c_body<L, MODE, 2, 1, ens_lines(T, L), SCHED, L == 11>(a, tile, tid, lds, tw);
 }
 
 template <int T, int MODE, int SCHED>
 __global__ void __launch_bounds__(T, 4)
     ens_c_pass(const PassArgs* __restrict__ descs, const uint32_t* __restrict__ items,
                int nitems) {
-  __shared__ double2 lds[T * 17 / 2];
+  __shared__ double2 lds[T * 9];
   __shared__ double2 twl[tw_span<kEnsMaxLogn>()];
   const double2* cur = nullptr;
   for (int w = blockIdx.x; w < nitems; w += gridDim.x) {
@@ -1925,7 +1933,7 @@ template <int TX, int TY, int SCHED>
 __global__ void __launch_bounds__(TX, 4)
     ens_r_pass(const PassArgs* __restrict__ descs, const uint32_t* __restrict__ items,
                int nitems) {
-  __shared__ double2 lds[TX * 17 / 2];
+  __shared__ double2 lds[TX * 9];
   __shared__ double2 twl[tw_span<kEnsMaxLogn>()];
   const double2* cur = nullptr;
   for (int w = blockIdx.x; w < nitems; w += gridDim.x) {

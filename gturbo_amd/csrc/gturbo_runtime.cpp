@@ -235,10 +235,11 @@ int rect_tables(gt_ctx* c, const Rect& r, RectTables** out) {
 }
 
 // Table of ka = k2**(alpv/2) of one rectangle for the passes that read it
-// (alpv != 2), built on the device once; null when the passes form ka.
+// (alpv != 2; from N = 2048 not for the square roots), built on the device
+// once; null when the passes form ka.
 int rect_ka(gt_ctx* c, const Rect& r, const double** out) {
   *out = nullptr;
-  if (c->ph.akind == 1 || c->logn > gt::kFpMaxLogn) return GT_OK;
+  if (c->ph.akind == 1 || (c->logn > gt::kFpMaxLogn && c->ph.akind != 0)) return GT_OK;
   RectTables& t = c->tab[rect_kind(c, r)];
   if (!t.ka) {
     const int kyp = kyp_of(r);

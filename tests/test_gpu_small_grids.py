@@ -158,3 +158,12 @@ def test_shell_sums(n, truncate, lx):
         assert np.all(np.abs(got - bins(v)) <= 1e-12 * bins(np.abs(v)))
     for got, v in ((fle, fz / k2), (flz, fz)):
         assert np.max(np.abs(got - np.cumsum(bins(v)[::-1])[::-1])) <= 1e-12 * np.abs(v[ok]).sum()
+
+
+@pytest.mark.parametrize("n,alpv,truncate", [(2048, 2.0, 1), (2048, 1.5, 0), (2048, 1.5, 1),
+                                             (4096, 1.5, 1)])
+def test_forced_steps_large(oracle_mod, n, alpv, truncate):
+    """The in-place y passes and the ka table at 2048 and 4096: two forced RK4
+    steps with the fused boundary between them (1e-12 as above)."""
+    p = params_for(n, alpv=alpv, truncate=truncate, ring=(10.0, 20.0))
+    assert _steps(oracle_mod, p, 2) < 1e-12

@@ -233,3 +233,61 @@ def test_row_pair_blocks_of_the_y1_fields(kc):
         assert len(half) == 4
     ntiles = (kc + 1) // 2
     assert 2 * ntiles <= cols  # the last tile's second column is inside the field
+
+
+def _ip_row11(j, r):
+    """Output index of the 2048-point fft_dif in thread j, register r."""
+    return (j >> 5) + 8 * ((j >> 2) & 7) + 128 * (j & 3) + 64 * (r >> 2) + 512 * (r & 3)
+
+
+def _ip_tw(k, n, s):
+    return np.exp(s * 2j * np.pi * k / n)
+
+
+def _bfly(v, s):
+    k = np.arange(len(v))
+    return np.exp(s * 2j * np.pi * np.outer(k, k) / len(v)) @ v
+
+
+@pytest.mark.parametrize("s", [+1, -1])
+def test_in_place_2048_transforms_reproduce_the_dft(s):
+    """fft_dif at 2048 points (strides 256, 32, 4, then two radix-4
+    butterflies a thread) leaves X[ip_row(j, r)]; fft_dit takes that order
+    back; after the first exchange every pass stays inside a wave's 512
+    elements, at the padded offsets the kernel uses."""
+    n, T, S2, S3 = 2048, 256, 32, 4
+    pad = lambda e: e + (e >> 3)  # noqa: E731
+    rng = np.random.default_rng(11)
+    x = rng.standard_normal(n) + 1j * rng.standard_normal(n)
+    ref = np.fft.ifft(x) * n if s > 0 else np.fft.fft(x)
+    r8 = np.arange(8)
+    runs = {1: lambda j: j + T * r8, 2: lambda j: (j // S2) * T + (j & (S2 - 1)) + S2 * r8,
+            3: lambda j: (j // S3) * S2 + (j & (S3 - 1)) + S3 * r8, 4: lambda j: 8 * j + r8}
+    offs = {1: T * r8 + T * r8 // 8, 2: S2 * r8 + S2 * r8 // 8, 3: S3 * r8 + S3 * r8 // 8, 4: r8}
+    tw = {1: lambda j: _ip_tw(j * r8, n, s), 2: lambda j: _ip_tw(8 * (j & (S2 - 1)) * r8, n, s),
+          3: lambda j: _ip_tw(64 * (j & (S3 - 1)) * r8, n, s)}
+    for p, run in runs.items():
+        for j in range(T):
+            e = run(j)
+            assert np.array_equal(pad(e), pad(e[0]) + offs[p])
+            assert p == 1 or np.all(e // 512 == j // 64)
+
+    def last(v):
+        return np.concatenate([_bfly(v[:4], s), _bfly(v[4:], s)])
+
+    buf = x.copy()
+    for p in (1, 2, 3):
+        for j in range(T):
+            buf[runs[p](j)] = _bfly(buf[runs[p](j)], s) * tw[p](j)
+    order = np.array([[_ip_row11(j, r) for r in range(8)] for j in range(T)])
+    out = np.array([last(buf[runs[4](j)]) for j in range(T)])
+    assert np.abs(out - ref[order]).max() < 1e-9 * np.abs(ref).max()
+    assert np.array_equal(np.sort(order.ravel()), np.arange(n))
+
+    buf = np.zeros(n, complex)
+    for j in range(T):
+        buf[runs[4](j)] = last(x[order[j]])
+    for p in (3, 2, 1):
+        for j in range(T):
+            buf[runs[p](j)] = _bfly(buf[runs[p](j)] * tw[p](j), s)
+    assert np.abs(buf - ref).max() < 1e-9 * np.abs(ref).max()
