@@ -2193,9 +2193,10 @@ __global__ void ens_tick_k(int* step) { step[0] = step[0] + 1; }
 // half.  One barrier per half instead of two per chunk, and the next chunk's
 // loads are issued before this one is summed.  The column's bins go to
 // part[c][b]; a second launch sums part[.][b] over the columns.  4096^2
-// spectrum: bins 42 us (54 with a barrier pair per chunk and hypot; 60 MB,
-// bound by the instructions of the root, the division and the scan), columns
-// 10 us (27 with one shell's column of part per wavefront).
+// spectrum: bins 36 us (54 with a barrier pair per chunk and hypot, 42 with
+// the scan through LDS and a double-precision root; 60 MB, bound by the some
+// 300 instructions a chunk), columns 10 us (27 with one shell's column of
+// part per wavefront).
 // ---------------------------------------------------------------------------
 
 __host__ __device__ __forceinline__ int shell_of(const Phys& ph, double fkxs, int p) {
@@ -2221,26 +2222,48 @@ __host__ __device__ __forceinline__ void column_shells(const Phys& ph, const Rec
 
 constexpr int kDiagT = 256;  // threads of a diagnostics workgroup (4 waves)
 
+// v of another lane of the wave, by a data-parallel move (0 where there is
+// none): row_shr d within 16 lanes, the last lane of the row or half before.
+template <int CTRL>
+__device__ __forceinline__ double lane_dpp(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
 // Inclusive sums of v1, v2 over each run of equal keys in the wave (runs are
-// contiguous, heads the ballot of their first lanes).
+// contiguous, heads the ballot of their first lanes): a scan within the rows
+// of 16 lanes, then the rows and halves a run crosses, without LDS traffic.
 __device__ __forceinline__ void wave_runs(unsigned long long heads, int lane, double& v1,
                                           double& v2) {
-  // lanes of the run at or below this one
+  // lanes of the run before this one, in the wave and in the lane's row
   const int back = lane - (63 - __clzll((long long)(heads & (~0ull >> (63 - lane)))));
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const double t1 = __shfl_up(v1, d), t2 = __shfl_up(v2, d);
-    if (d <= back) {
-      v1 = v1 + t1;
-      v2 = v2 + t2;
-    }
-  }
+  const int rb = back < (lane & 15) ? back : (lane & 15);
+  auto add = [&](bool c, double t1, double t2) {
+    v1 = c ? v1 + t1 : v1;
+    v2 = c ? v2 + t2 : v2;
+  };
+  add(rb >= 1, lane_dpp<0x111>(v1), lane_dpp<0x111>(v2));
+  add(rb >= 2, lane_dpp<0x112>(v1), lane_dpp<0x112>(v2));
+  add(rb >= 4, lane_dpp<0x114>(v1), lane_dpp<0x114>(v2));
+  add(rb >= 8, lane_dpp<0x118>(v1), lane_dpp<0x118>(v2));
+  // lane 15 to row 1, lane 47 to row 3; lane 31 to rows 2 and 3
+  add((lane & 16) != 0 && back > (lane & 15), lane_dpp<0x142>(v1), lane_dpp<0x142>(v2));
+  add((lane & 32) != 0 && back > (lane & 31), lane_dpp<0x143>(v1), lane_dpp<0x143>(v2));
 }
 
 __device__ __forceinline__ double lane_value(double v, int lane) {
   const int lo = __builtin_amdgcn_readlane(__double2loint(v), lane);
   const int hi = __builtin_amdgcn_readlane(__double2hiint(v), lane);
   return __hiloint2double(hi, lo);
+}
+
+// int(sqrt(k2)) of a whole number up to 2^25: the single-precision root, off
+// by at most one, put right.
+__device__ __forceinline__ int isqrt_of(double k2) {
+  const int m = (int)k2;
+  int q = (int)__builtin_amdgcn_sqrtf((float)m);
+  q += (q + 1) * (q + 1) <= m ? 1 : 0;
+  return q * q > m ? q - 1 : q;
 }
 
 // WHICH = 0: spectrum (sp, sz);  WHICH = 1: fluxes (flzm, flem)
@@ -2262,6 +2285,7 @@ __global__ void __launch_bounds__(kDiagT) shell_bin_k(DiagArgs d, int nbl) {
   const double fac = (c == 0 || c == n / 2) ? (WHICH ? 1.0 : 0.5)   // diagnostics.f90:29-30
                                             : (WHICH ? 2.0 : 1.0);  // :89-90
   const size_t cq = (size_t)c * d.kyp;
+  const bool unit = ph.dkx == 1.0 && ph.dky == 1.0;  // k2 a whole number
   int blo, bhi;
   column_shells(ph, rc, c, blo, bhi);
   if (bhi - blo + 1 > nbl) bhi = blo + nbl - 1;  // never: nbl is the maximum
@@ -2303,8 +2327,7 @@ __global__ void __launch_bounds__(kDiagT) shell_bin_k(DiagArgs d, int nbl) {
         const int p = fft_of(r, rc, n);
         const double fky = (double)kyi_of(p, n) * ph.dky;
         const double k2 = fkxs + fky * fky;
-        const double k = sqrt(k2);
-        const int ib = (int)(ph.dkx == 1.0 ? k : k / ph.dkx) + 1;  // diagnostics.f90:34
+        const int ib = unit ? isqrt_of(k2) + 1 : (int)(sqrt(k2) / ph.dkx) + 1;  // :34
         if (ib < nbin && ib >= blo && ib <= bhi) {
           key = ib;
           const double ka = kalpha(ph, k2);
