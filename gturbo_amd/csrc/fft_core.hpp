@@ -663,4 +663,155 @@ __device__ __forceinline__ void fft_dit2(double2* a, double2* buf, int t,
   }
 }
 
+// ---------------------------------------------------------------------------
+// 4096-point lines over 256 threads, sixteen elements each (thread j holds
+// x[j + 256 r]): three radix-16 passes (strides 256, 16, 1) and so two
+// exchanges through LDS instead of three, the second inside a wave; in place
+// as fft_dif and fft_dit, element e at lpad(e).
+//   dif16: natural order in; thread j, register r holds
+//          X[(j >> 4) + 16 (j & 15) + 256 r].
+//   dit16: that order in, natural order out.
+// Twiddles: W^k and W^4k of the two twiddled passes, held (products of at
+// most three factors).
+// ---------------------------------------------------------------------------
+constexpr int kLine16 = 4096 + 4096 / 16;  // double2 in LDS
+// a * exp(S*2*pi*i*M/16)
+template <int S, int M>
+__device__ __forceinline__ double2 w16(double2 a) {
+  constexpr int m = M & 15;
+  if constexpr (m % 2 == 0) return w8<S, m / 2>(a);
+  else {
+    constexpr double C = 0.92387953251128675613, D = 0.38268343236508977173;
+    constexpr double c = (m == 1 || m == 15)   ? C
+                         : (m == 7 || m == 9)  ? -C
+                         : (m == 3 || m == 13) ? D
+                                               : -D;
+    constexpr double s0 = (m == 1 || m == 7)    ? D
+                          : (m == 9 || m == 15) ? -D
+                          : (m == 3 || m == 5)  ? C
+                                                : -C;
+    constexpr double s = S > 0 ? s0 : -s0;
+    return make_double2(fma(a.x, c, -a.y * s), fma(a.x, s, a.y * c));
+  }
+}
+// Radix-16 as 4 x 4 (n = 4 n1 + n2, k = k1 + 4 k2), natural-order output.
+template <int S>
+__device__ __forceinline__ void dft16(double2* a) {
+#pragma unroll
+  for (int n = 0; n < 4; ++n) dft4<S>(a[n], a[n + 4], a[n + 8], a[n + 12]);
+  // a[n2 + 4 k1]
+  a[5] = w16<S, 1>(a[5]);
+  a[9] = w16<S, 2>(a[9]);
+  a[13] = w16<S, 3>(a[13]);
+  a[6] = w16<S, 2>(a[6]);
+  a[10] = w16<S, 4>(a[10]);
+  a[14] = w16<S, 6>(a[14]);
+  a[7] = w16<S, 3>(a[7]);
+  a[11] = w16<S, 6>(a[11]);
+  a[15] = w16<S, 9>(a[15]);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) dft4<S>(a[4 * k], a[4 * k + 1], a[4 * k + 2], a[4 * k + 3]);
+  // a[4 k1 + k2] holds X[k1 + 4 k2]: transpose
+  double2 y[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) y[(i >> 2) + 4 * (i & 3)] = a[i];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) a[i] = y[i];
+}
+// t[r] *= W^(k r) (conjugated for S > 0) from W^k and W^4k.
+template <int S>
+__device__ __forceinline__ void apply_tw16(double2* t, double2 w1, double2 w4) {
+  auto ap = [](double2& x, double2 w) { x = S < 0 ? cmul(x, w) : cmulc(x, w); };
+  ap(t[1], w1);
+  ap(t[4], w4);
+  ap(t[5], cmul(w1, w4));
+  const double2 w2 = cmul(w1, w1);
+  ap(t[2], w2);
+  ap(t[6], cmul(w2, w4));
+  const double2 w3 = cmul(w1, w2);
+  ap(t[3], w3);
+  ap(t[7], cmul(w3, w4));
+  const double2 w8v = cmul(w4, w4);
+  ap(t[8], w8v);
+  ap(t[9], cmul(w1, w8v));
+  ap(t[10], cmul(w2, w8v));
+  ap(t[11], cmul(w3, w8v));
+  const double2 w12 = cmul(w4, w8v);
+  ap(t[12], w12);
+  ap(t[13], cmul(w1, w12));
+  ap(t[14], cmul(w2, w12));
+  ap(t[15], cmul(w3, w12));
+}
+struct Tw16 {
+  double2 a1, a4, b1, b4;
+};
+__device__ __forceinline__ Tw16 tw16(const double2* __restrict__ tw, int j) {
+  return {tw[j], tw[4 * j], tw[16 * (j & 15)], tw[64 * (j & 15)]};
+}
+__device__ __forceinline__ Tw16 opaque16(Tw16 w) {
+  asm volatile("" : "+v"(w.a1.x), "+v"(w.a1.y), "+v"(w.a4.x), "+v"(w.a4.y), "+v"(w.b1.x),
+               "+v"(w.b1.y), "+v"(w.b4.x), "+v"(w.b4.y));
+  return w;
+}
+// bar: as fft_dif_t
+template <int S>
+__device__ __forceinline__ void dif16(double2* a, double2* buf, int j, const Tw16& wh, bool bar) {
+  asm volatile("" : "+v"(j));
+  const Tw16 w = opaque16(wh);
+  dft16<S>(a);
+  apply_tw16<S>(a, w.a1, w.a4);
+  if (bar) __syncthreads();
+  {
+    double2* p = buf + lpad(j);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) p[272 * r] = a[r];
+  }
+  __syncthreads();
+  {
+    double2* p = buf + (j >> 4) * 272 + (j & 15);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) a[r] = p[17 * r];
+    dft16<S>(a);
+    apply_tw16<S>(a, w.b1, w.b4);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) p[17 * r] = a[r];
+  }
+  wave_sync();
+  {
+    const double2* p = buf + 17 * j;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) a[r] = p[r];
+    dft16<S>(a);
+  }
+}
+template <int S>
+__device__ __forceinline__ void dit16(double2* a, double2* buf, int j, const Tw16& wh) {
+  asm volatile("" : "+v"(j));
+  const Tw16 w = opaque16(wh);
+  dft16<S>(a);
+  {
+    double2* p = buf + 17 * j;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) p[r] = a[r];
+  }
+  wave_sync();
+  {
+    double2* p = buf + (j >> 4) * 272 + (j & 15);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) a[r] = p[17 * r];
+    apply_tw16<S>(a, w.b1, w.b4);
+    dft16<S>(a);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) p[17 * r] = a[r];
+  }
+  __syncthreads();
+  {
+    const double2* p = buf + lpad(j);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) a[r] = p[272 * r];
+    apply_tw16<S>(a, w.a1, w.a4);
+    dft16<S>(a);
+  }
+}
+
 }  // namespace gt

@@ -1065,6 +1065,94 @@ __global__ void __launch_bounds__((1 << LOGN) / kE, 4)
                                                threadIdx.x, lds, a.tw);
 }
 
+// N = 4096 on the 2/3 rectangle: the row pair with sixteen elements a thread
+// (pair_body's steps).  A row pair's transforms move a third less through LDS
+// and form fewer twiddles; two workgroups of four waves share a CU as two of
+// eight did, each lane with twice the loads in flight.  x pass 128 -> 123.5
+// us, RK4 step 1130 -> 1105, RK2 549 -> 540 (its memory side alone, without
+// transforms, 96 us, the rest with cached lines 104).  On the full rectangle
+// the loads of sixteen live positions spill (205 -> 221 us), and the 8192-point
+// rows gain 1% (718 -> 712): both keep eight.
+
+// Positions j + 256 r the rectangle can keep (below 3N/8): not r = 6..9.
+__device__ __forceinline__ constexpr bool live16(int r) { return r < 6 || r > 9; }
+// As build_two / split_store, from the row-pair blocks of y1 and to y2.
+__device__ __forceinline__ void build16(double2* z, int j, const double2* __restrict__ y,
+                                        unsigned off, int kxm) {
+  constexpr int N = 4096;
+  double2 x0[16], x1[16];
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const int p = j + 256 * r, k = r < 8 ? p : N - p;
+    x0[r] = x1[r] = make_double2(0.0, 0.0);
+    if (live16(r) && k <= kxm) {
+      const double2* q = y + off + y1_off(0, k, 0);
+      x0[r] = q[0];
+      x1[r] = q[1];
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    if ((r == 0 || r == 8) && j == 0) z[r] = make_double2(x0[r].x, x1[r].x);
+    else if (r < 8) z[r] = make_double2(x0[r].x - x1[r].y, x0[r].y + x1[r].x);
+    else z[r] = make_double2(x0[r].x + x1[r].y, x1[r].x - x0[r].y);
+  }
+}
+__device__ __forceinline__ void split16(const double2* w, double2* buf, int j,
+                                        double2* __restrict__ y, unsigned off_a, unsigned off_b,
+                                        int kxm) {
+  double2* pj = buf + lpad(j);
+#pragma unroll
+  for (int r = 0; r < 16; ++r)
+    if (live16(r)) pj[272 * r] = w[r];
+  __syncthreads();
+  const double2* pm = buf + lpad(256 - j);
+#pragma unroll
+  for (int r = 0; r <= 8; ++r) {
+    const int k = j + 256 * r;
+    if (live16(r) && k <= kxm && k <= 2048) {
+      const double2 W = w[r];
+      const double2 Wc = r == 0 ? (j == 0 ? buf : pm + 272 * 15)[0] : pm[272 * (15 - r)];
+      y[off_a + koff<12, 2>(k)] = make_double2(0.5 * (W.x + Wc.x), 0.5 * (W.y - Wc.y));
+      y[off_b + koff<12, 2>(k)] = make_double2(0.5 * (W.y + Wc.y), -0.5 * (W.x - Wc.x));
+    }
+  }
+  __syncthreads();
+}
+template <int LOGN>
+__global__ void __launch_bounds__(256, 2) r_pass_pair16(PassArgs a) {
+  static_assert(LOGN == 12, "row pairs of 4096 points");
+  __shared__ double2 buf[kLine16];
+  const int j = threadIdx.x;
+  const int y0 = 2 * xcd_remap(blockIdx.x, gridDim.x);
+  const int kxm = a.rc.kx;
+  const unsigned fstride = (unsigned)a.ntiles * 4096 * 2;
+  const unsigned r0 = yrow_off(y0, a.ntiles, 2), r1 = r0 + 2;
+  const unsigned cols = (unsigned)y1_cols(a.rc.kc());
+  const unsigned fs1 = 4096 * cols;
+  const unsigned i0 = y1_off(y0, 0, cols);
+  const Tw16 w = tw16(a.tw, j);
+  double2 z[16], qq[16];
+  build16(z, j, a.y1, i0, kxm);
+  dif16<+1>(z, buf, j, w, false);
+#pragma unroll
+  for (int r = 0; r < 16; ++r) qq[r] = z[r];
+  build16(z, j, a.y1, 2 * fs1 + i0, kxm);
+  dif16<+1>(z, buf, j, w, true);
+#pragma unroll
+  for (int r = 0; r < 16; ++r) z[r] = make_double2(qq[r].x * z[r].x, qq[r].y * z[r].y);
+  dit16<-1>(z, buf, j, w);
+  __syncthreads();
+  split16(z, buf, j, a.y2, fstride + r0, fstride + r1, kxm);
+  build16(z, j, a.y1, fs1 + i0, kxm);
+  dif16<+1>(z, buf, j, w, false);
+#pragma unroll
+  for (int r = 0; r < 16; ++r) z[r] = make_double2(qq[r].x * z[r].x, qq[r].y * z[r].y);
+  dit16<-1>(z, buf, j, w);
+  __syncthreads();
+  split16(z, buf, j, a.y2, r0, r1, kxm);
+}
+
 // ---------------------------------------------------------------------------
 // 2D transforms of a physical field in the reference layout (real rows of
 // N+2 doubles; src/fft_dir.f90, src/fft_inv.f90) to and from a spectrum in
@@ -1771,6 +1859,8 @@ hipError_t r_pass_launch(const PassArgs& a, hipStream_t s) {
     if (rect_tr(a.rc, 1 << L)) {
       if constexpr (L == 13)
         r_pass_row<L><<<dim3(1 << L), dim3(T / 2), 0, s>>>(a);
+      else if constexpr (L == 12)
+        r_pass_pair16<L><<<dim3((1 << L) / 2), dim3(T / 2), 0, s>>>(a);
       else
         r_pass_pair<L, 1><<<dim3((1 << L) / 2), dim3(T), 0, s>>>(a);
     } else {

@@ -291,3 +291,38 @@ def test_in_place_2048_transforms_reproduce_the_dft(s):
         for j in range(T):
             buf[runs[p](j)] = _bfly(buf[runs[p](j)] * tw[p](j), s)
     assert np.abs(buf - ref).max() < 1e-9 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("s", [+1, -1])
+def test_radix16_4096_transforms_reproduce_the_dft(s):
+    """dif16 (strides 256, 16, 1 over 256 threads of sixteen elements) leaves
+    X[(j >> 4) + 16 (j & 15) + 256 r] in thread j, register r; dit16 takes
+    that order back; the second exchange stays inside a wave's 1024 elements,
+    at the padded offsets the kernel uses."""
+    n, T, r16 = 4096, 256, np.arange(16)
+    rng = np.random.default_rng(16)
+    x = rng.standard_normal(n) + 1j * rng.standard_normal(n)
+    ref = np.fft.ifft(x) * n if s > 0 else np.fft.fft(x)
+    runs = [lambda j: j + 256 * r16, lambda j: (j >> 4) * 256 + (j & 15) + 16 * r16,
+            lambda j: 16 * j + r16]
+    offs = [272 * r16, 17 * r16, r16]
+    base = [lpad, lambda j: (j >> 4) * 272 + (j & 15), lambda j: 17 * j]
+    tw = [lambda j: _ip_tw(j * r16, n, s), lambda j: _ip_tw(16 * (j & 15) * r16, n, s)]
+    for p, run in enumerate(runs):
+        for j in range(T):
+            assert np.array_equal(lpad(run(j)), base[p](j) + offs[p])
+            assert p == 0 or np.all(run(j) // 1024 == j // 64)
+    buf = x.copy()
+    for p in (0, 1):
+        for j in range(T):
+            buf[runs[p](j)] = _bfly(buf[runs[p](j)], s) * tw[p](j)
+    order = np.array([(j >> 4) + 16 * (j & 15) + 256 * r16 for j in range(T)])
+    out = np.array([_bfly(buf[runs[2](j)], s) for j in range(T)])
+    assert np.abs(out - ref[order]).max() < 1e-9 * np.abs(ref).max()
+    buf = np.zeros(n, complex)
+    for j in range(T):
+        buf[runs[2](j)] = _bfly(x[order[j]], s)
+    for p in (1, 0):
+        for j in range(T):
+            buf[runs[p](j)] = _bfly(buf[runs[p](j)] * tw[p](j), s)
+    assert np.abs(buf - ref).max() < 1e-9 * np.abs(ref).max()
