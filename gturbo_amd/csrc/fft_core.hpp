@@ -281,11 +281,9 @@ __device__ __forceinline__ void fft_reg(double2* a, double2* buf, int j,
 // W^k per radix-8 pass after the first and one per butterfly of a trailing
 // radix-2/4 pass, the same for every transform the thread runs, so a kernel
 // loads them once, beside its data, and stages no table.  Same operations
-// and roundings as fft_reg with SCHED 0.  A line of N <= 512 (at most 64
-// threads, N/8 dividing the wave) lies inside one wave: its transposes then
-// need no workgroup barrier, and its threads may call alone.  Longer lines:
-// every thread of the workgroup calls; waves with act = false only meet the
-// barriers.
+// and roundings as fft_reg with SCHED 0.  For lines inside one wave (N <=
+// 512: at most 64 threads, N/8 dividing the wave): the transposes need no
+// workgroup barrier, and a line's threads may call alone.
 // ---------------------------------------------------------------------------
 template <int LOGN>
 struct HeldTw {
@@ -310,68 +308,58 @@ __device__ __forceinline__ HeldTw<LOGN> held_tw(const double2* __restrict__ tw, 
 }
 template <int LOGN>
 constexpr bool line_in_wave() { return Line<LOGN>::TPL <= 64; }
-template <int LOGN>
-__device__ __forceinline__ void line_sync() {
-  if constexpr (line_in_wave<LOGN>()) wave_sync();
-  else __syncthreads();
-}
 template <int LOGN, int S, int R, int NS, bool LAST>
-__device__ __forceinline__ void held_pass(double2* a, double2* buf, int j, const double2* w,
-                                          bool act) {
+__device__ __forceinline__ void held_pass(double2* a, double2* buf, int j, const double2* w) {
   constexpr int N = 1 << LOGN;
   constexpr int TPL = N / kE;
   constexpr int NB = kE / R;
-  if (act) {
 #pragma unroll
-    for (int b = 0; b < NB; ++b) {
-      const int jj = j + TPL * b;
-      double2 t[R];
+  for (int b = 0; b < NB; ++b) {
+    const int jj = j + TPL * b;
+    double2 t[R];
 #pragma unroll
-      for (int r = 0; r < R; ++r) t[r] = a[b + NB * r];
-      if constexpr (NS > 1) apply_tw<R, S>(t, w[b]);
-      dft<R, S>(t);
-      if constexpr (LAST) {
+    for (int r = 0; r < R; ++r) t[r] = a[b + NB * r];
+    if constexpr (NS > 1) apply_tw<R, S>(t, w[b]);
+    dft<R, S>(t);
+    if constexpr (LAST) {
 #pragma unroll
-        for (int r = 0; r < R; ++r) a[b + NB * r] = t[r];
-      } else {
-        double2* p = buf + lpad((jj / NS) * NS * R + jj % NS);
+      for (int r = 0; r < R; ++r) a[b + NB * r] = t[r];
+    } else {
+      double2* p = buf + lpad((jj / NS) * NS * R + jj % NS);
 #pragma unroll
-        for (int r = 0; r < R; ++r) p[lpad_off(r * NS)] = t[r];
-      }
+      for (int r = 0; r < R; ++r) p[lpad_off(r * NS)] = t[r];
     }
   }
   if constexpr (!LAST) {
-    line_sync<LOGN>();
-    if (act) {
-      const double2* p = buf + lpad(j);
+    wave_sync();
+    const double2* p = buf + lpad(j);
 #pragma unroll
-      for (int r = 0; r < kE; ++r) a[r] = p[lpad_off(TPL * r)];
-    }
-    line_sync<LOGN>();
+    for (int r = 0; r < kE; ++r) a[r] = p[lpad_off(TPL * r)];
+    wave_sync();
   }
 }
 template <int LOGN, int S>
 __device__ __forceinline__ void fft_held(double2* a, double2* buf, int j,
-                                         const HeldTw<LOGN>& h, bool act = true) {
+                                         const HeldTw<LOGN>& h) {
   using L = Line<LOGN>;
+  static_assert(line_in_wave<LOGN>(), "a line inside a wave");
   constexpr int P8 = L::NPASS8;
   constexpr bool T = L::RLAST > 1;
-  held_pass<LOGN, S, 8, 1, P8 == 1 && !T>(a, buf, j, h.w, act);
-  if constexpr (P8 >= 2) held_pass<LOGN, S, 8, 8, P8 == 2 && !T>(a, buf, j, h.w, act);
-  if constexpr (P8 >= 3) held_pass<LOGN, S, 8, 64, P8 == 3 && !T>(a, buf, j, h.w + 1, act);
-  if constexpr (P8 >= 4) held_pass<LOGN, S, 8, 512, P8 == 4 && !T>(a, buf, j, h.w + 2, act);
+  held_pass<LOGN, S, 8, 1, P8 == 1 && !T>(a, buf, j, h.w);
+  if constexpr (P8 >= 2) held_pass<LOGN, S, 8, 8, P8 == 2 && !T>(a, buf, j, h.w);
+  if constexpr (P8 >= 3) held_pass<LOGN, S, 8, 64, P8 == 3 && !T>(a, buf, j, h.w + 1);
   if constexpr (T)
-    held_pass<LOGN, S, L::RLAST, (1 << (3 * P8)), true>(a, buf, j, h.w + P8 - 1, act);
+    held_pass<LOGN, S, L::RLAST, (1 << (3 * P8)), true>(a, buf, j, h.w + P8 - 1);
 }
 
 // ---------------------------------------------------------------------------
-// In-place radix-8 transforms of a 2048- or 4096-point line over T = N/8
-// threads (whole waves, thread j = lane + 64 wave).  The first pass combines
+// In-place radix-8 transforms of a 1024-, 2048- or 4096-point line over T =
+// N/8 threads (whole waves, thread j = lane + 64 wave).  The first pass combines
 // the elements j + T r that thread j holds; its outputs go to LDS, and each
 // later pass reads, transforms and writes back one run of the line that
 // belongs to a single wave (strides T/8 and T/64: runs inside the wave's 512
 // elements; the last pass eight consecutive ones, as one radix-8 butterfly at
-// 4096 and two radix-4 ones at 2048).  Only the first exchange crosses waves,
+// 4096, two radix-4 ones at 2048, four radix-2 ones at 1024).  Only the first exchange crosses waves,
 // so a transform needs one workgroup barrier plus one before its first write
 // (when LDS may still be read by another wave), instead of two per pass.
 //   fft_dif: natural order in, out of order: thread j, register r holds
@@ -393,11 +381,13 @@ __device__ __forceinline__ int ip_pad(int e) { return e + (e >> 3); }
 // Output index of fft_dif in thread j, register r.
 template <int LOGN>
 __host__ __device__ __forceinline__ int ip_row(int j, int r) {
-  static_assert(LOGN == 11 || LOGN == 12, "in-place lines of 2048 or 4096 points");
+  static_assert(LOGN >= 10 && LOGN <= 12, "in-place lines of 1024 to 4096 points");
   if constexpr (LOGN == 12)
     return 64 * (j & 7) + 8 * ((j >> 3) & 7) + (j >> 6) + 512 * r;
-  else
+  else if constexpr (LOGN == 11)
     return (j >> 5) + 8 * ((j >> 2) & 7) + 128 * (j & 3) + 64 * (r >> 2) + 512 * (r & 3);
+  else
+    return (j >> 4) + 8 * ((j >> 1) & 7) + 256 * (j & 1) + 64 * (r >> 1) + 512 * (r & 1);
 }
 
 // t[r] *= W^(k r) (conjugated for S > 0), from w1 = W^k; each power is
@@ -470,29 +460,37 @@ template <int LOGN, int S>
 __device__ __forceinline__ void ip_last(double2* a) {
   if constexpr (LOGN == 12) {
     dft<8, S>(a);
-  } else {
+  } else if constexpr (LOGN == 11) {
     dft<4, S>(a);
     dft<4, S>(a + 4);
+  } else {
+#pragma unroll
+    for (int r = 0; r < 8; r += 2) dft<2, S>(a + r);
   }
 }
 
 // bar: barrier before the first LDS write (another wave may still read
 // LDS); a uniform run-time flag, so that a loop holds one copy of the code.
+// act = false (uniform in a wave): the wave only meets the barriers.
 template <int LOGN, int S, class TW>
 __device__ __forceinline__ void fft_dif_t(double2* a, double2* buf, int j, const TW& T,
-                                          bool bar) {
+                                          bool bar, bool act = true) {
   using R = IpRun<LOGN>;
-  double2 wn = T.template at<1>();  // pass 1: W^(j r)
-  dft<8, S>(a);
-  apply_tw8<S>(a, wn);
-  wn = T.template at<2>();  // pass 2, in flight across the barrier
+  double2 wn;
+  if (act) {
+    wn = T.template at<1>();  // pass 1: W^(j r)
+    dft<8, S>(a);
+    apply_tw8<S>(a, wn);
+    wn = T.template at<2>();  // pass 2, in flight across the barrier
+  }
   if (bar) __syncthreads();
-  {
+  if (act) {
     double2* p = buf + ip_pad(j);
 #pragma unroll
     for (int r = 0; r < 8; ++r) p[R::off1(r)] = a[r];
   }
   __syncthreads();
+  if (!act) return;
   {  // pass 2
     double2* p = buf + R::base2(j);
 #pragma unroll
@@ -536,10 +534,10 @@ __device__ __forceinline__ IpTw opaque(IpTw w) {
 }
 template <int LOGN, int S>
 __device__ __forceinline__ void fft_dif_held(double2* a, double2* buf, int j, const IpTw& w,
-                                             bool bar) {
+                                             bool bar, bool act = true) {
   asm volatile("" : "+v"(j));
   const IpTw lw = opaque(w);
-  fft_dif_t<LOGN, S>(a, buf, j, TwHeld{lw}, bar);
+  fft_dif_t<LOGN, S>(a, buf, j, TwHeld{lw}, bar, act);
 }
 
 // Input as fft_dif leaves it; the thread's own LDS run is free to write
@@ -548,40 +546,46 @@ __device__ __forceinline__ void fft_dif_held(double2* a, double2* buf, int j, co
 // BAR: start with a workgroup barrier (another wave may still read this
 // wave's run of LDS, e.g. after a preceding fft_dit).
 template <int LOGN, int S, bool BAR, class TW>
-__device__ __forceinline__ void fft_dit_t(double2* a, double2* buf, int j, const TW& T) {
+__device__ __forceinline__ void fft_dit_t(double2* a, double2* buf, int j, const TW& T,
+                                          bool act = true) {
   using R = IpRun<LOGN>;
-  double2 wn = T.template at<3>();
-  ip_last<LOGN, S>(a);  // pass 4, stride 1
+  double2 wn;
+  if (act) {
+    wn = T.template at<3>();
+    ip_last<LOGN, S>(a);  // pass 4, stride 1
+  }
   if constexpr (BAR) __syncthreads();
-  {
-    double2* p = buf + 9 * j;
+  if (act) {
+    {
+      double2* p = buf + 9 * j;
 #pragma unroll
-    for (int r = 0; r < 8; ++r) p[r] = a[r];
-  }
-  wave_sync();
-  {  // pass 3
-    double2* p = buf + R::base3(j);
+      for (int r = 0; r < 8; ++r) p[r] = a[r];
+    }
+    wave_sync();
+    {  // pass 3
+      double2* p = buf + R::base3(j);
 #pragma unroll
-    for (int r = 0; r < 8; ++r) a[r] = p[R::off3(r)];
-    apply_tw8<S>(a, wn);
-    wn = T.template at<2>();
-    dft<8, S>(a);
+      for (int r = 0; r < 8; ++r) a[r] = p[R::off3(r)];
+      apply_tw8<S>(a, wn);
+      wn = T.template at<2>();
+      dft<8, S>(a);
 #pragma unroll
-    for (int r = 0; r < 8; ++r) p[R::off3(r)] = a[r];
-  }
-  wave_sync();
-  {  // pass 2
-    double2* p = buf + R::base2(j);
+      for (int r = 0; r < 8; ++r) p[R::off3(r)] = a[r];
+    }
+    wave_sync();
+    {  // pass 2
+      double2* p = buf + R::base2(j);
 #pragma unroll
-    for (int r = 0; r < 8; ++r) a[r] = p[R::off2(r)];
-    apply_tw8<S>(a, wn);
-    wn = T.template at<1>();
-    dft<8, S>(a);
+      for (int r = 0; r < 8; ++r) a[r] = p[R::off2(r)];
+      apply_tw8<S>(a, wn);
+      wn = T.template at<1>();
+      dft<8, S>(a);
 #pragma unroll
-    for (int r = 0; r < 8; ++r) p[R::off2(r)] = a[r];
+      for (int r = 0; r < 8; ++r) p[R::off2(r)] = a[r];
+    }
   }
   __syncthreads();
-  {  // pass 1: natural order out
+  if (act) {  // pass 1: natural order out
     const double2* p = buf + ip_pad(j);
 #pragma unroll
     for (int r = 0; r < 8; ++r) a[r] = p[R::off1(r)];
@@ -596,10 +600,11 @@ __device__ __forceinline__ void fft_dit(double2* a, double2* buf, int j,
   fft_dit_t<LOGN, S, BAR>(a, buf, j, TwFromTable<LOGN, TS>{tw, j});
 }
 template <int LOGN, int S, bool BAR = false>
-__device__ __forceinline__ void fft_dit_held(double2* a, double2* buf, int j, const IpTw& w) {
+__device__ __forceinline__ void fft_dit_held(double2* a, double2* buf, int j, const IpTw& w,
+                                             bool act = true) {
   asm volatile("" : "+v"(j));
   const IpTw lw = opaque(w);
-  fft_dit_t<LOGN, S, BAR>(a, buf, j, TwHeld{lw});
+  fft_dit_t<LOGN, S, BAR>(a, buf, j, TwHeld{lw}, act);
 }
 
 // 8192-point lines over 1024 threads (thread t holds x[t + 1024 r]): a

@@ -219,6 +219,12 @@ struct EnsForce {
 // workgroup sizes (threads; a workgroup holds T*8/N lines of a size).
 constexpr int kEnsMinLogn = 7, kEnsMaxLogn = 11;
 __host__ __device__ constexpr int ens_lines(int t, int logn) { return t * 8 >> logn; }
+// Columns of a tile of the y buffers for T threads per y-pass workgroup: the
+// workgroup's lines, whose threads interleave over a tile's row; from N = 1024
+// (lines of whole waves, each reading one column) two, as in the single runs.
+__host__ __device__ constexpr int ens_tile(int t, int logn) {
+  return logn >= 10 ? 2 : ens_lines(t, logn);
+}
 
 // 2D transform of a physical field in the reference layout to (dir < 0, with
 // /NY/NX) or from (dir > 0) a compact spectrum; y: io_size double2 of scratch.

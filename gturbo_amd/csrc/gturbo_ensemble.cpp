@@ -88,9 +88,15 @@ void drop_graph(gt_ens* e) {
   e->graph = nullptr;
 }
 
+// Work items (groups of columns) of a member's y pass, and the tiles its y
+// buffers need so that every column of the last group has a place.
+int ygroups_of(const EnsMember& m, int ty) {
+  const int lines = gt::ens_lines(ty, m.logn);
+  return (m.rc.kc() + lines - 1) / lines;
+}
 int ntiles_of(const EnsMember& m, int ty) {
-  const int bt = gt::ens_lines(ty, m.logn);
-  return (m.rc.kc() + bt - 1) / bt;
+  const int bt = gt::ens_tile(ty, m.logn);
+  return (ygroups_of(m, ty) * gt::ens_lines(ty, m.logn) + bt - 1) / bt;
 }
 
 // Pass arguments and work lists of a schedule; uploaded, graph dropped.
@@ -128,7 +134,7 @@ int apply(gt_ens* e, const int32_t* cfg) {
   }
   for (int m : order) {
     const EnsMember& mb = e->mem[m];
-    const int nt = d[m].ntiles;
+    const int nt = ygroups_of(mb, cfg[0]);
     for (int t = 0; t < nt; ++t) yi.push_back(((uint32_t)m << 16) | (uint32_t)t);
     const int rows = gt::ens_lines(cfg[1], mb.logn) * (d[m].xvar ? 2 : 1);
     const int ng = (1 << mb.logn) / rows;
@@ -376,7 +382,7 @@ int gt_ens_create(int32_t nmem, const int32_t* n, const double* params, gt_ens**
     ENS_HIP(hipMemsetAsync(mb.z, 0, sizeof(double2) * nc, e->stream));
     ENS_HIP(hipMemsetAsync(mb.znew, 0, sizeof(double2) * nc, e->stream));
     for (int ty : {256, 512}) {
-      const int bt = gt::ens_lines(ty, mb.logn);
+      const int bt = gt::ens_tile(ty, mb.logn);
       mb.ycap = std::max(mb.ycap, (size_t)ntiles_of(mb, ty) * bt * c->n);
     }
     ENS_HIP(hipMalloc(&mb.y1, sizeof(double2) * mb.ycap * 3));

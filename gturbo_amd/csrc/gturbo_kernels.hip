@@ -133,6 +133,13 @@ __device__ __forceinline__ void line_map(int tid, int& line, int& j) {
   j = (c / NL) * G + tid % G;
 }
 
+// The same for lines of whole waves (in-place transforms): line = wave mod NL.
+template <int NL>
+__device__ __forceinline__ void wave_line_map(int tid, int& line, int& j) {
+  line = (tid >> 6) % NL;
+  j = ((tid >> 6) / NL) * 64 + (tid & 63);
+}
+
 // ---------------------------------------------------------------------------
 // y pass
 // ---------------------------------------------------------------------------
@@ -257,24 +264,25 @@ __device__ __forceinline__ double2 field_of(int f, double2 s, double fkx, double
 // double2 of LDS of an in-place line (8192: two 4096-point problems).
 template <int LOGN>
 __host__ __device__ constexpr int ip_lds() {
-  return LOGN == 13 ? 2 * kIpLine : LOGN == 11 ? ip_line<11>() : kIpLine;
+  return LOGN == 13 ? 2 * kIpLine : ip_line<LOGN>();
 }
 
-// One tile of BT kx-columns; lds holds BT padded lines.  SCHED is the radix
+// A group of BT kx-columns; lds holds BT padded lines, the y buffers tiles of
+// LB columns.  SCHED is the radix
 // order of the transforms (fft_reg).
-// IP (N >= 2048): the y buffers hold the rows of a column in the order the
+// IP (N >= 1024): the y buffers hold the rows of a column in the order the
 // in-place transforms use (slot j + N/8 r holds physical row ip_row(j, r));
 // the forward transforms (fft_dit) take the loaded slots and return natural
 // ky order, the inverse ones (fft_dif) return slot order for the stores.
-// Each line is whole waves: of two lines, line b = wave mod 2, j = 64 (wave
-// / 2) + lane.  The x pass transforms rows, whichever rows a slot pair holds.
-template <int LOGN, int MODE, int AK, int TR, int BT, int SCHED, bool IP = false>
+// Each line is whole waves (wave_line_map).  The x pass transforms rows,
+// whichever rows a slot pair holds.
+template <int LOGN, int MODE, int AK, int TR, int BT, int SCHED, bool IP = false, int LB = BT>
 __device__ __forceinline__ void c_body(const PassArgs& a, int tile, int tid,
                                        double2* lds, const double2* tw) {
   constexpr int N = 1 << LOGN, TPL = N / kE;
   constexpr int LINE = IP ? ip_lds<LOGN>() : Line<LOGN>::PADDED;
-  static_assert(!IP || (LOGN == 13 && BT == 1) || ((LOGN == 11 || LOGN == 12) && BT <= 2),
-                "in-place y pass: up to two lines, or one 8192-point line");
+  static_assert(!IP || (LOGN == 13 && BT == 1) || (LOGN >= 10 && LOGN <= 12),
+                "in-place y pass: lines of 1024 to 4096 points, or one of 8192");
   constexpr bool FWD = MODE != C_START;
   constexpr bool INV = MODE == C_START || MODE == C_RK4_1 || MODE == C_RK4_2 ||
                        MODE == C_RK4_3 || MODE == C_RK2_1 || MODE == C_RK4_4S ||
@@ -286,15 +294,8 @@ __device__ __forceinline__ void c_body(const PassArgs& a, int tile, int tid,
   constexpr bool ONCE = LOGN >= 12;
   constexpr bool NT2 = LOGN == 12;   // Y2 reads likewise, at 4096 only
   int b, j;
-  if constexpr (IP && BT == 2) {
-    b = (tid >> 6) & 1;
-    j = ((tid >> 7) << 6) | (tid & 63);
-  } else if constexpr (IP) {
-    b = 0;
-    j = tid;
-  } else {
-    line_map<TPL, BT>(tid, b, j);
-  }
+  if constexpr (IP) wave_line_map<BT>(tid, b, j);
+  else line_map<TPL, BT>(tid, b, j);
   const int c = tile * BT + b;
   const Rect rc = a.rc;
   const bool colok = c <= rc.kx;
@@ -315,19 +316,19 @@ __device__ __forceinline__ void c_body(const PassArgs& a, int tile, int tid,
 
   if constexpr (FWD) {
     double2 A[kE];
-    const unsigned colo = ycol_off(c, BT);
+    const unsigned colo = ycol_off(c, LB);
     const double2* srcA = a.y2;
 #pragma unroll
-    for (int r = 0; r < kE; ++r) z[r] = ld_state<NT2>(&srcA[yrow_off(j + TPL * r, a.ntiles, BT) + colo]);
+    for (int r = 0; r < kE; ++r) z[r] = ld_state<NT2>(&srcA[yrow_off(j + TPL * r, a.ntiles, LB) + colo]);
     if constexpr (HELD) fft_dit_held<LOGN, -1>(z, buf, j, ytw);
     else if constexpr (IP && LOOP) fft_dit<-1, true, 1, LOGN>(z, buf, j, tw);
     else if constexpr (IP) fft_dit2<-1, false>(z, buf, j, tw);
     else fft_reg<LOGN, -1, SCHED>(z, buf, j, tw);
 #pragma unroll
     for (int r = 0; r < kE; ++r) A[r] = live_r<TR>(r) ? z[r] : make_double2(0.0, 0.0);
-    const double2* srcB = a.y2 + (size_t)a.ntiles * N * BT;
+    const double2* srcB = a.y2 + (size_t)a.ntiles * N * LB;
 #pragma unroll
-    for (int r = 0; r < kE; ++r) z[r] = ld_state<NT2>(&srcB[yrow_off(j + TPL * r, a.ntiles, BT) + colo]);
+    for (int r = 0; r < kE; ++r) z[r] = ld_state<NT2>(&srcB[yrow_off(j + TPL * r, a.ntiles, LB) + colo]);
     if constexpr (HELD) fft_dit_held<LOGN, -1, true>(z, buf, j, ytw);
     else if constexpr (IP && LOOP) fft_dit<-1, true, 1, LOGN>(z, buf, j, tw);
     else if constexpr (IP) fft_dit2<-1, true>(z, buf, j, tw);
@@ -423,10 +424,10 @@ __device__ __forceinline__ void c_body(const PassArgs& a, int tile, int tid,
 #pragma unroll
         for (int r = 0; r < kE; ++r) dst[y1_off(j + TPL * r, c, cols)] = z[r];
       } else {
-        double2* dst = a.y1 + (size_t)f * a.ntiles * N * BT;
-        const unsigned colo = ycol_off(c, BT);
+        double2* dst = a.y1 + (size_t)f * a.ntiles * N * LB;
+        const unsigned colo = ycol_off(c, LB);
 #pragma unroll
-        for (int r = 0; r < kE; ++r) dst[yrow_off(j + TPL * r, a.ntiles, BT) + colo] = z[r];
+        for (int r = 0; r < kE; ++r) dst[yrow_off(j + TPL * r, a.ntiles, LB) + colo] = z[r];
       }
     }
   }
@@ -474,19 +475,35 @@ __global__ void __launch_bounds__(bt_of(LOGN) * (1 << LOGN) / kE, 4) c_pass(Pass
 // 15.4 -> 7.5, 1024^2 29.4 -> 20.7; x pass 5.0 -> 4.1, 5.8 -> 4.8, 7.8 ->
 // 6.5, 16.6 -> 15.6.  Up to 512^2 the rest is a kernel's own start and end
 // (about 2 us), two memory round trips and two transforms; at 1024^2 the
-// 41 MB a stage moves take half of it (12.7 us with the transforms skipped).
+// 41 MB a stage moves take half of it (12.7 us with the transforms skipped),
+// and in-place transforms, whose few barriers and held twiddles (100 instead
+// of 160 VGPRs) replace Stockham ones there, the next part: y stage 18.3 ->
+// 16.4 us, boundary 20.9 -> 18.1, untruncated 27 -> 24, x pass 15.6 -> 15.3.
 // ---------------------------------------------------------------------------
 
 // Columns per workgroup of the y pass: a wave per field where a line is
-// shorter than a wave; 512: one (7.3 us; two 8.2); 1024: two (18.5 us; one,
-// whose workgroups each touch half of every line, 20.8).
+// shorter than a wave; 512: one (7.3 us; two 8.2); 1024: two (16.4 us; one,
+// whose workgroups each touch half of every line, 19.2).
 __host__ __device__ constexpr int fp_cols(int logn) { return logn < 9 ? 512 >> logn : logn == 9 ? 1 : 2; }
 constexpr int kFpForce = 32;  // forced modes of a column staged in LDS
+
+// Twiddles and LDS line of a field: Stockham inside a wave, in place beyond.
+template <int LOGN>
+__host__ __device__ constexpr int fp_line() {
+  return line_in_wave<LOGN>() ? Line<LOGN>::PADDED : ip_lds<LOGN < 10 ? 10 : LOGN>();
+}
+template <int LOGN>
+__device__ __forceinline__ auto fp_tw(const double2* __restrict__ tw, int j) {
+  if constexpr (line_in_wave<LOGN>()) return held_tw<LOGN>(tw, j);
+  else return ip_tw<LOGN>(tw, j);
+}
 
 template <int LOGN, int MODE, int AK, int TR>
 __global__ void __launch_bounds__(fp_cols(LOGN) * 3 * (1 << LOGN) / kE) f_pass(PassArgs a) {
   constexpr int N = 1 << LOGN, TPL = N / kE, BT = bt_of(LOGN), CW = fp_cols(LOGN);
-  constexpr int LINE = Line<LOGN>::PADDED, GT = CW * TPL;  // threads per field
+  // 1024: in-place transforms, the y buffers in their row order (see c_body)
+  constexpr bool IP = !line_in_wave<LOGN>();
+  constexpr int LINE = fp_line<LOGN>(), GT = CW * TPL;  // threads per field
   constexpr bool FWD = MODE != C_START;
   constexpr bool INV = MODE != C_NLT && MODE != C_RK4_4 && MODE != C_RK2_2;
   constexpr bool BOUND = MODE == C_RK4_4S || MODE == C_RK2_2S;
@@ -527,7 +544,7 @@ __global__ void __launch_bounds__(fp_cols(LOGN) * 3 * (1 << LOGN) / kE) f_pass(P
                                                    : make_double2(0.0, 0.0);
     }
   }
-  const HeldTw<LOGN> tw = held_tw<LOGN>(a.tw, j);
+  const auto tw = fp_tw<LOGN>(a.tw, j);
   // positions this thread updates: r = NOWN f + i of the live ones
   int pos[NOWN];
   bool own[NOWN];
@@ -552,9 +569,7 @@ __global__ void __launch_bounds__(fp_cols(LOGN) * 3 * (1 << LOGN) / kE) f_pass(P
       ka[r] = live_r<TR>(r) && colok && row >= 0 && f > 0 ? a.ka[cbase + (unsigned)row] : 1.0;
     }
   };
-  // 1024: after the forward transforms (768 threads leave 168 VGPRs)
-  constexpr bool KA_LATE = LOGN >= 10 && FWD;
-  if constexpr (INV && AK == 2 && !KA_LATE) load_ka();
+  if constexpr (INV && AK == 2) load_ka();
 
   if constexpr (FWD) {
     // The column's forcing entries (forcing.f90:25-31), formed by the third
@@ -580,13 +595,17 @@ __global__ void __launch_bounds__(fp_cols(LOGN) * 3 * (1 << LOGN) / kE) f_pass(P
         }
       }
     }
-    if (!line_in_wave<LOGN>() || f < 2) fft_held<LOGN, -1>(z, buf, j, tw, f < 2);
+    if constexpr (IP) {
+      fft_dit_held<LOGN, -1>(z, buf, j, tw, f < 2);
+      __syncthreads();  // every wave's reads done
+    } else if (f < 2) {
+      fft_held<LOGN, -1>(z, buf, j, tw);
+    }
     if (f < 2) {
 #pragma unroll
       for (int r = 0; r < kE; ++r)
         if (live_r<TR>(r)) (buf + lpad(j))[lpad_off(TPL * r)] = z[r];
     }
-    if constexpr (INV && AK == 2 && KA_LATE) load_ka();
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < NOWN; ++i) {
@@ -656,7 +675,8 @@ __global__ void __launch_bounds__(fp_cols(LOGN) * 3 * (1 << LOGN) / kE) f_pass(P
         z[r] = field_of(f, z[r], fkx, fky, AK == 1 ? fkxs + fky * fky : ka[r]);
       }
     }
-    fft_held<LOGN, +1>(z, buf, j, tw);
+    if constexpr (IP) fft_dif_held<LOGN, +1>(z, buf, j, tw, false);
+    else fft_held<LOGN, +1>(z, buf, j, tw);
     if (colok) {
       double2* dst = a.y1 + (size_t)f * a.ntiles * N * BT;
 #pragma unroll
@@ -771,9 +791,11 @@ template <int LOGN, int TR, int BT, int NL, int SCHED>
 __device__ __forceinline__ void r_body(const PassArgs& a, int g, int tid,
                                        double2* lds, const double2* tw) {
   constexpr int N = 1 << LOGN, TPL = N / kE;
-  constexpr int LINE = Line<LOGN>::PADDED;
+  constexpr bool IP = LOGN == 10;  // in-place transforms, as f_pass and fx_pass
+  constexpr int LINE = IP ? ip_line<10>() : Line<LOGN>::PADDED;
   int pl, j;
-  line_map<TPL, NL>(tid, pl, j);
+  if constexpr (IP) wave_line_map<NL>(tid, pl, j);
+  else line_map<TPL, NL>(tid, pl, j);
   const int yrow = g * NL + pl;
   double2* buf = lds + pl * LINE;
   const int kxm = a.rc.kx;
@@ -783,15 +805,24 @@ __device__ __forceinline__ void r_body(const PassArgs& a, int g, int tid,
 
   double2 z[kE];
   double qv[kE];
+  auto inv = [&](bool bar) {  // bar: another wave may still read LDS
+    if constexpr (IP) fft_dif<+1, 1, LOGN>(z, buf, j, tw, bar);
+    else fft_reg<LOGN, +1, SCHED>(z, buf, j, tw);
+  };
   build_two<LOGN, TR, BT>(z, j, a.y1, offQ, offV, kxm);
-  fft_reg<LOGN, +1, SCHED>(z, buf, j, tw);
+  inv(false);  // an item before ended with a barrier
 #pragma unroll
   for (int r = 0; r < kE; ++r) qv[r] = z[r].x * z[r].y;  // produ.f90:16
   build_two<LOGN, TR, BT>(z, j, a.y1, offQ, offU, kxm);
-  fft_reg<LOGN, +1, SCHED>(z, buf, j, tw);
+  inv(true);
 #pragma unroll
   for (int r = 0; r < kE; ++r) z[r] = make_double2(z[r].x * z[r].y, qv[r]);  // produ.f90:15
-  fft_reg<LOGN, -1, SCHED>(z, buf, j, tw);
+  if constexpr (IP) {
+    fft_dit<-1, false, 1, LOGN>(z, buf, j, tw);
+    __syncthreads();  // every wave's reads done
+  } else {
+    fft_reg<LOGN, -1, SCHED>(z, buf, j, tw);
+  }
   split_store<LOGN, TR, BT>(z, buf, j, a.y2, offQ, offQ + fstride, kxm);
 }
 
@@ -799,14 +830,15 @@ __device__ __forceinline__ void r_body(const PassArgs& a, int g, int tid,
 // q+iu, each on its own N/8 threads; the operations are r_body's.  q v
 // crosses to the q u threads through LDS, these run the forward transform of
 // q u + i q v, and both store their half of the split spectrum.
-// Rows per workgroup: 512: two (6.4 us; one 7.2); 1024: one (15.9; two 19.1).
+// Rows per workgroup: 512: two (6.4 us; one 7.2); 1024: one (15.3; two 15.5).
 __host__ __device__ constexpr int fx_rows(int logn) {
   return logn == 10 ? 1 : logn == 9 ? 2 : logn == 4 ? 16 : 512 >> logn;
 }
 template <int LOGN, int TR>
 __global__ void __launch_bounds__(2 * fx_rows(LOGN) * (1 << LOGN) / kE) fx_pass(PassArgs a) {
   constexpr int N = 1 << LOGN, TPL = N / kE, BT = bt_of(LOGN), RW = fx_rows(LOGN);
-  constexpr int LINE = Line<LOGN>::PADDED, GT = RW * TPL;
+  constexpr bool IP = !line_in_wave<LOGN>();  // 1024: in-place transforms
+  constexpr int LINE = fp_line<LOGN>(), GT = RW * TPL;
   __shared__ double2 lds[2 * RW * LINE];
   int f = threadIdx.x / GT;  // 0: q+iv, 1: q+iu
   if constexpr (GT % 64 == 0) f = __builtin_amdgcn_readfirstlane(f);
@@ -819,9 +851,14 @@ __global__ void __launch_bounds__(2 * fx_rows(LOGN) * (1 << LOGN) / kE) fx_pass(
   const unsigned off = yrow_off(yrow, a.ntiles, BT);
   double2 z[kE], x0[kE], x1[kE];
   load_two<LOGN, TR, BT>(x0, x1, j, a.y1, off, off + (f ? fstride : 2 * fstride), kxm);
-  const HeldTw<LOGN> tw = held_tw<LOGN>(a.tw, j);
+  const auto tw = fp_tw<LOGN>(a.tw, j);
   pack_two<LOGN>(z, j, x0, x1);
-  fft_held<LOGN, +1>(z, buf, j, tw);
+  if constexpr (IP) {
+    fft_dif_held<LOGN, +1>(z, buf, j, tw, false);
+    __syncthreads();  // the other wave's reads of the q+iv line
+  } else {
+    fft_held<LOGN, +1>(z, buf, j, tw);
+  }
   double* qv = reinterpret_cast<double*>(row);  // the q+iv line, free again
   if (f == 0) {
 #pragma unroll
@@ -833,7 +870,12 @@ __global__ void __launch_bounds__(2 * fx_rows(LOGN) * (1 << LOGN) / kE) fx_pass(
     for (int r = 0; r < kE; ++r)
       z[r] = make_double2(z[r].x * z[r].y, qv[j + TPL * r]);  // produ.f90:15
   }
-  if (!line_in_wave<LOGN>() || f == 1) fft_held<LOGN, -1>(z, buf, j, tw, f == 1);
+  if constexpr (IP) {
+    fft_dit_held<LOGN, -1>(z, buf, j, tw, f == 1);
+    __syncthreads();
+  } else if (f == 1) {
+    fft_held<LOGN, -1>(z, buf, j, tw);
+  }
   double2* wl = row + LINE;
   if (f == 1) {
 #pragma unroll
@@ -864,19 +906,15 @@ template <int LOGN, int TR, int BT, int NL, int SCHED, bool TWPF = false>
 __device__ __forceinline__ void pair_body(const PassArgs& a, int g, int tid,
                                           double2* lds, const double2* tw) {
   constexpr int N = 1 << LOGN, TPL = N / kE;
-  // 2048- and 4096-point lines use the in-place transforms (lines of whole
+  // 1024- to 4096-point lines use the in-place transforms (lines of whole
   // waves): the inverse ones leave x out of order, which the pointwise
   // products do not mind, and the forward ones restore natural order for
   // split_store.
-  constexpr bool IP = (LOGN == 11 && NL <= 2) || (LOGN == 12 && NL == 1);
-  constexpr int LINE = IP ? ip_lds<LOGN>() : Line<LOGN>::PADDED;
+  constexpr bool IP = LOGN >= 10 && LOGN <= 12;
+  constexpr int LINE = LOGN >= 10 ? ip_lds<LOGN < 10 ? 10 : LOGN>() : Line<LOGN>::PADDED;
   int pl, j;
-  if constexpr (IP && NL == 2) {
-    pl = (tid >> 6) & 1;
-    j = ((tid >> 7) << 6) | (tid & 63);
-  } else {
-    line_map<TPL, NL>(tid, pl, j);
-  }
+  if constexpr (IP) wave_line_map<NL>(tid, pl, j);
+  else line_map<TPL, NL>(tid, pl, j);
   double2* buf = lds + pl * LINE;
   const int y0 = 2 * (g * NL + pl);
   const int kxm = a.rc.kx;
@@ -1255,8 +1293,7 @@ template <int LOGN>
 __device__ __forceinline__ void io_map(int tid, int& b, int& j) {
   constexpr int TPL = (1 << LOGN) / kE;
   if constexpr (LOGN == 12) {
-    b = (tid >> 6) & 1;
-    j = ((tid >> 7) << 6) | (tid & 63);
+    wave_line_map<2>(tid, b, j);
   } else {
     b = tid / TPL;
     j = tid % TPL;
@@ -1981,7 +2018,8 @@ __device__ __forceinline__ const double2* ens_stage_tw(double2* twl, const PassA
 template <int T, int MODE, int SCHED, int L>
 __device__ __forceinline__ void ens_c_one(const PassArgs& a, int tile, int tid,
                                           double2* lds, const double2* tw) {
-  c_body<L, MODE, 2, 1, ens_lines(T, L), SCHED, L == 11>(a, tile, tid, lds, tw);
+  c_body<L, MODE, 2, 1, ens_lines(T, L), SCHED, L >= 10, ens_tile(T, L)>(a, tile, tid,
+                                                                               lds, tw);
 }
 
 template <int T, int MODE, int SCHED>
@@ -2014,7 +2052,7 @@ __global__ void __launch_bounds__(T, 4)
 template <int TX, int TY, int SCHED, int L>
 __device__ __forceinline__ void ens_r_one(const PassArgs& a, int g, int tid, double2* lds,
                                           const double2* tw) {
-  constexpr int NL = ens_lines(TX, L), BT = ens_lines(TY, L);
+  constexpr int NL = ens_lines(TX, L), BT = ens_tile(TY, L);
   if (a.xvar) pair_body<L, 1, BT, NL, SCHED>(a, g, tid, lds, tw);
   else r_body<L, 1, BT, NL, SCHED>(a, g, tid, lds, tw);
 }

@@ -293,6 +293,53 @@ def test_in_place_2048_transforms_reproduce_the_dft(s):
     assert np.abs(buf - ref).max() < 1e-9 * np.abs(ref).max()
 
 
+def _ip_row10(j, r):
+    """Output index of the 1024-point fft_dif in thread j, register r."""
+    return (j >> 4) + 8 * ((j >> 1) & 7) + 256 * (j & 1) + 64 * (r >> 1) + 512 * (r & 1)
+
+
+@pytest.mark.parametrize("s", [+1, -1])
+def test_in_place_1024_transforms_reproduce_the_dft(s):
+    """The same at 1024 points: strides 128, 16, 2, then four radix-2
+    butterflies a thread."""
+    n, T, S2, S3 = 1024, 128, 16, 2
+    pad = lambda e: e + (e >> 3)  # noqa: E731
+    rng = np.random.default_rng(12)
+    x = rng.standard_normal(n) + 1j * rng.standard_normal(n)
+    ref = np.fft.ifft(x) * n if s > 0 else np.fft.fft(x)
+    r8 = np.arange(8)
+    runs = {1: lambda j: j + T * r8, 2: lambda j: (j // S2) * T + (j & (S2 - 1)) + S2 * r8,
+            3: lambda j: (j // S3) * S2 + (j & (S3 - 1)) + S3 * r8, 4: lambda j: 8 * j + r8}
+    offs = {1: T * r8 + T * r8 // 8, 2: S2 * r8 + S2 * r8 // 8, 3: S3 * r8 + S3 * r8 // 8, 4: r8}
+    tw = {1: lambda j: _ip_tw(j * r8, n, s), 2: lambda j: _ip_tw(8 * (j & (S2 - 1)) * r8, n, s),
+          3: lambda j: _ip_tw(64 * (j & (S3 - 1)) * r8, n, s)}
+    for p, run in runs.items():
+        for j in range(T):
+            e = run(j)
+            assert np.array_equal(pad(e), pad(e[0]) + offs[p])
+            assert p == 1 or np.all(e // 512 == j // 64)
+
+    def last(v):
+        return np.concatenate([_bfly(v[2 * b:2 * b + 2], s) for b in range(4)])
+
+    buf = x.copy()
+    for p in (1, 2, 3):
+        for j in range(T):
+            buf[runs[p](j)] = _bfly(buf[runs[p](j)], s) * tw[p](j)
+    order = np.array([[_ip_row10(j, r) for r in range(8)] for j in range(T)])
+    out = np.array([last(buf[runs[4](j)]) for j in range(T)])
+    assert np.abs(out - ref[order]).max() < 1e-9 * np.abs(ref).max()
+    assert np.array_equal(np.sort(order.ravel()), np.arange(n))
+
+    buf = np.zeros(n, complex)
+    for j in range(T):
+        buf[runs[4](j)] = last(x[order[j]])
+    for p in (3, 2, 1):
+        for j in range(T):
+            buf[runs[p](j)] = _bfly(buf[runs[p](j)] * tw[p](j), s)
+    assert np.abs(buf - ref).max() < 1e-9 * np.abs(ref).max()
+
+
 @pytest.mark.parametrize("s", [+1, -1])
 def test_radix16_4096_transforms_reproduce_the_dft(s):
     """dif16 (strides 256, 16, 1 over 256 threads of sixteen elements) leaves
