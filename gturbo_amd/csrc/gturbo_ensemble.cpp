@@ -413,9 +413,16 @@ int gt_ens_create(int32_t nmem, const int32_t* n, const double* params, gt_ens**
   }
   ENS_HIP(hipEventCreate(&e->t0));
   ENS_HIP(hipEventCreate(&e->t1));
-  // default schedule: 512-thread workgroups, one workgroup per work item,
-  // radix 8 first, row pairs in the x pass from N = 2048, 10 steps a graph
-  int32_t cfg[GT_ENS_NCFG] = {512, 512, 0, 0, 1 << 11, 10};
+  // default schedule: x passes of 512 threads, one workgroup per work item,
+  // radix 8 first, row pairs in the x pass from N = 2048, 10 steps a graph.
+  // y passes of 256 threads while every line is shorter than that (one
+  // workgroup's barriers and LDS hold up fewer lines; step with 512 -> 256
+  // threads: 8 x 128^2 165 -> 136 us, 24 x 512^2 533 -> 451, 8 x 1024^2 763 ->
+  // 682), of 512 with a member of 2048 (its two columns a workgroup share
+  // their cache lines: 2 x 2048^2 693 us, 766 with 256).
+  int lmax = 0;
+  for (const EnsMember& mb : e->mem) lmax = std::max(lmax, mb.logn);
+  int32_t cfg[GT_ENS_NCFG] = {lmax <= 10 ? 256 : 512, 512, 0, 0, 1 << 11, 10};
   ENS_CHK(apply(e, cfg));
   ENS_HIP(hipStreamSynchronize(e->stream));
   *out = e;

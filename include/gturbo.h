@@ -213,7 +213,9 @@ typedef struct gt_ens gt_ens;
  * [2] waves per SIMD of the persistent grid (1, 2 or 4; 0 = one workgroup
  *     per work item), [3] radix order of the transforms (0 = radix 8 first,
  *     1 = the radix-2/4 pass first), [4] bit L set: members with N = 2^L
- *     use the row-pair x pass, [5] RK steps per captured graph (1-256). */
+ *     use the row-pair x pass, [5] RK steps per captured graph (1-256).
+ * A new ensemble has {256, 512, 0, 0, 1 << 11, 10}, with 512 first where a
+ * member has N >= 2048. */
 #define GT_ENS_NCFG 6
 
 /* nmem members; n[m] = N of member m; params holds nmem rows of the 17

@@ -6,6 +6,7 @@ import pytest
 
 from gturbo_amd import ic
 from gturbo_amd.adjoint import Adjoint
+from gturbo_amd.ensemble import SPECTRAL, Ensemble, solo_run
 from gturbo_amd.params import InitialSpectrum
 from gturbo_amd.solver import Solver
 from helpers import params_for, random_spectral
@@ -167,3 +168,23 @@ def test_forced_steps_large(oracle_mod, n, alpv, truncate):
     steps with the fused boundary between them (1e-12 as above)."""
     p = params_for(n, alpv=alpv, truncate=truncate, ring=(10.0, 20.0))
     assert _steps(oracle_mod, p, 2) < 1e-12
+
+
+@pytest.mark.parametrize("sizes", [(128, 512, 1024), (256,), (256, 2048)])
+def test_default_ensemble_schedule_matches_solo_runs(sizes):
+    """The schedule an ensemble starts with (256-thread y passes up to N =
+    1024, 512 with a member of 2048) keeps every member's arithmetic."""
+    ps = [params_for(n, alpv=(0.5, 1.0, 2.0)[m % 3], ring=(n / 8 - 1.0, n / 8 + 1.0))
+          for m, n in enumerate(sizes)]
+    fields = [ic.physical_field(p, InitialSpectrum(seed=70 + p.n, p=4.0, k0=p.n / 16.0,
+                                                   energy=0.5)) for p in ps]
+    ens = Ensemble(ps, seeds=[5 + m for m in range(len(ps))])
+    for m, w in enumerate(fields):
+        ens.set_field(m, w)
+    ens.run(11)
+    ens.synchronize()
+    for m, (p, w) in enumerate(zip(ps, fields)):
+        z, seed = solo_run(p, w, 5 + m, 11)
+        assert ens.get_seed(m) == seed
+        assert np.array_equal(ens.get_field(m, SPECTRAL), z), p.n
+    ens.close()
