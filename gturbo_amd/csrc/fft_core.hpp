@@ -19,6 +19,7 @@
 // latency, not by FP64 arithmetic, and one load per butterfly measured
 // faster than three (and three faster than seven).
 #pragma once
+#include <type_traits>
 #include <hip/hip_runtime.h>
 
 namespace gt {
@@ -407,12 +408,39 @@ __device__ __forceinline__ void apply_tw8(double2* t, double2 w1) {
   ap(t[7], cmul(w3, w4));
 }
 
+// The same from W^k and W^4k, both of the table.  A twiddle's error is the
+// same in every transform, so it adds up over a run where roundings of data
+// do not: 1024 points, whose three passes form seven powers each where the
+// Stockham passes formed them in two, take W^4k from the table too (1024^2
+// SQG, 100 steps: difference to the oracle 1.1e-15; from W^k alone 1.6e-15,
+// Stockham 2.4e-15; exact twiddles 0.8e-15), for 3 us of a 1024^2 RK4 step:
+// 130 -> 133, Stockham 139.
+struct W14 {
+  double2 w1, w4;
+};
+template <int S>
+__device__ __forceinline__ void apply_tw8(double2* t, const W14& w) {
+  auto ap = [](double2& x, double2 v) { x = S < 0 ? cmul(x, v) : cmulc(x, v); };
+  ap(t[1], w.w1);
+  ap(t[4], w.w4);
+  ap(t[5], cmul(w.w1, w.w4));
+  const double2 w2 = cmul(w.w1, w.w1);
+  ap(t[2], w2);
+  ap(t[6], cmul(w2, w.w4));
+  const double2 w3 = cmul(w.w1, w2);
+  ap(t[3], w3);
+  ap(t[7], cmul(w3, w.w4));
+}
+template <int LOGN>
+using ip_w = std::conditional_t<LOGN == 10, W14, double2>;
+
 // Twiddles of the three twiddled passes of an in-place transform in thread
 // j: W^j (stride T), W^(8 (j % (T/8))), W^(64 (j % (T/64))), from the table
 // read at stride TS.  The same for every transform a thread runs, so a kernel
 // running several may load them once.
+template <int LOGN>
 struct IpTw {
-  double2 w1, w2, w3;
+  ip_w<LOGN> w1, w2, w3;
 };
 // Twiddle sources for fft_dif / fft_dit: at<P>() gives the twiddle of pass P
 // (1-3), called where the transform first needs it in flight.
@@ -422,20 +450,22 @@ struct TwFromTable {
   const double2* __restrict__ tw;
   int j;
   template <int P>
-  __device__ __forceinline__ double2 at() const {
-    return P == 1 ? tw[TS * j] : P == 2 ? tw[TS * 8 * (j & (T / 8 - 1))]
-                                        : tw[TS * 64 * (j & (T / 64 - 1))];
+  __device__ __forceinline__ ip_w<LOGN> at() const {
+    const int k = P == 1 ? j : P == 2 ? 8 * (j & (T / 8 - 1)) : 64 * (j & (T / 64 - 1));
+    if constexpr (LOGN == 10) return {tw[TS * k], tw[TS * 4 * k]};
+    else return tw[TS * k];
   }
 };
 template <int LOGN, int TS = 1>
-__device__ __forceinline__ IpTw ip_tw(const double2* __restrict__ tw, int j) {
+__device__ __forceinline__ IpTw<LOGN> ip_tw(const double2* __restrict__ tw, int j) {
   const TwFromTable<LOGN, TS> t{tw, j};
   return {t.template at<1>(), t.template at<2>(), t.template at<3>()};
 }
+template <int LOGN>
 struct TwHeld {
-  const IpTw& w;
+  const IpTw<LOGN>& w;
   template <int P>
-  __device__ __forceinline__ double2 at() const {
+  __device__ __forceinline__ ip_w<LOGN> at() const {
     return P == 1 ? w.w1 : P == 2 ? w.w2 : w.w3;
   }
 };
@@ -476,7 +506,7 @@ template <int LOGN, int S, class TW>
 __device__ __forceinline__ void fft_dif_t(double2* a, double2* buf, int j, const TW& T,
                                           bool bar, bool act = true) {
   using R = IpRun<LOGN>;
-  double2 wn;
+  ip_w<LOGN> wn;
   if (act) {
     wn = T.template at<1>();  // pass 1: W^(j r)
     dft<8, S>(a);
@@ -527,17 +557,25 @@ __device__ __forceinline__ void fft_dif(double2* a, double2* buf, int j,
 }
 // Held twiddles enter each transform opaque, so that the compiler keeps
 // forming the powers inside it rather than holding them across transforms.
-__device__ __forceinline__ IpTw opaque(IpTw w) {
-  asm volatile("" : "+v"(w.w1.x), "+v"(w.w1.y), "+v"(w.w2.x), "+v"(w.w2.y), "+v"(w.w3.x),
-               "+v"(w.w3.y));
+__device__ __forceinline__ void hide(double2& w) { asm volatile("" : "+v"(w.x), "+v"(w.y)); }
+__device__ __forceinline__ void hide(W14& w) {
+  hide(w.w1);
+  hide(w.w4);
+}
+template <int LOGN>
+__device__ __forceinline__ IpTw<LOGN> opaque(IpTw<LOGN> w) {
+  hide(w.w1);
+  hide(w.w2);
+  hide(w.w3);
   return w;
 }
 template <int LOGN, int S>
-__device__ __forceinline__ void fft_dif_held(double2* a, double2* buf, int j, const IpTw& w,
+__device__ __forceinline__ void fft_dif_held(double2* a, double2* buf, int j,
+                                             const IpTw<LOGN>& w,
                                              bool bar, bool act = true) {
   asm volatile("" : "+v"(j));
-  const IpTw lw = opaque(w);
-  fft_dif_t<LOGN, S>(a, buf, j, TwHeld{lw}, bar, act);
+  const IpTw<LOGN> lw = opaque(w);
+  fft_dif_t<LOGN, S>(a, buf, j, TwHeld<LOGN>{lw}, bar, act);
 }
 
 // Input as fft_dif leaves it; the thread's own LDS run is free to write
@@ -549,7 +587,7 @@ template <int LOGN, int S, bool BAR, class TW>
 __device__ __forceinline__ void fft_dit_t(double2* a, double2* buf, int j, const TW& T,
                                           bool act = true) {
   using R = IpRun<LOGN>;
-  double2 wn;
+  ip_w<LOGN> wn;
   if (act) {
     wn = T.template at<3>();
     ip_last<LOGN, S>(a);  // pass 4, stride 1
@@ -600,11 +638,12 @@ __device__ __forceinline__ void fft_dit(double2* a, double2* buf, int j,
   fft_dit_t<LOGN, S, BAR>(a, buf, j, TwFromTable<LOGN, TS>{tw, j});
 }
 template <int LOGN, int S, bool BAR = false>
-__device__ __forceinline__ void fft_dit_held(double2* a, double2* buf, int j, const IpTw& w,
+__device__ __forceinline__ void fft_dit_held(double2* a, double2* buf, int j,
+                                             const IpTw<LOGN>& w,
                                              bool act = true) {
   asm volatile("" : "+v"(j));
-  const IpTw lw = opaque(w);
-  fft_dit_t<LOGN, S, BAR>(a, buf, j, TwHeld{lw}, act);
+  const IpTw<LOGN> lw = opaque(w);
+  fft_dit_t<LOGN, S, BAR>(a, buf, j, TwHeld<LOGN>{lw}, act);
 }
 
 // 8192-point lines over 1024 threads (thread t holds x[t + 1024 r]): a

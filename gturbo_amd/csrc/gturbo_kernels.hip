@@ -311,7 +311,7 @@ __device__ __forceinline__ void c_body(const PassArgs& a, int tile, int tid,
   constexpr bool LOOP = AK == 2;
   // in-place transforms up to 4096 points: their three twiddles, loaded once.
   constexpr bool HELD = IP && LOGN <= 12 && !LOOP;
-  IpTw ytw{};
+  IpTw<LOGN> ytw{};
   if constexpr (HELD) ytw = ip_tw<LOGN>(tw, j);
 
   if constexpr (FWD) {
@@ -930,7 +930,7 @@ __device__ __forceinline__ void pair_body(const PassArgs& a, int g, int tid,
   constexpr bool IP2 = LOGN == 13 && NL == 1 && TWPF;  // 8192: radix 2, then two 4096s
   // the three twiddles every transform of the thread uses, loaded once (from
   // memory; a table in LDS is read where it is needed)
-  IpTw w{};
+  IpTw<LOGN> w{};
   if constexpr (IP && TWPF) w = ip_tw<LOGN>(tw, j);
   // bar: another wave may still read LDS (ignored by the Stockham transforms,
   // which synchronise on every transpose)
@@ -1200,7 +1200,7 @@ __global__ void __launch_bounds__(256, 2) r_pass_pair16(PassArgs a) {
 // only the kept columns travel.  A y transform in place on the reference
 // layout touches 16 or 32 bytes of each row's line.  Both directions with
 // trunc between them, 4096^2: 505 us with transforms in the reference layout
-// and gather/scatter, IO4096_US us; 8192^2: 3040 and IO8192_US us.
+// and gather/scatter, 242 us; 8192^2: 3040 and 1163 us.
 // ---------------------------------------------------------------------------
 
 // Physical row held by slot s of a column: the in-place transforms' order at
