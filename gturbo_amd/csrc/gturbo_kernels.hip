@@ -478,7 +478,7 @@ __global__ void __launch_bounds__(bt_of(LOGN) * (1 << LOGN) / kE, 4) c_pass(Pass
 // 41 MB a stage moves take half of it (12.7 us with the transforms skipped),
 // and in-place transforms, whose few barriers and held twiddles (100 instead
 // of 160 VGPRs) replace Stockham ones there, the next part: y stage 18.3 ->
-// 16.4 us, boundary 20.9 -> 18.1, untruncated 27 -> 24, x pass 15.6 -> 15.3.
+// 17.0 us, boundary 20.9 -> 18.5, untruncated 27 -> 24.4, x pass 15.6 -> 15.9.
 // ---------------------------------------------------------------------------
 
 // Columns per workgroup of the y pass: a wave per field where a line is
