@@ -417,9 +417,9 @@ int gt_ens_create(int32_t nmem, const int32_t* n, const double* params, gt_ens**
   // radix 8 first, row pairs in the x pass from N = 2048, 10 steps a graph.
   // y passes of 256 threads while every line is shorter than that (one
   // workgroup's barriers and LDS hold up fewer lines; step with 512 -> 256
-  // threads: 8 x 128^2 165 -> 136 us, 24 x 512^2 533 -> 451, 8 x 1024^2 763 ->
-  // 682), of 512 with a member of 2048 (its two columns a workgroup share
-  // their cache lines: 2 x 2048^2 693 us, 766 with 256).
+  // threads: 8 x 128^2 165 -> 136 us, 24 x 512^2 533 -> 455, 8 x 1024^2 775 ->
+  // 699), of 512 with a member of 2048 (its two columns a workgroup share
+  // their cache lines: 2 x 2048^2 692 us, 768 with 256).
   int lmax = 0;
   for (const EnsMember& mb : e->mem) lmax = std::max(lmax, mb.logn);
   int32_t cfg[GT_ENS_NCFG] = {lmax <= 10 ? 256 : 512, 512, 0, 0, 1 << 11, 10};

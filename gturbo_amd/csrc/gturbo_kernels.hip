@@ -8,11 +8,14 @@
 //    truncation and the RK stage update (src/rkstep.f90 stage AXPYs).  Inverse
 //    part: from the next stage input, the spectral operator |k|^-alpha
 //    (src/nlt.f90:22-36) for q, u, v and their inverse y transforms.
-//  * x pass (r_pass): one workgroup per RP y rows.  Complex-to-real x
-//    transforms of q+iv and q+iu (two real sequences per complex transform),
-//    the products q u, q v (src/produ.f90), and one real-to-complex transform
-//    of q u + i q v.  At N = 8192 a workgroup takes one row, as the 4096-point
-//    complex transform of its even and odd samples (r_pass_row).
+//  * x pass (r_pass_*): complex-to-real x transforms of q, u and v, the
+//    products q u, q v (src/produ.f90), and their real-to-complex transforms,
+//    two real rows per complex transform: q of rows y and y+1 and so on
+//    (r_pass_pair, r_pass_pair16), at N = 8192 the even and odd samples of one
+//    row (r_pass_row).
+//  * N <= 1024: f_pass and fx_pass, the same passes with the fields of a column
+//    or row side by side on their own threads; the batched passes (ens_*) run
+//    c_body and r_body of every member's size.
 //
 // Between the passes the three (resp. two) fields live in HBM in blocks of
 // kYR rows x BT columns, [field][y / kYR][tile][y % kYR][kx % BT]: the y
