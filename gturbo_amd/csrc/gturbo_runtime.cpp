@@ -316,7 +316,10 @@ int lookup(gt_ctx* c, const void* host, Mirror** m) {
   return GT_OK;
 }
 
+// Room for a compact copy on rectangle r.  Its contents are to be written: the
+// old ones count no more, also where the allocation or the writing then fails.
 int alloc_cmp(gt_ctx*, Mirror& m, const Rect& r) {
+  m.cmp_valid = m.wide = false;
   const int kyp = kyp_of(r);
   const size_t need = (size_t)r.kc() * kyp;
   if (need > m.cmp_cap) {
@@ -331,9 +334,15 @@ int alloc_cmp(gt_ctx*, Mirror& m, const Rect& r) {
   return GT_OK;
 }
 
+// Neither copy is valid after a call that failed to write one.
+static int has_data(const Mirror& m) {
+  if (m.ref_valid || m.cmp_valid) return GT_OK;
+  return fail(GT_ERR_ARG, "array %p has no valid device data", m.host);
+}
+
 int ensure_ref(gt_ctx* c, Mirror& m) {
   if (m.ref_valid) return GT_OK;
-  if (!m.cmp_valid) return fail(GT_ERR_ARG, "array %p has no valid device data", m.host);
+  CHK(has_data(m));
   Timer t(c, GT_K_OTHER);
   HIPCHK(gt::launch_scatter(c->ph, m.rect, m.kyp, m.dcmp, m.dref, c->stream));
   m.ref_valid = true;
@@ -389,6 +398,7 @@ int ensure_cmp(gt_ctx* c, Mirror& m) {
     return narrow(c, m, 0);
   }
   if (m.cmp_valid) return GT_OK;
+  CHK(has_data(m));
   Rect r = c->rtr;
   if (has_tr(c)) {
     HIPCHK(hipMemsetAsync(c->flag, 0, sizeof(int), c->stream));
@@ -503,7 +513,6 @@ int same_rect(gt_ctx* c, Mirror& a, Mirror& b) {
   for (Mirror* m : {&a, &b}) {
     if (rect_kind(c, m->rect) == 0) {
       CHK(ensure_ref(c, *m));
-      m->cmp_valid = false;
       CHK(alloc_cmp(c, *m, c->rfull));
       Timer t(c, GT_K_OTHER);
       HIPCHK(gt::launch_gather(c->ph, c->rfull, m->kyp, m->dref, m->dcmp, 0, nullptr,
@@ -897,7 +906,7 @@ int gt_unmap_data(gt_ctx* c, void* key) {
   auto it = c->present.find(key);
   if (it == c->present.end()) return fail(GT_ERR_NOT_PRESENT, "key %p not present", key);
   if (it->second.owned) return fail(GT_ERR_ARG, "key %p was not mapped", key);
-  if (!it->second.ref_valid) CHK(ensure_ref(c, it->second));
+  if (it->second.cmp_valid && !it->second.ref_valid) CHK(ensure_ref(c, it->second));
   return drop(c, key);
 }
 
@@ -956,6 +965,7 @@ int gt_copy(gt_ctx* c, void* dst, const void* src) {
   CHK(lookup(c, dst, &d));
   CHK(lookup(c, src, &s));
   if (d == s) return GT_OK;
+  CHK(has_data(*s));
   Timer t(c, GT_K_OTHER);
   if (s->cmp_valid) {
     CHK(alloc_cmp(c, *d, s->rect));
@@ -1010,8 +1020,7 @@ int gt_fft_inv(gt_ctx* c, double* z, int32_t plan) {
   if (plan != GT_PLAN_Z2D) return fail(GT_ERR_ARG, "fft_inv needs a Z2D plan (got %d)", plan);
   Mirror* m;
   CHK(lookup(c, z, &m));
-  if (!m->ref_valid && !m->cmp_valid)
-    return fail(GT_ERR_ARG, "array %p has no valid device data", m->host);
+  CHK(has_data(*m));
   if (m->ref_valid) {  // a spectrum in the reference layout, all of it
     CHK(alloc_cmp(c, *m, c->rfull));
     HIPCHK(gt::launch_gather(c->ph, m->rect, m->kyp, m->dref, m->dcmp, 0, nullptr, c->stream));
@@ -1046,6 +1055,7 @@ int gt_trunc(gt_ctx* c, double* z) {
   CHK(flush_pending(c));
   Mirror* m;
   CHK(lookup(c, z, &m));
+  CHK(has_data(*m));
   Timer t(c, GT_K_OTHER);
   if (m->cmp_valid) {
     if (m->wide) {

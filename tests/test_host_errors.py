@@ -1,0 +1,284 @@
+"""The host runtime's error paths on the CPU: the runtime's sources linked
+against a HIP whose allocations and launches are made to fail on request.
+Launches do nothing but check that every buffer they are given is allocated
+(on a GPU, one that is not would be a memory fault) and note their order."""
+import ctypes as C
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(ROOT, "gturbo_amd", "csrc")
+
+SHIM = r"""
+#include <hip/hip_runtime.h>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+#include <string>
+#include "gt_internal.hpp"
+static std::map<const char*, size_t> live;
+static std::string log_, fail_name;
+static int bad = 0, fail_in = 0;  // allocations until one fails (0: none)
+static int outside = 0;           // what a look for modes outside the rectangle finds
+static bool dies() { return fail_in > 0 && --fail_in == 0; }
+static hipError_t get(void** p, size_t n) {
+  *p = nullptr;
+  if (dies()) return hipErrorOutOfMemory;
+  *p = calloc(1, n ? n : 1);
+  live[(char*)*p] = n;
+  return hipSuccess;
+}
+static hipError_t drop(void* p) {
+  if (p && !live.erase((char*)p)) ++bad;
+  free(p);
+  return hipSuccess;
+}
+static bool ok(const void* q) {
+  const char* p = (const char*)q;
+  auto it = live.upper_bound(p);
+  const bool in = p && it != live.begin() && (--it, p < it->first + it->second);
+  bad += !in;
+  return in;
+}
+static bool may(const void* q) { return !q || ok(q); }
+static hipError_t ran(const char* name, std::initializer_list<const void*> ps) {
+  for (const void* p : ps) ok(p);
+  log_ += std::string(name) + " ";
+  if (fail_name != name) return hipSuccess;
+  fail_name.clear();
+  return hipErrorLaunchFailure;
+}
+extern "C" {
+void shim_reset() { log_.clear(); fail_name.clear(); bad = fail_in = outside = 0; }
+void shim_outside(int v) { outside = v; }
+void shim_fail_alloc(int k) { fail_in = k; }
+void shim_fail_launch(const char* n) { fail_name = n; }
+const char* shim_log() { return log_.c_str(); }
+int shim_bad() { return bad; }
+void* shim_device(int n) { void* p; return get(&p, n) == hipSuccess ? p : nullptr; }
+hipError_t hipMalloc(void** p, size_t n) { return get(p, n); }
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return get(p, n); }
+hipError_t hipFree(void* p) { return drop(p); }
+hipError_t hipHostFree(void* p) { return drop(p); }
+hipError_t hipHostGetDevicePointer(void** d, void* h, unsigned) {
+  *d = nullptr;
+  if (dies()) return hipErrorInvalidValue;
+  *d = h;
+  return hipSuccess;
+}
+hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind k) {
+  bool in = true;
+  if (k == hipMemcpyHostToDevice || k == hipMemcpyDeviceToDevice) in = ok(d) && in;
+  if (k == hipMemcpyDeviceToHost || k == hipMemcpyDeviceToDevice) in = ok(s) && in;
+  if (in) memcpy(d, s, n);
+  return hipSuccess;
+}
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind k, hipStream_t) {
+  return hipMemcpy(d, s, n, k);
+}
+hipError_t hipMemsetAsync(void* d, int v, size_t n, hipStream_t) {
+  if (ok(d)) memset(d, v, n);
+  return hipSuccess;
+}
+hipError_t hipMemGetInfo(size_t* f, size_t* t) { *f = *t = 0; return hipSuccess; }
+hipError_t hipGetDeviceCount(int* n) { *n = 1; return hipSuccess; }
+const char* hipGetErrorString(hipError_t) { return "made to fail"; }
+hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { *s = nullptr; return hipSuccess; }
+hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
+  *e = (hipEvent_t)malloc(1);
+  return hipSuccess;
+}
+hipError_t hipEventDestroy(hipEvent_t e) { free((void*)e); return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { log_ += "event "; return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventElapsedTime(float* t, hipEvent_t, hipEvent_t) { *t = 1.f; return hipSuccess; }
+int roctxRangePushA(const char*) { return 0; }
+int roctxRangePop() { return 0; }
+}
+namespace gt {
+static double scratch[6 * 4097 + 6];
+hipError_t glob_scratch(double** p, size_t* n) {
+  live[(char*)scratch] = sizeof scratch;
+  *p = scratch;
+  *n = 6 * 4097 + 6;
+  return hipSuccess;
+}
+static hipError_t y_pass(const char* name, const PassArgs& a, int mode) {
+  may(a.sst);
+  may(a.ka);
+  may(a.fcs);
+  may(a.fce);
+  may(a.fph);
+  if (mode == C_NLT) ok(a.out);
+  else if (mode != C_START) ok(a.emk);
+  if (mode == C_RK4_1 || mode == C_RK4_2 || mode == C_RK4_3 || mode == C_RK4_4 ||
+      mode == C_RK4_4S)
+    ok(a.znew);
+  if (a.ph.akind != 1) ok(a.ka);
+  if (a.fcs) { ok(a.fce); ok(a.fph); }
+  return ran(name, {a.tw, a.y1, a.y2, a.z});
+}
+hipError_t launch_c_pass(int, int m, const PassArgs& a, hipStream_t) { return y_pass("y", a, m); }
+hipError_t launch_r_pass(int, const PassArgs& a, hipStream_t) {
+  return ran("x", {a.tw, a.y1, a.y2});
+}
+hipError_t launch_io(int, const IoArgs& a, hipStream_t) {
+  log_ += a.rc.kx == a.ph.n / 2 ? "full:" : "kept:";
+  return ran("io", {a.ref, a.tw, a.y, a.cmp});
+}
+hipError_t launch_j_pass(int, int, const AdjArgs& a, hipStream_t) {
+  may(a.snext);
+  return ran("j", {a.tw, a.y1, a.y2, a.lam, a.lacc, a.emk});
+}
+hipError_t launch_jr_pass(int, const AdjArgs& a, hipStream_t) {
+  return ran("jr", {a.tw, a.y1, a.y2});
+}
+hipError_t launch_produ(int, const double* z, double* u, double* v, hipStream_t) {
+  return ran("produ", {z, u, v});
+}
+hipError_t launch_trunc_cmp(const Phys&, const Rect&, int, double2* z, hipStream_t) {
+  return ran("trunc", {z});
+}
+hipError_t launch_gather(const Phys&, const Rect&, int, const double* r, double2* c, int, int* f,
+                         hipStream_t) {
+  if (f && ok(f)) *f = outside;
+  return ran("gather", {r, c});
+}
+hipError_t launch_narrow(const Phys&, const Rect&, int, const double2* s, const Rect&, int,
+                         double2* d, int, int* f, hipStream_t) {
+  if (f && ok(f)) *f = outside;
+  return ran("narrow", {s, d});
+}
+hipError_t launch_scatter(const Phys&, const Rect&, int, const double2* c, double* r,
+                          hipStream_t) {
+  return ran("scatter", {c, r});
+}
+hipError_t launch_forcing(const Phys&, int, const ForcedMode* m, const double2* p, double,
+                          double2* z, hipStream_t) {
+  return ran("forcing", {m, p, z});
+}
+hipError_t launch_spectrum(const DiagArgs& d, int which, hipStream_t) {
+  if (which) ok(d.znl);
+  return ran("spectrum", {d.z, d.part1, d.part2, d.lohi, d.out1, d.out2});
+}
+hipError_t launch_glob(const DiagArgs& d, hipStream_t) {
+  return ran("glob", {d.z, d.gpart, d.gout});
+}
+hipError_t launch_shell_index(const Phys&, int* ib, hipStream_t) { return ran("shell", {ib}); }
+hipError_t launch_ka_table(const Phys&, const Rect&, int, double* k, hipStream_t) {
+  return ran("ka", {k});
+}
+}  // namespace gt
+"""
+
+N = 32
+
+
+@pytest.fixture(scope="module")
+def lib(tmp_path_factory):
+    d = tmp_path_factory.mktemp("host")
+    (d / "shim.cpp").write_text(SHIM)
+    srcs = [str(d / "shim.cpp")] + [os.path.join(CSRC, f"gturbo_{s}.cpp")
+                                    for s in ("runtime", "adjoint", "phases")]
+    out = str(d / "host.so")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__",
+                    "-Wno-unused-result", "-Wl,-Bsymbolic", f"-I{CSRC}",
+                    f"-I{os.path.join(ROOT, 'include')}", "-I/opt/rocm/include", *srcs, "-o", out],
+                   check=True)
+    L = C.CDLL(out)
+    L.shim_log.restype = C.c_char_p
+    L.shim_device.restype = C.c_void_p
+    return L
+
+
+class Run:
+    """A context and named arrays on that HIP; every call gives its code."""
+
+    def __init__(self, lib):
+        self.L = lib
+        lib.shim_reset()
+        p = [2 * np.pi, 2 * np.pi, 1e-9, 4.0, 0.1, 0.0, 2.0, 1e-3, 4, 1, 1, 1, 2.0 / 3.0, 1, 1.0,
+             2.0, 4.0]
+        self.h = C.c_void_p()
+        self.a = {}
+        self.out = np.zeros(2 * N)
+        assert lib.gt_create(N, (C.c_double * 17)(*p), C.byref(self.h)) == 0
+
+    def __call__(self, name, *args):
+        return getattr(self.L, "gt_" + name)(self.h, *[self.ptr(x) for x in args])
+
+    def ptr(self, x):
+        if not isinstance(x, str):
+            return x
+        if x not in self.a:
+            self.a[x] = np.zeros((N, N + 2))
+        return C.c_void_p(self.a[x].ctypes.data)
+
+    def enter(self, *names):
+        return [self("enter_data", n, C.c_int64(N * (N + 2) * 8), 1) for n in names]
+
+    def log(self):
+        return self.L.shim_log().decode().split()
+
+    def diag(self, name, *args):
+        o = self.out.ctypes.data
+        two = [C.c_void_p(o), C.c_void_p(o + 8 * N)][:1 if name == "glob" else 2]
+        return self(name, *args, *two)
+
+    def close(self):
+        self.L.gt_destroy(self.h)
+        return self.L.shim_bad()
+
+
+D2Z = 1
+
+
+@pytest.mark.parametrize("what,fails", [("fft_dir", "allocation"), ("fft_dir", "launch"),
+                                        ("copy", "allocation"), ("step4", "allocation"),
+                                        ("step4", "launch")])
+def test_failed_growth_of_a_compact_copy(lib, what, fails):
+    """A compact copy that is to be replaced by a larger one is gone when that
+    fails: what comes next reads the reference copy, or is refused where there
+    is none; the array can be given back and used again."""
+    r = Run(lib)
+    assert r.enter("z", "w", "a", "b", "c") == [0] * 5
+    assert r("trunc", "z") == 0  # z: the kept rectangle alone
+    lib.shim_outside(1)
+    assert r("step4", "w", "a", "c", "b", "b") == 0  # w: the whole half-spectrum
+    assert r("synchronize") == 0
+    if fails == "allocation":
+        lib.shim_fail_alloc(1)
+    else:
+        lib.shim_fail_launch(b"io" if what == "fft_dir" else b"y")
+    assert 0 != (r("fft_dir", "z", D2Z) if what == "fft_dir" else r("copy", "z", "w")
+                 if what == "copy" else r("step4", "w", "a", "z", "b", "c"))
+    n = len(r.log())
+    rc = r.diag("spectrum", "z")
+    if what == "fft_dir":  # its input is still there
+        assert rc == 0 and r.log()[n:] == ["gather", "gather", "spectrum"]
+        assert r("fft_dir", "z", D2Z) == 0
+    else:
+        assert rc != 0 and r.log()[n:] == [] and r("update_host", "z") != 0
+        assert r("copy", "z", "w") == 0 and r("update_host", "z") == 0
+    assert r("exit_data", "z", 0) == 0
+    assert r.close() == 0
+
+
+def test_unmapping_what_a_failed_copy_left(lib):
+    """A mapped array that holds nothing after a failed copy can be unmapped."""
+    r = Run(lib)
+    assert r.enter("w") == [0]
+    lib.shim_outside(1)
+    assert r.diag("spectrum", "w") == 0
+    nbytes = N * (N + 2) * 8
+    assert r("map_data", "z", C.c_void_p(lib.shim_device(nbytes)), C.c_int64(nbytes)) == 0
+    assert r("trunc", "z") == 0
+    lib.shim_fail_alloc(1)
+    assert r("copy", "z", "w") != 0 and r("update_host", "z") != 0
+    assert r("unmap_data", "z") == 0
+    assert r.close() == 0
