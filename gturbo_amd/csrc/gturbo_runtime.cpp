@@ -472,10 +472,15 @@ int r_pass(gt_ctx* c, const gt::PassArgs& a) {
 int ensure_diag(gt_ctx* c, const Rect& r) {
   const size_t nbin = c->n / 2;
   if (!c->dg_out) {
-    void* d = nullptr;
-    HIPCHK(hipHostMalloc(&c->dg_out, sizeof(double) * (2 * nbin + 6),
+    void *h = nullptr, *d = nullptr;
+    HIPCHK(hipHostMalloc(&h, sizeof(double) * (2 * nbin + 6),
                          hipHostMallocCoherent | hipHostMallocMapped));
-    HIPCHK(hipHostGetDevicePointer(&d, c->dg_out, 0));
+    const hipError_t e = hipHostGetDevicePointer(&d, h, 0);
+    if (e != hipSuccess) {
+      (void)hipHostFree(h);
+      return fail(GT_ERR_HIP, "diagnostics results: %s", hipGetErrorString(e));
+    }
+    c->dg_out = static_cast<double*>(h);
     c->dg_dev = static_cast<double*>(d);
   }
   const size_t need = 2 * (size_t)(r.kc() + 1) * nbin + (size_t)r.kc() * 7;

@@ -282,3 +282,15 @@ def test_unmapping_what_a_failed_copy_left(lib):
     assert r("copy", "z", "w") != 0 and r("update_host", "z") != 0
     assert r("unmap_data", "z") == 0
     assert r.close() == 0
+
+
+@pytest.mark.parametrize("k", [1, 2, 3])
+def test_failed_allocation_of_the_diagnostics(lib, k):
+    """Result buffer, its device address, partial sums: whichever fails, the
+    next diagnostic call allocates what is missing."""
+    r = Run(lib)
+    assert r.enter("z") == [0] and r("trunc", "z") == 0
+    lib.shim_fail_alloc(k)
+    assert r.diag("glob", "z") != 0
+    assert r.diag("glob", "z") == 0 and r.diag("spectrum", "z") == 0
+    assert r.close() == 0
