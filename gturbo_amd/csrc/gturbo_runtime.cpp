@@ -171,11 +171,14 @@ int upload_twiddles(gt_ctx* c) {
   return GT_OK;
 }
 
+static void drop_tables(RectTables& t) {
+  for (void* p : {(void*)t.emk, (void*)t.ka, (void*)t.modes, (void*)t.fcs, (void*)t.fce})
+    if (p) (void)hipFree(p);
+  t = RectTables{};
+}
+
 // Integrating-factor table and forced-mode table for one rectangle.
-int rect_tables(gt_ctx* c, const Rect& r, RectTables** out) {
-  RectTables& t = c->tab[rect_kind(c, r)];
-  *out = &t;
-  if (t.emk) return GT_OK;
+static int build_tables(gt_ctx* c, const Rect& r, RectTables& t) {
   t.rc = r;
   t.kyp = kyp_of(r);
   const int n = c->n, nh = c->nh;
@@ -231,6 +234,20 @@ int rect_tables(gt_ctx* c, const Rect& r, RectTables** out) {
   HIPCHK(hipMemcpy(t.fcs, fcs.data(), sizeof(int) * fcs.size(), hipMemcpyHostToDevice));
   HIPCHK(hipMalloc(&t.fce, sizeof(gt::FEntry) * fce.size()));
   HIPCHK(hipMemcpy(t.fce, fce.data(), sizeof(gt::FEntry) * fce.size(), hipMemcpyHostToDevice));
+  return GT_OK;
+}
+int rect_tables(gt_ctx* c, const Rect& r, RectTables** out) {
+  RectTables& t = c->tab[rect_kind(c, r)];
+  *out = &t;
+  if (t.emk) return GT_OK;
+  RectTables b;  // all of them or none
+  const int rc = build_tables(c, r, b);
+  if (rc != GT_OK) {
+    drop_tables(b);
+    return rc;
+  }
+  b.ka = t.ka;
+  t = b;
   return GT_OK;
 }
 
@@ -774,13 +791,7 @@ int gt_destroy(gt_ctx* c) {
     if (m.owned && m.dref) (void)hipFree(m.dref);
     if (m.dcmp) (void)hipFree(m.dcmp);
   }
-  for (auto& t : c->tab) {
-    if (t.emk) (void)hipFree(t.emk);
-    if (t.ka) (void)hipFree(t.ka);
-    if (t.modes) (void)hipFree(t.modes);
-    if (t.fcs) (void)hipFree(t.fcs);
-    if (t.fce) (void)hipFree(t.fce);
-  }
+  for (auto& t : c->tab) drop_tables(t);
   if (c->tw) (void)hipFree(c->tw);
   if (c->y1) (void)hipFree(c->y1);
   if (c->y2) (void)hipFree(c->y2);

@@ -235,7 +235,7 @@ class Run:
         return self.L.shim_bad()
 
 
-D2Z = 1
+D2Z, Z2D = 1, 2
 
 
 @pytest.mark.parametrize("what,fails", [("fft_dir", "allocation"), ("fft_dir", "launch"),
@@ -294,3 +294,31 @@ def test_failed_allocation_of_the_diagnostics(lib, k):
     assert r.diag("glob", "z") != 0
     assert r.diag("glob", "z") == 0 and r.diag("spectrum", "z") == 0
     assert r.close() == 0
+
+
+@pytest.mark.parametrize("call", ["forced steps"])
+def test_every_allocation_may_fail(lib, call):
+    """Each allocation of the calls in turn fails; the same calls again then
+    succeed, on buffers that are all there."""
+    for k in range(1, 100):
+        r = Run(lib)
+        assert r.enter("z", "w", "a", "b", "c") == [0] * 5
+        seed = C.c_int32(5)
+
+        def calls():
+            if call == "gradient":
+                return [r("adj_forward", "z", "w", 3, 2, C.byref(seed)),
+                        r("adj_backward", "w", "a")]
+            return [r("step4", "z", "a", "w", "b", "c"), r("forcing", "z", C.byref(seed)),
+                    r("step4", "z", "a", "w", "b", "c"), r("fft_inv", "z", Z2D)]
+
+        lib.shim_fail_alloc(k)
+        failed = any(calls())
+        assert lib.shim_bad() == 0
+        lib.shim_fail_alloc(0)
+        r("update_device", "z")
+        assert not any(calls())
+        assert r.close() == 0
+        if not failed:
+            break
+    assert 5 < k < 99
