@@ -74,9 +74,6 @@ int adj_alloc(gt_ctx* c, int nsteps, int kchk) {
     s = c->adj;
     s->rc = c->rtr;
     s->kyp = kyp_of(c->rtr);
-    s->nc = nc;
-    s->kchk = kchk;
-    s->nstage = nstage;
     const int bt = gt::bt_of(c->logn);
     const size_t ycap = (size_t)((s->rc.kc() + bt - 1) / bt) * bt * c->n;
     HIPCHK(hipMalloc(&s->z, sizeof(double2) * nc));
@@ -91,6 +88,10 @@ int adj_alloc(gt_ctx* c, int nsteps, int kchk) {
     HIPCHK(hipMemsetAsync(s->stages, 0, sizeof(double2) * nc * nstage * kchk, c->stream));
     HIPCHK(hipMemsetAsync(s->y1, 0, sizeof(double2) * ycap * 5, c->stream));
     HIPCHK(hipMemsetAsync(s->y2, 0, sizeof(double2) * ycap * 3, c->stream));
+    // every buffer is there: until now a later call starts over
+    s->nc = nc;
+    s->kchk = kchk;
+    s->nstage = nstage;
   }
   while ((int)s->ck.size() < nck) {
     double2* p = nullptr;

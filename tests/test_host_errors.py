@@ -296,7 +296,7 @@ def test_failed_allocation_of_the_diagnostics(lib, k):
     assert r.close() == 0
 
 
-@pytest.mark.parametrize("call", ["forced steps"])
+@pytest.mark.parametrize("call", ["forced steps", "gradient"])
 def test_every_allocation_may_fail(lib, call):
     """Each allocation of the calls in turn fails; the same calls again then
     succeed, on buffers that are all there."""
