@@ -55,6 +55,10 @@ struct Mirror {
   // compact copy on the full rectangle straight from fft_dir: whether its
   // modes outside the 2/3 rectangle vanish has not been looked at
   bool wide = false;
+  // compact copy as fft_dir left it, the reference copy holding fft_dir's
+  // input: a mapped array's owner may put the next input there, or take the
+  // spectrum with gt_sync_ref and write to it
+  bool from_dir = false;
 };
 
 struct RectTables {

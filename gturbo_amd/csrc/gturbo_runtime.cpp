@@ -336,7 +336,7 @@ int lookup(gt_ctx* c, const void* host, Mirror** m) {
 // Room for a compact copy on rectangle r.  Its contents are to be written: the
 // old ones count no more, also where the allocation or the writing then fails.
 int alloc_cmp(gt_ctx*, Mirror& m, const Rect& r) {
-  m.cmp_valid = m.wide = false;
+  m.cmp_valid = m.wide = m.from_dir = false;
   const int kyp = kyp_of(r);
   const size_t need = (size_t)r.kc() * kyp;
   if (need > m.cmp_cap) {
@@ -443,12 +443,12 @@ int ensure_cmp(gt_ctx* c, Mirror& m) {
 void set_cmp_only(Mirror& m) {
   m.cmp_valid = true;
   m.ref_valid = false;
-  m.wide = false;
+  m.wide = m.from_dir = false;
 }
 void set_ref_only(Mirror& m) {
   m.ref_valid = true;
   m.cmp_valid = false;
-  m.wide = false;
+  m.wide = m.from_dir = false;
 }
 
 int pass_args(gt_ctx* c, Mirror& z, RectTables* t, gt::PassArgs* out) {
@@ -951,6 +951,8 @@ int gt_update_host(gt_ctx* c, void* host) {
   if (m.bytes >= ((size_t)c->n + 2) * c->n * sizeof(double)) CHK(ensure_ref(c, m));
   if (m.owned) {
     HIPCHK(hipMemcpyAsync(host, m.dref, m.bytes, hipMemcpyDeviceToHost, c->stream));
+  } else if (m.from_dir) {
+    set_ref_only(m);  // its owner may write to the spectrum
   }
   HIPCHK(hipStreamSynchronize(c->stream));
   return GT_OK;
@@ -989,6 +991,7 @@ int gt_copy(gt_ctx* c, void* dst, const void* src) {
                           hipMemcpyDeviceToDevice, c->stream));
     d->cmp_valid = true;
     d->wide = s->wide;
+    d->from_dir = s->from_dir;
     d->ref_valid = false;
     if (s->ref_valid) {
       HIPCHK(hipMemcpyAsync(d->dref, s->dref, ((size_t)c->n + 2) * c->n * sizeof(double),
@@ -1019,13 +1022,15 @@ int gt_fft_dir(gt_ctx* c, double* z, int32_t plan) {
   if (plan != GT_PLAN_D2Z) return fail(GT_ERR_ARG, "fft_dir needs a D2Z plan (got %d)", plan);
   Mirror* m;
   CHK(lookup(c, z, &m));
-  CHK(ensure_ref(c, *m));
+  if (m->owned || !m->from_dir) CHK(ensure_ref(c, *m));
+  m->ref_valid = true;  // a mapped array's next input, in place of its last one
   // the spectrum stays in the compact layout, every mode of it
   CHK(alloc_cmp(c, *m, c->rfull));
   Timer t(c, GT_K_OTHER);
   CHK(io_forward(c, m->dref, c->rfull, m->dcmp, 0));
   set_cmp_only(*m);
   m->wide = has_tr(c);
+  m->from_dir = true;
   return GT_OK;
 }
 

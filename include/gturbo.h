@@ -83,7 +83,12 @@ int gt_update_host(gt_ctx *ctx, void *host);
 int gt_update_device(gt_ctx *ctx, void *host);
 /* acc_map_data: attach caller-owned device memory (e.g. a torch tensor) as
  * the device copy of key; gt_sync_ref makes that memory current in the
- * reference layout. */
+ * reference layout.  The library keeps newer data in a layout of its own
+ * where it can: call gt_sync_ref before reading the memory and
+ * gt_update_device after writing to it.  (Not needed for the next input of
+ * gt_fft_dir where the last one was transformed and at most observed since,
+ * nor for writes to a spectrum that gt_sync_ref gave right after
+ * gt_fft_dir.) */
 int gt_map_data(gt_ctx *ctx, void *key, void *dev, int64_t bytes);
 int gt_unmap_data(gt_ctx *ctx, void *key);
 int gt_sync_ref(gt_ctx *ctx, void *key);

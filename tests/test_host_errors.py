@@ -222,6 +222,10 @@ class Run:
     def enter(self, *names):
         return [self("enter_data", n, C.c_int64(N * (N + 2) * 8), 1) for n in names]
 
+    def map(self, name):
+        n = N * (N + 2) * 8
+        return self("map_data", name, C.c_void_p(self.L.shim_device(n)), C.c_int64(n))
+
     def log(self):
         return self.L.shim_log().decode().split()
 
@@ -275,8 +279,7 @@ def test_unmapping_what_a_failed_copy_left(lib):
     assert r.enter("w") == [0]
     lib.shim_outside(1)
     assert r.diag("spectrum", "w") == 0
-    nbytes = N * (N + 2) * 8
-    assert r("map_data", "z", C.c_void_p(lib.shim_device(nbytes)), C.c_int64(nbytes)) == 0
+    assert r.map("z") == 0
     assert r("trunc", "z") == 0
     lib.shim_fail_alloc(1)
     assert r("copy", "z", "w") != 0 and r("update_host", "z") != 0
@@ -322,3 +325,21 @@ def test_every_allocation_may_fail(lib, call):
         if not failed:
             break
     assert 5 < k < 99
+
+
+@pytest.mark.parametrize("owned", [True, False])
+def test_what_an_owner_may_have_written(lib, owned):
+    """A mapped array that was transformed: its memory is read again by the next
+    fft_dir, and by whatever follows gt_sync_ref.  Host arrays, which only
+    gt_update_device changes, keep to the compact copy."""
+    r = Run(lib)
+    assert (r.enter("z") == [0]) if owned else (r.map("z") == 0)
+    assert r("fft_dir", "z", D2Z) == 0 and r.diag("spectrum", "z") == 0
+    n = len(r.log())
+    assert r("fft_dir", "z", D2Z) == 0
+    assert ("scatter" in r.log()[n:]) == owned
+    assert r("sync_ref", "z") == 0
+    n = len(r.log())
+    assert r.diag("spectrum", "z") == 0
+    assert ("gather" in r.log()[n:]) != owned
+    assert r.close() == 0
