@@ -1042,7 +1042,9 @@ int gt_fft_inv(gt_ctx* c, double* z, int32_t plan) {
   Mirror* m;
   CHK(lookup(c, z, &m));
   CHK(has_data(*m));
-  if (m->ref_valid) {  // a spectrum in the reference layout, all of it
+  if (m->ref_valid && !(m->owned && m->cmp_valid)) {
+    // a spectrum in the reference layout, all of it (a mapped array's owner
+    // may have written to it; a host array's copies hold the same)
     CHK(alloc_cmp(c, *m, c->rfull));
     HIPCHK(gt::launch_gather(c->ph, m->rect, m->kyp, m->dref, m->dcmp, 0, nullptr, c->stream));
   }

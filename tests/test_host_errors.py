@@ -343,3 +343,16 @@ def test_what_an_owner_may_have_written(lib, owned):
     assert r.diag("spectrum", "z") == 0
     assert ("gather" in r.log()[n:]) != owned
     assert r.close() == 0
+
+
+@pytest.mark.parametrize("owned", [True, False])
+def test_fft_inv_of_a_field_with_both_copies(lib, owned):
+    """A host array's compact copy is transformed as it is, in its own size; the
+    memory of a mapped one, which its owner may have written to, is read."""
+    r = Run(lib)
+    assert (r.enter("z") == [0]) if owned else (r.map("z") == 0)
+    assert r("trunc", "z") == 0 and r("sync_ref", "z") == 0
+    n = len(r.log())
+    assert r("fft_inv", "z", Z2D) == 0
+    assert r.log()[n:] == (["kept:io"] if owned else ["gather", "full:io"])
+    assert r.close() == 0
