@@ -1042,13 +1042,13 @@ int gt_fft_inv(gt_ctx* c, double* z, int32_t plan) {
   Mirror* m;
   CHK(lookup(c, z, &m));
   CHK(has_data(*m));
-  if (m->ref_valid && !(m->owned && m->cmp_valid)) {
-    // a spectrum in the reference layout, all of it (a mapped array's owner
-    // may have written to it; a host array's copies hold the same)
-    CHK(alloc_cmp(c, *m, c->rfull));
-    HIPCHK(gt::launch_gather(c->ph, m->rect, m->kyp, m->dref, m->dcmp, 0, nullptr, c->stream));
-  }
+  // A spectrum in the reference layout, all of it (a mapped array's owner may
+  // have written to it; a host array's copies hold the same).
+  const bool gather = m->ref_valid && !(m->owned && m->cmp_valid);
+  if (gather) CHK(alloc_cmp(c, *m, c->rfull));
   Timer t(c, GT_K_OTHER);
+  if (gather)
+    HIPCHK(gt::launch_gather(c->ph, m->rect, m->kyp, m->dref, m->dcmp, 0, nullptr, c->stream));
   CHK(io_inverse(c, m->dcmp, m->rect, m->dref));
   set_ref_only(*m);
   return GT_OK;
@@ -1079,13 +1079,14 @@ int gt_trunc(gt_ctx* c, double* z) {
   Mirror* m;
   CHK(lookup(c, z, &m));
   CHK(has_data(*m));
+  if (m->cmp_valid && m->wide) {
+    CHK(narrow(c, *m, 1));  // timed there
+    set_cmp_only(*m);
+    return GT_OK;
+  }
   Timer t(c, GT_K_OTHER);
   if (m->cmp_valid) {
-    if (m->wide) {
-      CHK(narrow(c, *m, 1));
-    } else {
-      HIPCHK(gt::launch_trunc_cmp(c->ph, m->rect, m->kyp, m->dcmp, c->stream));
-    }
+    HIPCHK(gt::launch_trunc_cmp(c->ph, m->rect, m->kyp, m->dcmp, c->stream));
     set_cmp_only(*m);
     return GT_OK;
   }

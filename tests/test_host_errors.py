@@ -356,3 +356,20 @@ def test_fft_inv_of_a_field_with_both_copies(lib, owned):
     assert r("fft_inv", "z", Z2D) == 0
     assert r.log()[n:] == (["kept:io"] if owned else ["gather", "full:io"])
     assert r.close() == 0
+
+
+@pytest.mark.parametrize("call,launches", [("fft_dir", ["full:io"]), ("trunc", ["narrow"]),
+                                           ("fft_inv", ["gather", "full:io"])])
+def test_timed_launches(lib, call, launches):
+    """Every launch of a transform or of trunc lies inside one timed interval."""
+    r = Run(lib)
+    assert r.map("z") == 0
+    if call == "trunc":
+        assert r("fft_dir", "z", D2Z) == 0
+    assert r("timing_enable", 1) == 0
+    n = len(r.log())
+    assert r(call, "z", *{"fft_dir": [D2Z], "trunc": [], "fft_inv": [Z2D]}[call]) == 0
+    assert r.log()[n:] == ["event", *launches, "event"]
+    count = (C.c_int32 * 16)()
+    assert r("timing_read", None, count) == 0 and sum(count) == 1
+    assert r.close() == 0
