@@ -411,8 +411,9 @@ static int narrow(gt_ctx* c, Mirror& m, int apply_trunc) {
 // rectangle is used unless the field has nonzero modes outside it.
 int ensure_cmp(gt_ctx* c, Mirror& m) {
   if (m.cmp_valid && m.wide) {
+    CHK(narrow(c, m, 0));
     m.wide = false;
-    return narrow(c, m, 0);
+    return GT_OK;
   }
   if (m.cmp_valid) return GT_OK;
   CHK(has_data(m));

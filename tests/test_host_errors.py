@@ -373,3 +373,15 @@ def test_timed_launches(lib, call, launches):
     count = (C.c_int32 * 16)()
     assert r("timing_read", None, count) == 0 and sum(count) == 1
     assert r.close() == 0
+
+
+def test_failed_look_outside_the_kept_rectangle(lib):
+    """A launch that fails while a transformed field is looked at for modes
+    outside the kept rectangle: the next call looks again."""
+    r = Run(lib)
+    assert r.enter("z") == [0] and r("fft_dir", "z", D2Z) == 0
+    lib.shim_fail_launch(b"narrow")
+    assert r.diag("spectrum", "z") != 0
+    n = len(r.log())
+    assert r.diag("spectrum", "z") == 0 and r.log()[n:] == ["narrow", "spectrum"]
+    assert r.close() == 0
