@@ -2388,6 +2388,16 @@ __device__ __forceinline__ double lane_value(double v, int lane) {
   return __hiloint2double(hi, lo);
 }
 
+// |v|^2.  As the square of the modulus (hypot): infinite where a part is, also
+// beside a NaN.  The wave looks only if one of its sums is a NaN.
+__device__ __forceinline__ double abs2(double2 v) {
+  double a = v.x * v.x + v.y * v.y;
+  if (__builtin_expect(__ballot(a != a) != 0, 0)) {
+    if (isinf(v.x) || isinf(v.y)) a = __builtin_huge_val();
+  }
+  return a;
+}
+
 // int(sqrt(k2)) of a whole number up to 2^25: the single-precision root, off
 // by at most one, put right.
 __device__ __forceinline__ int isqrt_of(double k2) {
@@ -2463,7 +2473,7 @@ __global__ void __launch_bounds__(kDiagT) shell_bin_k(DiagArgs d, int nbl) {
           key = ib;
           const double ka = kalpha(ph, k2);
           if (WHICH == 0) {
-            const double a2 = zv.x * zv.x + zv.y * zv.y;
+            const double a2 = abs2(zv);
             v1 = fac * a2 / ka;  // sp, diagnostics.f90:36
             v2 = fac * a2;       // sz, :37
           } else {
@@ -2666,7 +2676,7 @@ __global__ void __launch_bounds__(kDiagT) glob_col_k(DiagArgs d) {
       const double fky = (double)kyi_of(p, n) * ph.dky;
       const double k2 = fkxs + fky * fky;
       const double ka = kalpha(ph, k2);
-      const double a2 = fac * (zv[i].x * zv[i].x + zv[i].y * zv[i].y), ae = a2 / ka;
+      const double a2 = fac * abs2(zv[i]), ae = a2 / ka;
       const double gnu = 2.0 * ph.nu * pow_k2(k2, ph.alpnu);
       const double gmu = 2.0 * ph.mu * pow_k2(k2, ph.alpmu);
       acc[0] = acc[0] + ae;        // ee
