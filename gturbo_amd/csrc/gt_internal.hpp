@@ -238,7 +238,11 @@ struct IoArgs {
   int kyp;
   double2* cmp;
   int apply_trunc;  // dir < 0: the mask of src/trunc.f90
+  // dir < 0, if set: where kIoMark is written once ref has been read
+  unsigned long long* mark;
 };
+// A quiet NaN that no computation gives.
+constexpr unsigned long long kIoMark = 0x7FF8F1ECA55E7A6Eull;
 inline size_t io_size(int logn, const Rect& rc) {
   const int bt = bt_of(logn);
   return (size_t)((rc.kc() + bt - 1) / bt * bt) << logn;

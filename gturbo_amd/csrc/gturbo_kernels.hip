@@ -1308,12 +1308,14 @@ __device__ __forceinline__ void io_map(int tid, int& b, int& j) {
 template <int LOGN>
 __global__ void __launch_bounds__(io_cols(LOGN) * (1 << LOGN) / kE)
     io_cols_fwd(Phys ph, const double2* __restrict__ tw, const double2* __restrict__ y,
-                int ntiles, Rect rc, int kyp, double2* __restrict__ cmp, int apply_trunc) {
+                int ntiles, Rect rc, int kyp, double2* __restrict__ cmp, int apply_trunc,
+                unsigned long long* mark) {
   constexpr int N = 1 << LOGN, TPL = N / kE, CW = io_cols(LOGN), BT = bt_of(LOGN);
   __shared__ double2 lds[CW * io_line<LOGN>()];
   int b, j;
   io_map<LOGN>(threadIdx.x, b, j);
   const int wg = LOGN == 13 ? xcd_remap(blockIdx.x, gridDim.x) : (int)blockIdx.x;
+  if (mark != nullptr && blockIdx.x == 0 && threadIdx.x == 0) *mark = kIoMark;
   const int c = wg * CW + b;
   const bool ok = c <= rc.kx;
   double2* buf = lds + b * io_line<LOGN>();
@@ -1924,7 +1926,8 @@ hipError_t io_launch(const IoArgs& a, hipStream_t s) {
   const int nt = (a.rc.kc() + BT - 1) / BT;
   if (a.dir < 0) {
     io_rows_fwd<L><<<gr, br, 0, s>>>(a.ref, a.tw, a.y, nt, a.rc.kx);
-    io_cols_fwd<L><<<gc, bc, 0, s>>>(a.ph, a.tw, a.y, nt, a.rc, a.kyp, a.cmp, a.apply_trunc);
+    io_cols_fwd<L><<<gc, bc, 0, s>>>(a.ph, a.tw, a.y, nt, a.rc, a.kyp, a.cmp, a.apply_trunc,
+                                       a.mark);
   } else {
     io_cols_inv<L><<<gc, bc, 0, s>>>(a.tw, a.y, nt, a.rc, a.kyp, a.cmp);
     io_rows_inv<L><<<gr, br, 0, s>>>(a.ref, a.tw, a.y, nt, a.rc.kx);

@@ -304,17 +304,20 @@ int ensure_io(gt_ctx* c, const Rect& r) {
   return grow(&c->y1, &c->y1cap, std::max(gt::io_size(c->logn, r), 3 * yfield(c, c->rtr)));
 }
 
-int io_forward(gt_ctx* c, const double* ref, const Rect& r, double2* cmp, int apply_trunc) {
+int io_forward(gt_ctx* c, const double* ref, const Rect& r, double2* cmp, int apply_trunc,
+               bool mark) {
   CHK(ensure_io(c, r));
-  const gt::IoArgs a{-1, c->ph, const_cast<double*>(ref), c->tw, c->y1, r, kyp_of(r), cmp,
-                     apply_trunc};
+  double* p = const_cast<double*>(ref);
+  const gt::IoArgs a{-1, c->ph, p, c->tw, c->y1, r, kyp_of(r), cmp, apply_trunc,
+                     mark ? reinterpret_cast<unsigned long long*>(p) : nullptr};
   HIPCHK(gt::launch_io(c->logn, a, c->stream));
   return GT_OK;
 }
 
 int io_inverse(gt_ctx* c, const double2* cmp, const Rect& r, double* ref) {
   CHK(ensure_io(c, r));
-  const gt::IoArgs a{1, c->ph, ref, c->tw, c->y1, r, kyp_of(r), const_cast<double2*>(cmp), 0};
+  const gt::IoArgs a{1, c->ph, ref, c->tw, c->y1, r, kyp_of(r), const_cast<double2*>(cmp), 0,
+                     nullptr};
   HIPCHK(gt::launch_io(c->logn, a, c->stream));
   return GT_OK;
 }
@@ -360,6 +363,15 @@ static int has_data(const Mirror& m) {
 int ensure_ref(gt_ctx* c, Mirror& m) {
   if (m.ref_valid) return GT_OK;
   CHK(has_data(m));
+  if (m.from_dir) {
+    unsigned long long w = 0;
+    HIPCHK(hipMemcpyAsync(&w, m.dref, sizeof w, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(hipStreamSynchronize(c->stream));
+    if (w != gt::kIoMark) {  // its owner's data
+      set_ref_only(m);
+      return GT_OK;
+    }
+  }
   Timer t(c, GT_K_OTHER);
   HIPCHK(gt::launch_scatter(c->ph, m.rect, m.kyp, m.dcmp, m.dref, c->stream));
   m.ref_valid = true;
@@ -992,7 +1004,6 @@ int gt_copy(gt_ctx* c, void* dst, const void* src) {
                           hipMemcpyDeviceToDevice, c->stream));
     d->cmp_valid = true;
     d->wide = s->wide;
-    d->from_dir = s->from_dir;
     d->ref_valid = false;
     if (s->ref_valid) {
       HIPCHK(hipMemcpyAsync(d->dref, s->dref, ((size_t)c->n + 2) * c->n * sizeof(double),
@@ -1023,15 +1034,14 @@ int gt_fft_dir(gt_ctx* c, double* z, int32_t plan) {
   if (plan != GT_PLAN_D2Z) return fail(GT_ERR_ARG, "fft_dir needs a D2Z plan (got %d)", plan);
   Mirror* m;
   CHK(lookup(c, z, &m));
-  if (m->owned || !m->from_dir) CHK(ensure_ref(c, *m));
-  m->ref_valid = true;  // a mapped array's next input, in place of its last one
+  CHK(ensure_ref(c, *m));
   // the spectrum stays in the compact layout, every mode of it
   CHK(alloc_cmp(c, *m, c->rfull));
   Timer t(c, GT_K_OTHER);
-  CHK(io_forward(c, m->dref, c->rfull, m->dcmp, 0));
+  CHK(io_forward(c, m->dref, c->rfull, m->dcmp, 0, !m->owned));
   set_cmp_only(*m);
   m->wide = has_tr(c);
-  m->from_dir = true;
+  m->from_dir = !m->owned;
   return GT_OK;
 }
 

@@ -84,11 +84,11 @@ int gt_update_device(gt_ctx *ctx, void *host);
 /* acc_map_data: attach caller-owned device memory (e.g. a torch tensor) as
  * the device copy of key; gt_sync_ref makes that memory current in the
  * reference layout.  The library keeps newer data in a layout of its own
- * where it can: call gt_sync_ref before reading the memory and
- * gt_update_device after writing to it.  (Not needed for the next input of
- * gt_fft_dir where the last one was transformed and at most observed since,
- * nor for writes to a spectrum that gt_sync_ref gave right after
- * gt_fft_dir.) */
+ * where it can, and the memory's contents then mean nothing: call gt_sync_ref
+ * before reading it and gt_update_device after writing to it.  (After
+ * gt_fft_dir, and diagnostics of its result, the next gt_fft_dir,
+ * gt_sync_ref or gt_unmap_data notices a new frame in the memory by itself,
+ * and a spectrum that gt_sync_ref gave may be written to.) */
 int gt_map_data(gt_ctx *ctx, void *key, void *dev, int64_t bytes);
 int gt_unmap_data(gt_ctx *ctx, void *key);
 int gt_sync_ref(gt_ctx *ctx, void *key);

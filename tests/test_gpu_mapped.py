@@ -16,29 +16,49 @@ def _frame(n, seed):
     return w
 
 
-@pytest.mark.parametrize("n,copied", [(64, False), (64, True), (2048, False)])
-def test_frames_written_one_after_the_other(oracle_mod, n, copied):
+@pytest.mark.parametrize("n", [16, 64, 2048, 4096])
+def test_frames_written_one_after_the_other(oracle_mod, n):
     """A spectrum per frame, each frame put into the mapped array in place of
-    the one before (1e-12 as for the other spectra)."""
+    the one before; then one transformed twice, whose second transform is that
+    of its spectrum (1e-12 as for the other spectra)."""
     p = params_for(n)
     s, o = Solver(p), oracle_mod.Oracle(p)
-    t, src = (torch.zeros((n, n + 2), dtype=torch.float64, device="cuda") for _ in range(2))
-    for a in (t, src):
-        s.map_data(a)
-    for seed in (1, 2, 3):
+    t = torch.zeros((n, n + 2), dtype=torch.float64, device="cuda")
+    s.map_data(t)
+    for seed, times in ((1, 1), (1, 1), (2, 2), (3, 1)):
         w = _frame(n, seed)
-        (src if copied and seed == 1 else t).copy_(torch.from_numpy(w))
+        t.copy_(torch.from_numpy(w))
         torch.cuda.synchronize()
-        if copied and seed == 1:  # t starts as the copy of a transformed array
-            s.fft_dir(src)
-            s.copy(t, src)
-        else:
+        for _ in range(times):
             s.fft_dir(t)
-        got = s.spectrum(t)
-        o.fft_dir(w)
-        for g, e in zip(got, o.spectrum(w)):
-            assert np.max(np.abs(g - e)) <= 1e-12 * np.max(np.abs(e))
+            got = s.spectrum(t)
+            o.fft_dir(w)
+            for g, e in zip(got, o.spectrum(w)):
+                assert np.max(np.abs(g - e)) <= 1e-12 * np.max(np.abs(e))
     s.close()
+
+
+@pytest.mark.parametrize("written", [False, True])
+def test_unmapped_after_fft_dir(oracle_mod, written):
+    """The spectrum, or what its owner has put into the memory since."""
+    n = 64
+    p = params_for(n)
+    s, o = Solver(p), oracle_mod.Oracle(p)
+    w = _frame(n, 9)
+    t = torch.from_numpy(w).cuda()
+    torch.cuda.synchronize()
+    s.map_data(t)
+    s.fft_dir(t)
+    s.synchronize()
+    if written:
+        t.fill_(2.5)
+        torch.cuda.synchronize()
+        w[:] = 2.5
+    else:
+        o.fft_dir(w)
+    s.unmap_data(t)
+    s.close()
+    assert np.linalg.norm(t.cpu().numpy() - w) <= 1e-12 * np.linalg.norm(w)
 
 
 @pytest.mark.parametrize("n", [64, 2048])
