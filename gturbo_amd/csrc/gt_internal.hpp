@@ -256,7 +256,6 @@ hipError_t launch_j_pass(int logn, int mode, const AdjArgs& a, hipStream_t s);
 hipError_t launch_jr_pass(int logn, const AdjArgs& a, hipStream_t s);
 hipError_t launch_produ(int n, const double* z, double* u, double* v,
                         hipStream_t s);
-hipError_t launch_trunc_ref(const Phys& ph, double* z, hipStream_t s);
 hipError_t launch_trunc_cmp(const Phys& ph, const Rect& rc, int kyp,
                             double2* z, hipStream_t s);
 hipError_t launch_gather(const Phys& ph, const Rect& rc, int kyp,

@@ -442,7 +442,7 @@ __device__ __forceinline__ void c_body(const PassArgs& a, int tile, int tid,
 // 6397 -> 5829 (Stockham passes with ka in registers, which spilled).  On the
 // full one only at 8192 (9784 -> 9324); at 4096 its eight live values a field
 // leave no registers for the held twiddles (1887 -> 2080), at 2048 no change.
-template <int LOGN, int AK, int TR>
+template <int LOGN, int TR>
 __host__ __device__ constexpr bool c_pass_ip() { return TR == 1 || LOGN == 13; }
 template <int LOGN, int MODE, int AK, int TR>
 __global__ void __launch_bounds__(bt_of(LOGN) * (1 << LOGN) / kE, 4) c_pass(PassArgs a) {
@@ -450,7 +450,7 @@ __global__ void __launch_bounds__(bt_of(LOGN) * (1 << LOGN) / kE, 4) c_pass(Pass
   // Row slots in transform order (in-place transforms) on the 2/3 rectangle;
   // every y pass of a run has the same AK and TR, so the buffers' row order is
   // the same in all of them.
-  constexpr bool IP = c_pass_ip<LOGN, AK, TR>();
+  constexpr bool IP = c_pass_ip<LOGN, TR>();
   // The in-place transforms up to 4096 points hold their three twiddles in
   // registers (read once from memory): no table in LDS.
   constexpr bool HELD = IP && LOGN <= 12;
@@ -905,7 +905,7 @@ __global__ void __launch_bounds__(2 * fx_rows(LOGN) * (1 << LOGN) / kE) fx_pass(
 // of both rows; V0 + iV1 and U0 + iU1 likewise, and the products of the two
 // rows are again packed two-for-one for the forward transforms: five
 // transforms per row pair, only q carried across them.
-template <int LOGN, int TR, int BT, int NL, int SCHED, bool TWPF = false>
+template <int LOGN, int TR, int BT, int NL, int SCHED, bool HELD = false>
 __device__ __forceinline__ void pair_body(const PassArgs& a, int g, int tid,
                                           double2* lds, const double2* tw) {
   constexpr int N = 1 << LOGN, TPL = N / kE;
@@ -930,27 +930,27 @@ __device__ __forceinline__ void pair_body(const PassArgs& a, int g, int tid,
   const unsigned i0 = Y1 ? y1_off(y0, 0, cols) : r0, i1 = Y1 ? y1_off(y0 + 1, 0, cols) : r1;
   const unsigned fq = 0, fu = fs1, fv = 2 * fs1;
 
-  constexpr bool IP2 = LOGN == 13 && NL == 1 && TWPF;  // 8192: radix 2, then two 4096s
-  // the three twiddles every transform of the thread uses, loaded once (from
-  // memory; a table in LDS is read where it is needed)
+  constexpr bool IP2 = LOGN == 13;  // 8192: radix 2, then two 4096s
+  // HELD: the three twiddles every transform of the thread uses, loaded once
+  // (from memory; a table in LDS is read where it is needed)
   IpTw<LOGN> w{};
-  if constexpr (IP && TWPF) w = ip_tw<LOGN>(tw, j);
+  if constexpr (IP && HELD) w = ip_tw<LOGN>(tw, j);
   // bar: another wave may still read LDS (ignored by the Stockham transforms,
   // which synchronise on every transpose)
   auto inv = [&](double2* v, bool bar) {
-    if constexpr (IP && TWPF) fft_dif_held<LOGN, +1>(v, buf, j, w, bar);
+    if constexpr (IP && HELD) fft_dif_held<LOGN, +1>(v, buf, j, w, bar);
     else if constexpr (IP) fft_dif<+1, 1, LOGN>(v, buf, j, tw, bar);
     else if constexpr (IP2) fft_dif2<+1>(v, buf, j, tw, bar);
-    else fft_reg<LOGN, +1, SCHED, TWPF>(v, buf, j, tw);
+    else fft_reg<LOGN, +1, SCHED>(v, buf, j, tw);
   };
   auto fwd = [&](double2* v) {
     if constexpr (IP || IP2) {
-      if constexpr (IP && TWPF) fft_dit_held<LOGN, -1>(v, buf, j, w);
+      if constexpr (IP && HELD) fft_dit_held<LOGN, -1>(v, buf, j, w);
       else if constexpr (IP) fft_dit<-1, false, 1, LOGN>(v, buf, j, tw);
       else fft_dit2<-1>(v, buf, j, tw);
       __syncthreads();  // every wave's reads done before split_store writes
     } else {
-      fft_reg<LOGN, -1, SCHED, TWPF>(v, buf, j, tw);
+      fft_reg<LOGN, -1, SCHED>(v, buf, j, tw);
     }
   };
   double2 z[kE], qq[kE];
@@ -2147,18 +2147,7 @@ __global__ void produ_k(int n, const double* __restrict__ z, double* u,
   }
 }
 
-// src/trunc.f90:10-25 on the reference layout.
-__global__ void trunc_ref_k(Phys ph, double2* z) {
-  const int n = ph.n, nh = n / 2 + 1;
-  const size_t tot = (size_t)nh * n;
-  for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < tot;
-       e += (size_t)gridDim.x * blockDim.x) {
-    const int i = (int)(e % nh), jj = (int)(e / nh);
-    const double fkx = (double)i * ph.dkx, fky = (double)kyi_of(jj, n) * ph.dky;
-    if (cut_mode(ph, fkx * fkx, fky * fky) || e == 0) z[e] = make_double2(0.0, 0.0);
-  }
-}
-
+// src/trunc.f90:10-25 on a compact rectangle.
 __global__ void trunc_cmp_k(Phys ph, Rect rc, int kyp, double2* z) {
   const int n = ph.n, ky = rc.ky();
   const size_t tot = (size_t)rc.kc() * ky;
@@ -2784,12 +2773,6 @@ hipError_t launch_io(int logn, const IoArgs& a, hipStream_t s) {
 hipError_t launch_produ(int n, const double* z, double* u, double* v,
                         hipStream_t s) {
   produ_k<<<grid_for(((size_t)n + 2) * n, 256), 256, 0, s>>>(n, z, u, v);
-  return hipGetLastError();
-}
-
-hipError_t launch_trunc_ref(const Phys& ph, double* z, hipStream_t s) {
-  trunc_ref_k<<<grid_for((size_t)(ph.n / 2 + 1) * ph.n, 256), 256, 0, s>>>(
-      ph, reinterpret_cast<double2*>(z));
   return hipGetLastError();
 }
 
