@@ -124,7 +124,8 @@ enum CMode : int {
 };
 
 // Column-tile width of the y pass (BT) and y rows per workgroup of the x
-// pass, per log2 N.  A line is N/8 threads and (N + N/16) double2 of LDS.  Two
+// pass, per log2 N.  A line is N/8 threads and N + N/16 double2 of LDS (N + N/8
+// where it is transformed in place).  Two
 // columns (rows) per workgroup up to N = 4096: a 4-row block of two columns
 // is one 128-byte line, and small grids get as many workgroups as there
 // are column pairs (wider tiles left 256^2 with six y workgroups).

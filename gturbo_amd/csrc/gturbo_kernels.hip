@@ -476,12 +476,13 @@ __global__ void __launch_bounds__(bt_of(LOGN) * (1 << LOGN) / kE, 4) c_pass(Pass
 // bit-identical): y stage 64^2 11.1 -> 4.4 us, 256^2 12.0 -> 5.5, 512^2
 // (alpha 1) 14.6 -> 7.2, 1024^2 (alpha 1) 24.0 -> 18.0; step boundary 256^2
 // 15.4 -> 7.5, 1024^2 29.4 -> 20.7; x pass 5.0 -> 4.1, 5.8 -> 4.8, 7.8 ->
-// 6.5, 16.6 -> 15.6.  Up to 512^2 the rest is a kernel's own start and end
+// 6.5, 16.8 -> 16.2.  Up to 512^2 the rest is a kernel's own start and end
 // (about 2 us), two memory round trips and two transforms; at 1024^2 the
 // 41 MB a stage moves take half of it (12.7 us with the transforms skipped),
 // and in-place transforms, whose few barriers and held twiddles (100 instead
 // of 160 VGPRs) replace Stockham ones there, the next part: y stage 18.3 ->
-// 17.0 us, boundary 20.9 -> 18.5, untruncated 27 -> 24.4, x pass 15.6 -> 15.9.
+// 17.0 us, boundary 20.9 -> 18.5, untruncated 27 -> 24.4, x pass 16.2 -> 16.3
+// (the same within a run's spread, with half the twiddle error).
 // ---------------------------------------------------------------------------
 
 // Columns per workgroup of the y pass: a wave per field where a line is
@@ -833,7 +834,7 @@ __device__ __forceinline__ void r_body(const PassArgs& a, int g, int tid,
 // q+iu, each on its own N/8 threads; the operations are r_body's.  q v
 // crosses to the q u threads through LDS, these run the forward transform of
 // q u + i q v, and both store their half of the split spectrum.
-// Rows per workgroup: 512: two (6.4 us; one 7.2); 1024: one (15.3; two 15.5).
+// Rows per workgroup: 512: two (6.4 us; one 7.2); 1024: one (two 1% slower).
 __host__ __device__ constexpr int fx_rows(int logn) {
   return logn == 10 ? 1 : logn == 9 ? 2 : logn == 4 ? 16 : 512 >> logn;
 }
@@ -1093,9 +1094,10 @@ __global__ void __launch_bounds__(512, 4) r_pass_row(PassArgs a) {
   row_body13(a, xcd_remap(blockIdx.x, gridDim.x), threadIdx.x, lds, a.tw);
 }
 
-// One row pair per workgroup: two workgroups share a CU up to N = 4096 (at
-// 8192 one fills it: the rectangle wider than 3N/8 only).  Twiddles come
-// from memory, each transform pass loading the next pass's entry ahead.
+// One row pair per workgroup: four workgroups share a CU at N = 2048, two at
+// 4096 (at 8192 one fills it: the rectangle wider than 3N/8 only).  Twiddles
+// come from memory: the three of a thread loaded once and held, at 8192 each
+// where a transform needs it.
 template <int LOGN, int TR>
 __global__ void __launch_bounds__((1 << LOGN) / kE, 4)
     r_pass_pair(PassArgs a) {
@@ -1304,7 +1306,8 @@ __device__ __forceinline__ void io_map(int tid, int& b, int& j) {
 }
 
 // Block layout -> compact column, /NY/NX (src/fft_dir.f90:19; a power of
-// two: exact), with the mask of src/trunc.f90 when apply_trunc is set.
+// two: exact), with the mask of src/trunc.f90 when apply_trunc is set.  mark
+// (if set) lies in the physical field, which io_rows_fwd has read by now.
 template <int LOGN>
 __global__ void __launch_bounds__(io_cols(LOGN) * (1 << LOGN) / kE)
     io_cols_fwd(Phys ph, const double2* __restrict__ tw, const double2* __restrict__ y,
@@ -1996,8 +1999,9 @@ template hipError_t io_launch<GT_INST_LOGN>(const IoArgs&, hipStream_t);
 // Batched ensemble passes.  One launch covers the pass of every member,
 // whatever its N and alpha: the workgroups loop over a list of work items
 // (member, tile) and run the pass body of the member's size.  For T threads
-// a workgroup holds T*8/N lines of N points, i.e. T*8*17/16 double2 of LDS
-// for every N, so the sizes share one LDS allocation.  Alpha enters through
+// a workgroup holds T*8/N lines of N points, T*8 elements of any N; padded they
+// take T*17/2 double2 of LDS (Stockham lines, N + N/16) or T*9 (in-place lines,
+// N + N/8, from 1024 on), so the sizes share one allocation of T*9.  Alpha enters through
 // kalpha_t<2>, the x-pass packing per member through PassArgs::xvar, the
 // radix order (SCHED) per launch.  Every member has the 2/3 rectangle
 // (TR = 1).  Compiled once per (T, SCHED): -DGT_INST_ENS=T
@@ -2206,9 +2210,10 @@ __global__ void outside_cmp_k(Phys ph, Rect rf, int kypf, const double2* __restr
   if (v.x != 0.0 || v.y != 0.0) atomicOr(flag, 1);
 }
 
-// ka = k2**(alpv/2) over the compact rectangle, with the expressions of the
-// y pass (c_body, AK = 0), so that a batched member reading the table and a
-// single run computing ka in place get the same values.
+// ka = k2**(alpv/2) over the compact rectangle, with kalpha's expressions.  Read
+// by the batched passes, by f_pass and fj_pass (N <= 1024, 512) away from alpha
+// = 2 and by c_pass for powers other than roots, so that a member and the same
+// run alone use the same values.
 __global__ void ka_table_k(Phys ph, Rect rc, int kyp, double* ka) {
   const int n = ph.n, ky = rc.ky();
   const size_t tot = (size_t)rc.kc() * ky;
