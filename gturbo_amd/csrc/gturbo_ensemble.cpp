@@ -142,11 +142,13 @@ int apply(gt_ens* e, const int32_t* cfg) {
   }
   const size_t need = yi.size() + xi.size();
   if (need > e->items_cap) {
+    // the lists in use stay until the new ones have their room
+    uint32_t* p = nullptr;
+    HIPCHK(hipMalloc(&p, sizeof(uint32_t) * need));
     if (e->items) (void)hipFree(e->items);
-    e->items = nullptr;
-    e->items_cap = 0;
-    HIPCHK(hipMalloc(&e->items, sizeof(uint32_t) * need));
+    e->items = p;
     e->items_cap = need;
+    drop_graph(e);  // it reads the old ones
   }
   HIPCHK(hipStreamSynchronize(e->stream));
   HIPCHK(hipMemcpy(e->items, yi.data(), sizeof(uint32_t) * yi.size(), hipMemcpyHostToDevice));

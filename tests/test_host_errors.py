@@ -86,6 +86,18 @@ hipError_t hipMemsetAsync(void* d, int v, size_t n, hipStream_t) {
 hipError_t hipMemGetInfo(size_t* f, size_t* t) { *f = *t = 0; return hipSuccess; }
 hipError_t hipGetDeviceCount(int* n) { *n = 1; return hipSuccess; }
 const char* hipGetErrorString(hipError_t) { return "made to fail"; }
+hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
+hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) { *v = 256; return hipSuccess; }
+hipError_t hipEventCreate(hipEvent_t* e) { return hipEventCreateWithFlags(e, 0); }
+hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return hipSuccess; }
+hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t* g) { *g = nullptr; return hipSuccess; }
+hipError_t hipGraphInstantiate(hipGraphExec_t* e, hipGraph_t, hipGraphNode_t*, char*, size_t) {
+  *e = (hipGraphExec_t)malloc(1);
+  return hipSuccess;
+}
+hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { return hipSuccess; }
+hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
+hipError_t hipGraphExecDestroy(hipGraphExec_t e) { free((void*)e); return hipSuccess; }
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { *s = nullptr; return hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
@@ -171,6 +183,18 @@ hipError_t launch_glob(const DiagArgs& d, hipStream_t) {
   return ran("glob", {d.z, d.gpart, d.gout});
 }
 hipError_t launch_shell_index(const Phys&, int* ib, hipStream_t) { return ran("shell", {ib}); }
+hipError_t launch_ens_c_pass(int, int, int, const PassArgs* d, const uint32_t* it, int n, int,
+                             hipStream_t) {
+  return ran("ens y", {d, it, it + n - 1});
+}
+hipError_t launch_ens_r_pass(int, int, int, const PassArgs* d, const uint32_t* it, int n, int,
+                             hipStream_t) {
+  return ran("ens x", {d, it, it + n - 1});
+}
+hipError_t launch_ens_forcing(const EnsForce* f, int, int, const int* s, hipStream_t) {
+  return ran("ens forcing", {f, s});
+}
+hipError_t launch_ens_tick(int* s, hipStream_t) { return ran("tick", {s}); }
 hipError_t launch_ka_table(const Phys&, const Rect&, int, double* k, hipStream_t) {
   return ran("ka", {k});
 }
@@ -185,9 +209,9 @@ def lib(tmp_path_factory):
     d = tmp_path_factory.mktemp("host")
     (d / "shim.cpp").write_text(SHIM)
     srcs = [str(d / "shim.cpp")] + [os.path.join(CSRC, f"gturbo_{s}.cpp")
-                                    for s in ("runtime", "adjoint", "phases")]
+                                    for s in ("runtime", "adjoint", "ensemble", "phases")]
     out = str(d / "host.so")
-    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__",
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-pthread", "-D__HIP_PLATFORM_AMD__",
                     "-Wno-unused-result", "-Wl,-Bsymbolic", f"-I{CSRC}",
                     f"-I{os.path.join(ROOT, 'include')}", "-I/opt/rocm/include", *srcs, "-o", out],
                    check=True)
@@ -197,18 +221,21 @@ def lib(tmp_path_factory):
     return L
 
 
+def _params(alpv):
+    return [2 * np.pi, 2 * np.pi, 1e-9, 4.0, 0.1, 0.0, alpv, 1e-3, 4, 1, 1, 1, 2.0 / 3.0, 1, 1.0,
+            2.0, 4.0]
+
+
 class Run:
     """A context and named arrays on that HIP; every call gives its code."""
 
     def __init__(self, lib):
         self.L = lib
         lib.shim_reset()
-        p = [2 * np.pi, 2 * np.pi, 1e-9, 4.0, 0.1, 0.0, 2.0, 1e-3, 4, 1, 1, 1, 2.0 / 3.0, 1, 1.0,
-             2.0, 4.0]
         self.h = C.c_void_p()
         self.a = {}
         self.out = np.zeros(2 * N)
-        assert lib.gt_create(N, (C.c_double * 17)(*p), C.byref(self.h)) == 0
+        assert lib.gt_create(N, (C.c_double * 17)(*_params(2.0)), C.byref(self.h)) == 0
 
     def __call__(self, name, *args):
         return getattr(self.L, "gt_" + name)(self.h, *[self.ptr(x) for x in args])
@@ -391,3 +418,29 @@ def test_failed_look_outside_the_kept_rectangle(lib):
     n = len(r.log())
     assert r.diag("spectrum", "z") == 0 and r.log()[n:] == ["narrow", "spectrum"]
     assert r.close() == 0
+
+
+def test_allocations_of_an_ensemble_may_fail(lib):
+    """Each allocation of an ensemble's making and of a schedule with more work
+    items fails in turn: no ensemble, or one that still runs the schedule it
+    had."""
+    n = (C.c_int32 * 2)(128, 256)
+    p = (C.c_double * 34)(*_params(2.0), *_params(1.0))
+    wide = (C.c_int32 * 6)(256, 256, 0, 0, 0, 1)
+    for k in range(1, 100):
+        lib.shim_reset()
+        e = C.c_void_p()
+        lib.shim_fail_alloc(k)
+        rc = lib.gt_ens_create(2, n, p, C.byref(e))
+        if rc != 0:
+            assert not e.value and lib.shim_bad() == 0
+            continue
+        assert lib.gt_ens_run(e, 3) == 0
+        rc = lib.gt_ens_schedule(e, wide, 1)
+        lib.shim_fail_alloc(0)
+        assert lib.gt_ens_run(e, 3) == 0 and lib.shim_bad() == 0
+        assert lib.gt_ens_schedule(e, wide, 1) == 0 and lib.gt_ens_run(e, 3) == 0
+        assert lib.gt_ens_destroy(e) == 0 and lib.shim_bad() == 0
+        if rc == 0:
+            break
+    assert 20 < k < 99
