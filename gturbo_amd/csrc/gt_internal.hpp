@@ -239,9 +239,21 @@ struct IoArgs {
   int kyp;
   double2* cmp;
   int apply_trunc;  // dir < 0: the mask of src/trunc.f90
-  // dir < 0, if set: where kIoMark is written once ref has been read
+  // dir > 0: row stride of cmp, whose column stride is kyp: 1, or N/2 + 1 (and
+  // kyp = 1) for a spectrum in the reference layout
+  int rs;
+  // dir < 0, once ref has been read, if set: where kIoMark is written, and where
+  // the spectrum goes in the reference layout, too (rc the whole half-spectrum)
   unsigned long long* mark;
+  double2* dual;
 };
+// Largest log2 N whose 2D transforms read (mapped arrays: also write) spectra in
+// the reference layout themselves, in 16-byte pieces, instead of through
+// gather_k and scatter_k: up to there a launch costs more than the pieces do
+// (fft_inv of such a spectrum 64^2 19.1 -> 16.0 us, 512^2 24.2 -> 20.4; fft_dir and
+// gt_sync_ref 19.4 -> 17.1, 27.2 -> 20.1; fft_dir and trunc, which have no use for
+// it, 18.9 -> 19.1, 21.0 -> 22.2).
+constexpr int kIoDirect = 9;
 // A quiet NaN that no computation gives.
 constexpr unsigned long long kIoMark = 0x7FF8F1ECA55E7A6Eull;
 inline size_t io_size(int logn, const Rect& rc) {
@@ -269,6 +281,9 @@ hipError_t launch_narrow(const Phys& ph, const Rect& rf, int kypf, const double2
                          int* outside_flag, hipStream_t s);
 hipError_t launch_scatter(const Phys& ph, const Rect& rc, int kyp,
                           const double2* cmp, double* ref, hipStream_t s);
+// The same if ref starts with kIoMark, else nothing.
+hipError_t launch_scatter_marked(const Phys& ph, const Rect& rc, int kyp, const double2* cmp,
+                                 double* ref, hipStream_t s);
 hipError_t launch_forcing(const Phys& ph, int nf, const ForcedMode* modes,
                           const double2* phases, double amp, double2* z,
                           hipStream_t s);

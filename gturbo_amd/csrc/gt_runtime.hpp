@@ -55,9 +55,9 @@ struct Mirror {
   // compact copy on the full rectangle straight from fft_dir: whether its
   // modes outside the 2/3 rectangle vanish has not been looked at
   bool wide = false;
-  // mapped array, compact copy as fft_dir left it, kIoMark in its memory: its
-  // owner may put the next input there (the mark is gone then), or take the
-  // spectrum with gt_sync_ref and write to it
+  // mapped array, compact copy as fft_dir left it; its memory holds the spectrum,
+  // too (ref_valid), or kIoMark: its owner may put the next input there (the mark
+  // is gone then), or take the spectrum with gt_sync_ref and write to it
   bool from_dir = false;
 };
 
@@ -164,9 +164,10 @@ int ensure_ybuf(gt_ctx* c, const Rect& r);
 int ensure_io(gt_ctx* c, const Rect& r);
 // fft_dir (with or without trunc) of a physical field into a compact one on
 // rectangle r, and fft_inv of a compact one; scratch is the y1 buffer.
-// mark: kIoMark goes to the start of ref when it has been read.
+// When ref has been read, kIoMark goes to its start (mark), or the spectrum
+// into it in the reference layout (dual; r the whole half-spectrum).
 int io_forward(gt_ctx* c, const double* ref, const Rect& r, double2* cmp, int apply_trunc,
-               bool mark = false);
+               bool mark = false, bool dual = false);
 int io_inverse(gt_ctx* c, const double2* cmp, const Rect& r, double* ref);
 int lookup(gt_ctx* c, const void* host, Mirror** m);
 int alloc_cmp(gt_ctx* c, Mirror& m, const Rect& r);

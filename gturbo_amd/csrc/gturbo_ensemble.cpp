@@ -448,7 +448,8 @@ int gt_ens_set_field(gt_ens* e, int32_t m, const double* z, int32_t space) {
   hipError_t err = hipMemcpyAsync(tmp, z, bytes, hipMemcpyHostToDevice, e->stream);
   if (err == hipSuccess) err = hipMemsetAsync(e->flag, 0, sizeof(int), e->stream);
   if (err == hipSuccess && space == GT_SPACE_PHYSICAL)  // fft_dir and trunc
-    err = gt::launch_io(c->logn, {-1, c->ph, tmp, c->tw, mb.y1, mb.rc, mb.kyp, mb.z, 1, nullptr},
+    err = gt::launch_io(c->logn,
+                        {-1, c->ph, tmp, c->tw, mb.y1, mb.rc, mb.kyp, mb.z, 1, 1, nullptr, nullptr},
                         e->stream);
   if (err == hipSuccess && space == GT_SPACE_SPECTRAL)  // the rectangle as is
     err = gt::launch_gather(c->ph, mb.rc, mb.kyp, tmp, mb.z, 0, e->flag, e->stream);
@@ -474,7 +475,8 @@ int gt_ens_get_field(gt_ens* e, int32_t m, double* z, int32_t space) {
   HIPCHK(hipMalloc(&tmp, bytes));
   hipError_t err =
       space == GT_SPACE_PHYSICAL  // fft_inv
-          ? gt::launch_io(c->logn, {1, c->ph, tmp, c->tw, mb.y1, mb.rc, mb.kyp, mb.z, 0, nullptr},
+          ? gt::launch_io(c->logn,
+                          {1, c->ph, tmp, c->tw, mb.y1, mb.rc, mb.kyp, mb.z, 0, 1, nullptr, nullptr},
                           e->stream)
           : gt::launch_scatter(c->ph, mb.rc, mb.kyp, mb.z, tmp, e->stream);
   if (err == hipSuccess) err = hipMemcpyAsync(z, tmp, bytes, hipMemcpyDeviceToHost, e->stream);

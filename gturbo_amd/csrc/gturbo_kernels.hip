@@ -1312,7 +1312,7 @@ template <int LOGN>
 __global__ void __launch_bounds__(io_cols(LOGN) * (1 << LOGN) / kE)
     io_cols_fwd(Phys ph, const double2* __restrict__ tw, const double2* __restrict__ y,
                 int ntiles, Rect rc, int kyp, double2* __restrict__ cmp, int apply_trunc,
-                unsigned long long* mark) {
+                unsigned long long* mark, double2* __restrict__ dual) {
   constexpr int N = 1 << LOGN, TPL = N / kE, CW = io_cols(LOGN), BT = bt_of(LOGN);
   __shared__ double2 lds[CW * io_line<LOGN>()];
   int b, j;
@@ -1341,14 +1341,16 @@ __global__ void __launch_bounds__(io_cols(LOGN) * (1 << LOGN) / kE)
     if (apply_trunc && (cut_mode(ph, fkx * fkx, fky * fky) || (c == 0 && p == 0)))
       v = make_double2(0.0, 0.0);
     cmp[(size_t)c * kyp + row] = v;
+    if (LOGN <= kIoDirect && dual != nullptr) dual[(size_t)p * (N / 2 + 1) + c] = v;
   }
 }
 
-// Compact column (zero outside the rectangle) -> block layout.
+// Column of a spectrum (element (c, row) at c cs + row rs; zero outside the
+// rectangle) -> block layout.
 template <int LOGN>
 __global__ void __launch_bounds__(io_cols(LOGN) * (1 << LOGN) / kE)
     io_cols_inv(const double2* __restrict__ tw, double2* __restrict__ y, int ntiles, Rect rc,
-                int kyp, const double2* __restrict__ cmp) {
+                int cs, int rs, const double2* __restrict__ cmp) {
   constexpr int N = 1 << LOGN, TPL = N / kE, CW = io_cols(LOGN), BT = bt_of(LOGN);
   __shared__ double2 lds[CW * io_line<LOGN>()];
   int b, j;
@@ -1361,7 +1363,7 @@ __global__ void __launch_bounds__(io_cols(LOGN) * (1 << LOGN) / kE)
 #pragma unroll
   for (int r = 0; r < kE; ++r) {
     const int row = row_of(j + TPL * r, rc, N);
-    w[r] = ok && row >= 0 ? cmp[(size_t)c * kyp + row] : make_double2(0.0, 0.0);
+    w[r] = ok && row >= 0 ? cmp[(size_t)c * cs + (size_t)row * rs] : make_double2(0.0, 0.0);
   }
   if constexpr (LOGN == 12) fft_dif<+1>(w, buf, j, tw, false);
   else if constexpr (LOGN == 13) fft_dif2<+1>(w, buf, j, tw, false);
@@ -1930,9 +1932,9 @@ hipError_t io_launch(const IoArgs& a, hipStream_t s) {
   if (a.dir < 0) {
     io_rows_fwd<L><<<gr, br, 0, s>>>(a.ref, a.tw, a.y, nt, a.rc.kx);
     io_cols_fwd<L><<<gc, bc, 0, s>>>(a.ph, a.tw, a.y, nt, a.rc, a.kyp, a.cmp, a.apply_trunc,
-                                       a.mark);
+                                       a.mark, a.dual);
   } else {
-    io_cols_inv<L><<<gc, bc, 0, s>>>(a.tw, a.y, nt, a.rc, a.kyp, a.cmp);
+    io_cols_inv<L><<<gc, bc, 0, s>>>(a.tw, a.y, nt, a.rc, a.kyp, a.rs, a.cmp);
     io_rows_inv<L><<<gr, br, 0, s>>>(a.ref, a.tw, a.y, nt, a.rc.kx);
   }
   return hipGetLastError();
@@ -2254,6 +2256,30 @@ __global__ void scatter_k(Phys ph, Rect rc, int kyp, const double2* __restrict__
     ref[e] = (i <= rc.kx && r >= 0) ? cmp[(size_t)i * kyp + r]
                                     : make_double2(0.0, 0.0);
   }
+}
+
+// The same if ref starts with kIoMark, else nothing: all but the element that the
+// mark lies in, which one thread writes after that.  (A block counter in place of
+// the second launch took 300 us at 4096^2: 65536 atomics on one address.)
+__device__ __forceinline__ bool io_marked(const double2* ref) {
+  return *reinterpret_cast<const unsigned long long*>(ref) == kIoMark;
+}
+__global__ void scatter_marked_k(Phys ph, Rect rc, int kyp, const double2* __restrict__ cmp,
+                                 double2* ref) {
+  if (!io_marked(ref)) return;
+  const int n = ph.n, nh = n / 2 + 1;
+  const size_t tot = (size_t)nh * n;
+  for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < tot;
+       e += (size_t)gridDim.x * blockDim.x) {
+    const int i = (int)(e % nh), p = (int)(e / nh);
+    const int r = row_of(p, rc, n);
+    if (e > 0)
+      ref[e] = (i <= rc.kx && r >= 0) ? cmp[(size_t)i * kyp + r]
+                                      : make_double2(0.0, 0.0);
+  }
+}
+__global__ void scatter_mark_k(const double2* __restrict__ cmp, double2* ref) {
+  if (io_marked(ref)) ref[0] = cmp[0];  // mode (0, 0) lies in every rectangle
 }
 
 // src/forcing.f90:16-33.  One thread per forced mode: no two modes share an
@@ -2814,6 +2840,15 @@ hipError_t launch_scatter(const Phys& ph, const Rect& rc, int kyp, const double2
                           double* ref, hipStream_t s) {
   scatter_k<<<grid_for((size_t)(ph.n / 2 + 1) * ph.n, 256), 256, 0, s>>>(
       ph, rc, kyp, cmp, reinterpret_cast<double2*>(ref));
+  return hipGetLastError();
+}
+
+hipError_t launch_scatter_marked(const Phys& ph, const Rect& rc, int kyp, const double2* cmp,
+                                 double* ref, hipStream_t s) {
+  double2* r = reinterpret_cast<double2*>(ref);
+  scatter_marked_k<<<grid_for((size_t)(ph.n / 2 + 1) * ph.n, 256), 256, 0, s>>>(ph, rc, kyp, cmp,
+                                                                               r);
+  scatter_mark_k<<<1, 1, 0, s>>>(cmp, r);
   return hipGetLastError();
 }
 

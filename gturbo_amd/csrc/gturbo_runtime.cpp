@@ -305,19 +305,29 @@ int ensure_io(gt_ctx* c, const Rect& r) {
 }
 
 int io_forward(gt_ctx* c, const double* ref, const Rect& r, double2* cmp, int apply_trunc,
-               bool mark) {
+               bool mark, bool dual) {
   CHK(ensure_io(c, r));
   double* p = const_cast<double*>(ref);
-  const gt::IoArgs a{-1, c->ph, p, c->tw, c->y1, r, kyp_of(r), cmp, apply_trunc,
-                     mark ? reinterpret_cast<unsigned long long*>(p) : nullptr};
+  const gt::IoArgs a{-1, c->ph, p, c->tw, c->y1, r, kyp_of(r), cmp, apply_trunc, 1,
+                     mark ? reinterpret_cast<unsigned long long*>(p) : nullptr,
+                     dual ? reinterpret_cast<double2*>(p) : nullptr};
   HIPCHK(gt::launch_io(c->logn, a, c->stream));
   return GT_OK;
 }
 
 int io_inverse(gt_ctx* c, const double2* cmp, const Rect& r, double* ref) {
   CHK(ensure_io(c, r));
-  const gt::IoArgs a{1, c->ph, ref, c->tw, c->y1, r, kyp_of(r), const_cast<double2*>(cmp), 0,
-                     nullptr};
+  const gt::IoArgs a{1, c->ph, ref, c->tw, c->y1, r, kyp_of(r), const_cast<double2*>(cmp), 0, 1,
+                     nullptr, nullptr};
+  HIPCHK(gt::launch_io(c->logn, a, c->stream));
+  return GT_OK;
+}
+
+// fft_inv of a spectrum in the reference layout, all of it, in place.
+static int io_inverse_ref(gt_ctx* c, double* ref) {
+  CHK(ensure_io(c, c->rfull));
+  const gt::IoArgs a{1, c->ph, ref, c->tw, c->y1, c->rfull, 1, reinterpret_cast<double2*>(ref),
+                     0, c->nh, nullptr, nullptr};
   HIPCHK(gt::launch_io(c->logn, a, c->stream));
   return GT_OK;
 }
@@ -363,16 +373,12 @@ static int has_data(const Mirror& m) {
 int ensure_ref(gt_ctx* c, Mirror& m) {
   if (m.ref_valid) return GT_OK;
   CHK(has_data(m));
-  if (m.from_dir) {
-    unsigned long long w = 0;
-    HIPCHK(hipMemcpyAsync(&w, m.dref, sizeof w, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    if (w != gt::kIoMark) {  // its owner's data
-      set_ref_only(m);
-      return GT_OK;
-    }
-  }
   Timer t(c, GT_K_OTHER);
+  if (m.from_dir) {  // the spectrum, or what its owner has put there since
+    HIPCHK(gt::launch_scatter_marked(c->ph, m.rect, m.kyp, m.dcmp, m.dref, c->stream));
+    set_ref_only(m);
+    return GT_OK;
+  }
   HIPCHK(gt::launch_scatter(c->ph, m.rect, m.kyp, m.dcmp, m.dref, c->stream));
   m.ref_valid = true;
   return GT_OK;
@@ -1005,7 +1011,7 @@ int gt_copy(gt_ctx* c, void* dst, const void* src) {
     d->cmp_valid = true;
     d->wide = s->wide;
     d->ref_valid = false;
-    if (s->ref_valid) {
+    if (s->ref_valid && !s->from_dir) {
       HIPCHK(hipMemcpyAsync(d->dref, s->dref, ((size_t)c->n + 2) * c->n * sizeof(double),
                             hipMemcpyDeviceToDevice, c->stream));
       d->ref_valid = true;
@@ -1038,8 +1044,10 @@ int gt_fft_dir(gt_ctx* c, double* z, int32_t plan) {
   // the spectrum stays in the compact layout, every mode of it
   CHK(alloc_cmp(c, *m, c->rfull));
   Timer t(c, GT_K_OTHER);
-  CHK(io_forward(c, m->dref, c->rfull, m->dcmp, 0, !m->owned));
+  const bool dual = !m->owned && c->logn <= gt::kIoDirect;
+  CHK(io_forward(c, m->dref, c->rfull, m->dcmp, 0, !m->owned && !dual, dual));
   set_cmp_only(*m);
+  m->ref_valid = dual;
   m->wide = has_tr(c);
   m->from_dir = !m->owned;
   return GT_OK;
@@ -1055,12 +1063,14 @@ int gt_fft_inv(gt_ctx* c, double* z, int32_t plan) {
   CHK(has_data(*m));
   // A spectrum in the reference layout, all of it (a mapped array's owner may
   // have written to it; a host array's copies hold the same).
-  const bool gather = m->ref_valid && !(m->owned && m->cmp_valid);
+  const bool of_ref = m->ref_valid && !(m->owned && m->cmp_valid);
+  const bool gather = of_ref && c->logn > gt::kIoDirect;
   if (gather) CHK(alloc_cmp(c, *m, c->rfull));
   Timer t(c, GT_K_OTHER);
   if (gather)
     HIPCHK(gt::launch_gather(c->ph, m->rect, m->kyp, m->dref, m->dcmp, 0, nullptr, c->stream));
-  CHK(io_inverse(c, m->dcmp, m->rect, m->dref));
+  if (of_ref && !gather) CHK(io_inverse_ref(c, m->dref));
+  else CHK(io_inverse(c, m->dcmp, m->rect, m->dref));
   set_ref_only(*m);
   return GT_OK;
 }

@@ -142,7 +142,8 @@ hipError_t launch_r_pass(int, const PassArgs& a, hipStream_t) {
 hipError_t launch_io(int, const IoArgs& a, hipStream_t) {
   log_ += a.rc.kx == a.ph.n / 2 ? "full:" : "kept:";
   if (a.mark && ok(a.mark)) *a.mark = kIoMark;
-  return ran("io", {a.ref, a.tw, a.y, a.cmp});
+  if (a.dual) ok(a.dual);
+  return ran(a.dual ? "io+ref" : "io", {a.ref, a.tw, a.y, a.cmp});
 }
 hipError_t launch_j_pass(int, int, const AdjArgs& a, hipStream_t) {
   may(a.snext);
@@ -170,6 +171,12 @@ hipError_t launch_narrow(const Phys&, const Rect&, int, const double2* s, const 
 hipError_t launch_scatter(const Phys&, const Rect&, int, const double2* c, double* r,
                           hipStream_t) {
   return ran("scatter", {c, r});
+}
+hipError_t launch_scatter_marked(const Phys&, const Rect&, int, const double2* c, double* r,
+                                 hipStream_t) {
+  unsigned long long w;
+  memcpy(&w, r, sizeof w);
+  return w == kIoMark ? ran("scatter", {c, r}) : ran("keep", {r});
 }
 hipError_t launch_forcing(const Phys&, int, const ForcedMode* m, const double2* p, double,
                           double2* z, hipStream_t) {
@@ -201,7 +208,7 @@ hipError_t launch_ka_table(const Phys&, const Rect&, int, double* k, hipStream_t
 }  // namespace gt
 """
 
-N = 32
+N = 1024  # (up to 512 the 2D transforms read and write reference layouts themselves)
 
 
 @pytest.fixture(scope="module")
@@ -229,13 +236,13 @@ def _params(alpv):
 class Run:
     """A context and named arrays on that HIP; every call gives its code."""
 
-    def __init__(self, lib):
-        self.L = lib
+    def __init__(self, lib, n=N):
+        self.L, self.n = lib, n
         lib.shim_reset()
         self.h = C.c_void_p()
         self.a = {}
-        self.out = np.zeros(2 * N)
-        assert lib.gt_create(N, (C.c_double * 17)(*_params(2.0)), C.byref(self.h)) == 0
+        self.out = np.zeros(2 * n)
+        assert lib.gt_create(n, (C.c_double * 17)(*_params(2.0)), C.byref(self.h)) == 0
 
     def __call__(self, name, *args):
         return getattr(self.L, "gt_" + name)(self.h, *[self.ptr(x) for x in args])
@@ -244,14 +251,14 @@ class Run:
         if not isinstance(x, str):
             return x
         if x not in self.a:
-            self.a[x] = np.zeros((N, N + 2))
+            self.a[x] = np.zeros((self.n, self.n + 2))
         return C.c_void_p(self.a[x].ctypes.data)
 
     def enter(self, *names):
-        return [self("enter_data", n, C.c_int64(N * (N + 2) * 8), 1) for n in names]
+        return [self("enter_data", n, C.c_int64(self.n * (self.n + 2) * 8), 1) for n in names]
 
     def map(self, name):
-        n = N * (N + 2) * 8
+        n = self.n * (self.n + 2) * 8
         self.dev = self.L.shim_device(n)
         return self("map_data", name, C.c_void_p(self.dev), C.c_int64(n))
 
@@ -260,7 +267,7 @@ class Run:
 
     def diag(self, name, *args):
         o = self.out.ctypes.data
-        two = [C.c_void_p(o), C.c_void_p(o + 8 * N)][:1 if name == "glob" else 2]
+        two = [C.c_void_p(o), C.c_void_p(o + 8 * self.n)][:1 if name == "glob" else 2]
         return self(name, *args, *two)
 
     def close(self):
@@ -356,39 +363,57 @@ def test_every_allocation_may_fail(lib, call):
     assert 5 < k < 99
 
 
+@pytest.mark.parametrize("n", [32, N])
 @pytest.mark.parametrize("array", ["host", "mapped", "mapped, a new frame"])
-def test_what_an_owner_may_have_written(lib, array):
+def test_what_an_owner_may_have_written(lib, array, n):
     """An array that was transformed and transformed again: its spectrum, unless
     the owner of a mapped one has put something else into it.  What gt_sync_ref
     gives of a mapped one is read again, too; a host array, which only
     gt_update_device changes, keeps to the compact copy."""
-    r = Run(lib)
+    r = Run(lib, n)
     host = array == "host"
     assert (r.enter("z") == [0]) if host else (r.map("z") == 0)
     assert r("fft_dir", "z", D2Z) == 0 and r.diag("spectrum", "z") == 0
     if "frame" in array:
         C.memset(C.c_void_p(r.dev), 1, 64)
-    n = len(r.log())
+    k = len(r.log())
     assert r("fft_dir", "z", D2Z) == 0
-    assert r.log()[n:] == (["full:io"] if "frame" in array else ["scatter", "full:io"])
+    if n == N or host:  # a mapped array's small spectrum is in its memory already
+        assert r.log()[k] == ("keep" if "frame" in array else "scatter")
+    assert r.log()[-1] == ("full:io" if n == N or host else "full:io+ref")
     assert r("sync_ref", "z") == 0
-    n = len(r.log())
+    k = len(r.log())
     assert r.diag("spectrum", "z") == 0
-    assert ("gather" in r.log()[n:]) != host
+    assert ("gather" in r.log()[k:]) != host
     assert r.close() == 0
 
 
+@pytest.mark.parametrize("n", [32, N])
 @pytest.mark.parametrize("owned", [True, False])
-def test_fft_inv_of_a_field_with_both_copies(lib, owned):
+def test_fft_inv_of_a_field_with_both_copies(lib, owned, n):
     """A host array's compact copy is transformed as it is, in its own size; the
     memory of a mapped one, which its owner may have written to, is read."""
-    r = Run(lib)
+    r = Run(lib, n)
     assert (r.enter("z") == [0]) if owned else (r.map("z") == 0)
     assert r("trunc", "z") == 0 and r("sync_ref", "z") == 0
-    n = len(r.log())
+    k = len(r.log())
     assert r("fft_inv", "z", Z2D) == 0
-    assert r.log()[n:] == (["kept:io"] if owned else ["gather", "full:io"])
+    assert r.log()[k:] == (["kept:io"] if owned else ["full:io"] if n < N
+                           else ["gather", "full:io"])
     assert r.close() == 0
+
+
+def test_copy_of_a_transformed_array(lib):
+    """One transfer, whether or not the memory holds the spectrum, too; the copy
+    has no part in what the source's owner may write."""
+    for n in (32, N):
+        r = Run(lib, n)
+        assert r.map("z") == 0 and r.enter("w") == [0]
+        assert r("fft_dir", "z", D2Z) == 0 and r("copy", "w", "z") == 0
+        k = len(r.log())
+        assert r("sync_ref", "w") == 0 and r.log()[k:] == ["scatter"]
+        assert r.diag("spectrum", "w") == 0 and r.log()[-2:] == ["narrow", "spectrum"]
+        assert r.close() == 0
 
 
 @pytest.mark.parametrize("call,launches", [("fft_dir", ["full:io"]), ("trunc", ["narrow"]),
