@@ -138,8 +138,8 @@ int fwd_steps(gt_ctx* c, RectTables* t, int n0, int n1, int32_t* seed, bool keep
   a.emk = t->emk;
   CHK(rect_ka(c, s->rc, &a.ka));
   const bool rk4 = c->rko == 4;
-  const std::vector<int> stages = rk4 ? std::vector<int>{gt::C_RK4_1, gt::C_RK4_2, gt::C_RK4_3}
-                                      : std::vector<int>{gt::C_RK2_1};
+  const int stages[] = {rk4 ? gt::C_RK4_1 : gt::C_RK2_1, gt::C_RK4_2, gt::C_RK4_3};
+  const int nstages = rk4 ? 3 : 1;
   for (int n = n0; n < n1; ++n) {
     auto st = [&](int k) { return keep ? stage_ptr(s, n - n0, k) : nullptr; };
     a.sst = st(0);
@@ -153,9 +153,9 @@ int fwd_steps(gt_ctx* c, RectTables* t, int n0, int n1, int32_t* seed, bool keep
                             hipMemcpyDeviceToDevice, c->stream));
       s->ckseed[n / s->kchk] = *seed;
     }
-    for (size_t k = 0; k < stages.size(); ++k) {
+    for (int k = 0; k < nstages; ++k) {
       CHK(r_pass(c, a));
-      a.sst = st((int)k + 1);
+      a.sst = st(k + 1);
       CHK(c_pass(c, stages[k], a));
     }
     if (!keep || n + 1 < n1) CHK(r_pass(c, a));

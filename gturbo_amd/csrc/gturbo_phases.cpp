@@ -3,7 +3,6 @@
 #include "gturbo_phases.hpp"
 
 #include <cmath>
-#include <vector>
 
 namespace gtr {
 
@@ -16,9 +15,9 @@ struct Node {
 };
 constexpr int kNodes = 6 * 128 + 64;  // beyond 2 pi * 128 = 804.2
 
-const std::vector<Node>& nodes() {
-  static const std::vector<Node> t = [] {
-    std::vector<Node> v(kNodes);
+struct Nodes {  // static storage: the C entries that draw must not throw
+  Node v[kNodes];
+  Nodes() noexcept {
     for (int i = 0; i < kNodes; ++i) {
       const long double a = (long double)i / 128.0L, c = cosl(a), s = sinl(a);
       v[i].ch = (double)c;
@@ -26,9 +25,11 @@ const std::vector<Node>& nodes() {
       v[i].sh = (double)s;
       v[i].sl = (double)(s - (long double)v[i].sh);
     }
-    return v;
-  }();
-  return t;
+  }
+};
+const Node* nodes() {
+  static const Nodes t;
+  return t.v;
 }
 
 void sincos_ext(double te, double* c, double* s) {
@@ -80,7 +81,7 @@ __attribute__((target("fma"))) void sincos_fma(const Node* t, double te, double*
 void forcing_phases(int nf, int32_t* seed, double* out) {
   static const bool fast = __builtin_cpu_supports("fma");
   const double pi2 = 2.0 * 3.14159265358979;
-  const Node* t = nodes().data();
+  const Node* t = nodes();
   uint32_t s = (uint32_t)*seed;
   for (int k = 0; k < nf; ++k) {
     s = (69069u * s + 1u) & 0x7FFFFFFFu;
